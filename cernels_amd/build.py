@@ -24,7 +24,7 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I", str(PKG.parent / "include")]
 DEVICE = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-munsafe-fp-atomics"]
 
-SOURCES = ["moe_route.hip", "moe_gemm.hip", "moe_gemm_packed.hip", "moe_decode.hip", "moe_router.hip", "moe_capi.cpp"]
+SOURCES = ["moe_route.hip", "moe_gemm.hip", "moe_gemm_packed.hip", "moe_stream.hip", "moe_decode.hip", "moe_router.hip", "moe_capi.cpp"]
 
 
 def _compile(src: str) -> Path:

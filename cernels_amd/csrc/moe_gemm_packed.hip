@@ -44,6 +44,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "moe_packed.h"
 #include "moe_split.h"
 #include "moe_tile.h"
 
@@ -54,7 +55,6 @@ constexpr int kPkThreads = kPkWaves * kWave;
 constexpr int kPkBM = 256;
 constexpr int kPkMB = kPkBM / 32;           // 32-row MFMA blocks per item
 constexpr int kPkABytes = kPkBM * kBK * 2;  // 32 KB A stage
-constexpr int kPkFrag = 512;                // bf16 elements of one fragment (1 KB)
 constexpr int kPkGlu = kPkWaves * 16;       // glu columns of a GEMM1 N-tile
 constexpr int kPkStages = 3;                // activation LDS buffers = weight register slots per wave
 constexpr int kPkMaxTail = 16;              // most items split into halves at the end of an XCD's range
@@ -65,32 +65,6 @@ constexpr int kPkMaxTail = 16;              // most items split into halves at t
 // M-tiles split its rows evenly) 502.8/502.6 -> 512.5/510.1 (16 items: within a few µs of 12); down with 8 or
 // 12 items: equal or up to 12 µs slower on gpt-oss.
 constexpr int kPkTailGateUp = 12;
-// glu segments: scaled up below this largest |glu| (2^-8), down at or above 2^15; an all-zero segment
-// records kGluAnyScale in gexp
-constexpr float kGluSmall = 0.00390625f;
-constexpr int kGluAnyScale = -128;
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int kModePkGateUp = 0;
-constexpr int kModePkDown = 1;
-constexpr int kModePkUp = 2;  // non-gated first projection (megablocks): glu[r, :] = act(X[tok(r), :] · W1_e)
-
-// Packed layout of one projection, viewed as B[k][n] (reduction length Kd, KS = Kd/16 k-steps) cut
-// into NF fragments of 32 columns:
-//   gate_up: fragment c = gate columns [16c, 16c+16) then up columns [16c, 16c+16). Kd = H, NF = F/16.
-//   down:    fragment c = output columns [32c, 32c+32).                           Kd = F, NF = H/32.
-//   up:      (non-gated) fragment c = columns [32c, 32c+32), packed as a down projection with H and F
-//            exchanged.                                                           Kd = H, NF = F/32.
-// Fragments are bundled by eight (an N-tile: one fragment per wave) and stored k-step-major inside a
-// tile, so the eight waves of a workgroup read one contiguous 8 KB run per k-step. Lane l of
-// fragment (c, ks) holds B[16ks + 8(l/32) + j][column l%32 of the fragment], j = 0..7.
-// Returns the fragment's index in 1 KB units.
-__host__ __device__ inline long long packed_frag(int e, int c, int ks, int NF, int KS) {
-    const int t = c >> 3, w = c & 7, nw = min(8, NF - 8 * t);
-    return (long long)e * NF * KS + 8LL * KS * t + (long long)ks * nw + w;
-}
-
 // ---- packing (one-time, per weight tensor) ---------------------------------------------------------
 // One thread per 16-byte lane chunk of the packed output, in logical (e, c, ks, lane) order.
 // WHICH 0: gate_up (bf16). WHICH 1: down or the non-gated first projection. For down, `exps` holds
@@ -690,14 +664,6 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
             // is 2^15 or more (or not finite) or below 2^-8 (and not 0); then the segment is stored
             // again, scaled by 2^-s. m = 0 records kGluAnyScale. fmaxf passes over nan values.
             uint16_t* glu = reinterpret_cast<uint16_t*>(prm.out);
-            auto needs_scale = [](float m) { return !(m < 32768.f) || (m < kGluSmall && m > 0.f); };
-            // s with m * 2^-s in [2^14, 2^15): s >= 1 for m >= 2^15 (inf or nan: s = 1), s <= -23 for
-            // 0 < m < 2^-8 (clamped at -126, so 2^s stays a normal fp32 and s an int8 other than
-            // kGluAnyScale)
-            auto glu_scale = [](float m) {
-                const int s = __builtin_amdgcn_frexp_expf(m) - 15;
-                return m < 32768.f ? max(-126, s) : max(1, s);
-            };
             auto mark_scaled = [&](long long r) {
                 if (half == 0) prm.rsig[r] = 1;
                 prm.sync[1] = 1;
@@ -752,8 +718,8 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                         store_glu(g, h);
                         m = max_halves(m);  // the same on both lanes of the row
                         if (half == 0) prm.gexp[(long long)fc * prm.p_cap + r] = (int8_t)(m == 0.f ? kGluAnyScale : 0);
-                        if (needs_scale(m)) {  // rare: the segment stored again, scaled, by the same lanes
-                            const int sg = glu_scale(m);
+                        if (glu_needs_scale(m)) {  // rare: the segment stored again, scaled, by the same lanes
+                            const int sg = glu_scale_exp(m);
 #pragma unroll
                             for (int i = 0; i < 2; ++i) {
                                 float v[4];
@@ -810,8 +776,8 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                             prm.gexp[(long long)(2 * fc) * prm.p_cap + r] = s0;
                             prm.gexp[(long long)(2 * fc + 1) * prm.p_cap + r] = s0;
                         }
-                        if (needs_scale(m)) {  // rare: the segment stored again, scaled, by the same lanes
-                            const int sg = glu_scale(m);
+                        if (glu_needs_scale(m)) {  // rare: the segment stored again, scaled, by the same lanes
+                            const int sg = glu_scale_exp(m);
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
                                 float v[4];
@@ -1048,15 +1014,60 @@ hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t
                             const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
                             hipStream_t s);
 
-// route -> packed gate_up GEMM -> packed down GEMM -> combine, all on stream s. Shapes were checked
+bool few_supported(int T, int K, int E);
+bool tiles_supported(int T, int K, int E);
+hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
+                      const float* route_w, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
+                      uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev);
+int stream_tile_m();
+hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
+                               int bias_interleaved, int act, const int32_t* offsets, const int32_t* tile_offsets,
+                               const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles,
+                               uint16_t* glu, int8_t* gexp, int8_t* rsig, int32_t* sync, hipStream_t s);
+hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float* route_w, int T, int H, int F, int E, int K,
+                               const int32_t* offsets, const int32_t* tile_offsets, const int32_t* meta,
+                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, unsigned char* Y,
+                               hipStream_t s);
+
+// route -> packed gate_up GEMM -> packed down GEMM -> combine, all on stream s; few rows per expert take the streaming
+// forms of moe_stream.hip instead (its header states where the lines lie and why). Shapes were checked
 // by the caller (H % 64 == 0, F % 64 == 0, E <= 1024, T >= 1).
 hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2,
                                  const int32_t* idx, const float* route_w, int T, int H, int F, int E, int K,
                                  int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
                                  int32_t* meta, int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts,
                                  int max_tiles, uint16_t* glu, float* Y, int8_t* gexp, int8_t* rsig,
-                                 int8_t* psig, hipStream_t s, hipEvent_t* ev) {
+                                 int8_t* psig, unsigned char* few_lists, hipStream_t s, hipEvent_t* ev) {
+    if (few_supported(T, K, E))
+        return launch_few(x, w1p, b1, w2p, b2, idx, route_w, T, H, F, E, K, bias_interleaved, act, out, glu, gexp,
+                          reinterpret_cast<unsigned char*>(Y), few_lists, s, ev);
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
+    if (tiles_supported(T, K, E)) {  // moe_stream.hip
+        const int bm = stream_tile_m();
+        const long long P = (long long)T * K;
+        const int tiles = (int)((P + bm - 1) / bm + std::min<long long>(P, E));
+        mark(0);
+        hipError_t st = launch_route(idx, T, K, E, bm, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
+                                     meta + 8, s, rsig, nullptr);
+        if (st != hipSuccess) return st;
+        mark(1);
+        st = launch_stream_gemm1(x, w1p, b1, T, H, F, E, K, bias_interleaved, act, offsets, tile_offsets, meta, sorted_pairs,
+                                 tile_expert, tiles, glu, gexp, rsig, meta + 24, s);
+        if (st != hipSuccess) return st;
+        hipLaunchKernelGGL(moe_glu_fixup_kernel, dim3(32), dim3(256), 0, s, glu, gexp, rsig, psig, sorted_pairs, meta + 24,
+                           meta, T * K, F);
+        st = hipGetLastError();
+        if (st != hipSuccess) return st;
+        mark(2);
+        st = launch_stream_gemm2(glu, w2p, route_w, T, H, F, E, K, offsets, tile_offsets, meta, sorted_pairs, tile_expert,
+                                 tiles, reinterpret_cast<unsigned char*>(Y), s);
+        if (st != hipSuccess) return st;
+        mark(3);
+        st = launch_combine_h(reinterpret_cast<const unsigned char*>(Y), idx, static_cast<uint16_t*>(out), T, K, E, H,
+                              meta + 24, psig, b2, route_w, s);
+        mark(4);
+        return st;
+    }
     // Launch shapes of both GEMMs, from the shape alone; the route then splits each one's items over
     // the XCDs (meta[32..40] gate_up, meta[41..49] down). Where even the most M-tiles the route can
     // make (ceil(P / 256) + min(P, E)) would give each workgroup fewer than 8 rounds of items, the

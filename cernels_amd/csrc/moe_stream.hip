@@ -1,0 +1,733 @@
+// Routed experts on packed weights where experts average few rows, so that a call is bound by streaming the selected
+// experts' weights from HBM rather than by the matrix units (bf16 / fp16 MFMA, gfx950).
+//
+// The grouped GEMMs of moe_gemm_packed.hip keep one workgroup per CU on 256-row tiles; with a handful of rows per
+// expert they leave most of the chip without work (one token of gpt-oss: 92 items on 256 CUs) and wait for an LDS
+// stage and a barrier per 64 reduction columns. Here a workgroup owns one 32-column weight fragment of one expert and
+// its four waves split the reduction: weights (1 KB per fragment and k-step, read once) and activation rows (L2) both go
+// straight to registers, and no wave waits for another until the four partial sums meet in LDS at the end. Four such
+// workgroups per CU keep 128 KB of weights in flight (a plain read of 126 MB reaches 5.9 TB/s with 64 KB in flight on
+// 176 and more CUs, 4.2 TB/s on 88). What bounds it: HBM, 5.2-5.8 TB/s of weights in a launch of 130 MB and more.
+// Two, eight or five workgroups' worth of waves (64, 512 threads; 102 registers, which spill) measured 0-5%, 2-25% and
+// 35% slower.
+//
+// Two forms share the first projection:
+//   few    (T <= 32 tokens, at most 512 pairs): no route. Each workgroup finds its expert and that expert's tokens from
+//          the indices by itself (rows are tokens). Up to 16 pairs the down kernel sums every expert's contribution to
+//          its 16 output columns in registers (two launches), above that it writes a row per pair and the combine sums
+//          them (three; the general path takes five).
+//   tiles  (up to 512 tokens, at most 8 rows per expert on average): the route's list with M-tiles of 32 rows, then the
+//          glu fixup and the combine as on the general path.
+// Measured, whole op in us, general path -> here (seeded routing, weights of three layers in turn): gpt-oss shapes (H = F =
+// 2880, E = 32, k = 4) T=1 85 -> 43, T=8 234 -> 195, T=32 299 -> 273, T=48 311 -> 297 (tiles); H=2048 F=512 E=513 k=11
+// T=3 90 -> 58, T=28 291 -> 257, T=128 580 -> 521, T=400 635 -> 599 (tiles); H=2048 F=768 E=128 k=8 T=1 82 -> 34,
+// T=32 221 -> 189, T=65 239 -> 221, T=128 245 -> 237 (tiles). Above 8 rows per expert the tiles form loses (12.5 rows:
+// 245 -> 252): each wave fetches every row's 128-byte lines itself, where the general path shares them through LDS.
+// Precision is the general path's: fp32 accumulation, glu in fp16 segments scaled where needed (moe_packed.h), fp16
+// weights scaled per fragment, the routing weight and the sum over slots in fp32, one rounding to bf16.
+#include <algorithm>
+#include <climits>
+#include <type_traits>
+
+#include "moe_packed.h"
+#include "moe_split.h"
+#include "moe_tile.h"
+
+namespace cmoe {
+
+constexpr int kStWaves = 4, kStThreads = kStWaves * kWave;
+constexpr int kStRows = 32;         // rows of an M-tile (one 32-row MFMA block)
+constexpr int kFewMaxTokens = 32;   // one 32-row block: rows are tokens
+constexpr int kFewMaxPairs = 512;
+constexpr int kFewMaxExperts = 1024;  // bitmap of 32 words
+constexpr int kFdWaves = 8, kFdThreads = kFdWaves * kWave;  // few: down workgroup with the sum over slots
+constexpr int kFdStages = 4;
+constexpr int kFdMaxPairs = 16;    // above: rows per pair and the combine. gpt-oss 4 pairs 16.7 us against 15.4 + 4.6, 16
+                                   // pairs 50.6 / 46.6 + 5.2; 33 pairs of 30B-A3B-like experts 23.1 / 15.6 + 4.0: H / 16
+                                   // workgroups stream less than the whole chip, which the launch saved pays for up to here
+constexpr int kFewMaxTopk = 64;    // few_select's division by K
+constexpr int kTilesMaxTokens = 512;  // bounds the M-tiles of one popular expert, each of which streams its weights
+constexpr int kTilesMaxRows = 8;      // rows per expert on average
+
+struct StreamParams {
+    const uint16_t* A;            // first projection: x [T, H]; down: glu fp16
+    const uint16_t* B;            // packed weights of this projection
+    const float* bias;            // first: [E, 2F]; few down: [E, H]; or null
+    const int32_t* idx;           // few: [T, K]
+    const float* route_w;         // [T, K]
+    const int32_t* sorted_pairs;  // tiles: the route's lists
+    const int32_t* offsets;
+    const int32_t* tile_offsets;
+    const int32_t* tile_expert;
+    const int32_t* meta;
+    uint16_t* glu;                // few: row p of pair p; tiles: expert order
+    unsigned char* Y;             // tiles down: 24-bit rows, row p of pair p
+    uint16_t* out;                // few down: [T, H] bf16
+    int8_t* gexp;                 // [F/16, p_cap] power of two of each 16-column glu segment
+    int8_t* rsig;                 // tiles: rows with a scaled segment
+    int32_t* sync;                // tiles: [1] = some segment is scaled
+    const int8_t* wexp;           // down: [E, NF] power of two of each weight fragment
+    int32_t* few_e;               // few: [U_max] the u-th smallest expert chosen, -1 past the last
+    int16_t* few_row;             // few: [U_max, T] glu row (pair) of (expert u, token t), bit 14 if t names u again, -1: not chosen
+    float* few_w;                 // few: [U_max, T] routing weight (summed over slots that name the expert twice)
+    uint8_t* few_scaled;          // few: [U_max, NF of the first projection] some segment is scaled
+    int T, K, E, H, F, NF, KS, u_max, nf1;
+    int p_cap, a_bytes, bias_interleaved;
+};
+
+// One wave's share of an item's reduction: stages [s0, s0 + n) of 64 columns, acc += W_frag * A_block (32 rows). Two stages
+// are in flight, 8 KB of weights per wave; the last rounds are peeled so that no load sits behind a branch and the waits
+// stay exact. ao: byte offset of this lane's row (and 8-column half) in A.
+template <typename OpT>
+__device__ __forceinline__ void stream_stages(__amdgpu_buffer_rsrc_t rw, uint32_t wo, int bs, __amdgpu_buffer_rsrc_t ra,
+                                              uint32_t ao, int s0, int n, f32x16& acc) {
+    u32x4 w[2][4], a[2][4];
+    auto load = [&](int d, int s) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            w[d][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (4 * s + q) * bs, 0));
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            a[d][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, ao + 32 * q, s * kBK * 2, 0));
+    };
+    auto mul = [&](int d) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const OpT wq = __builtin_bit_cast(OpT, w[d][q]), aq = __builtin_bit_cast(OpT, a[d][q]);
+            if constexpr (std::is_same_v<OpT, f16x8>) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq, aq, acc, 0, 0, 0);
+            else acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq, aq, acc, 0, 0, 0);
+        }
+    };
+    if (n <= 0) return;
+    load(0, s0);
+    load(1, s0 + min(1, n - 1));
+    int s = 0;
+    for (; s + 3 < n; s += 2) {
+        mul(0);
+        load(0, s0 + s + 2);
+        mul(1);
+        load(1, s0 + s + 3);
+    }
+    if (s + 2 < n) {  // three left
+        mul(0);
+        load(0, s0 + s + 2);
+        mul(1);
+        mul(0);
+    } else {
+        mul(0);
+        if (s + 1 < n) mul(1);
+    }
+}
+
+// The sum of the four waves' partial accumulators, by one wave.
+__device__ __forceinline__ void sum_parts(const float (*part)[16][kWave], int lane, float (&v)[16]) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        float s = part[0][r][lane];
+#pragma unroll
+        for (int w = 1; w < kStWaves; ++w) s += part[w][r][lane];
+        v[r] = s;
+    }
+}
+
+// Y row of pair p, 32 columns of fragment fc, as 24-bit floats: a lane holds columns 8i + 4 half + 0..3 of its row (both
+// half-waves active for it); after the exchange lane l stores columns 0-15 and lane l + 32 columns 16-31.
+__device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, int fc, int half, const float (&v)[16], float ws) {
+    f24x4 q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = pack_f24x4(v[4 * i] * ws, v[4 * i + 1] * ws, v[4 * i + 2] * ws, v[4 * i + 3] * ws);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        swap_halves(q[0].d[d], q[2].d[d]);
+        swap_halves(q[1].d[d], q[3].d[d]);
+    }
+    u32x4* y = reinterpret_cast<u32x4*>(Y + (p * H + 32 * fc + 16 * half) * 3);
+    y[0] = u32x4{q[0].d[0], q[0].d[1], q[0].d[2], q[2].d[0]};
+    y[1] = u32x4{q[2].d[1], q[2].d[2], q[1].d[0], q[1].d[1]};
+    y[2] = u32x4{q[1].d[2], q[3].d[0], q[3].d[1], q[3].d[2]};
+}
+
+// few: the u-th smallest distinct expert of the indices (-1: fewer than u + 1), and in tokp[t] the first pair of token t
+// that names it, with bit 16 set if further pairs of t do (INT_MAX: none). One wave by itself: its own LDS words (a wave's LDS operations run in order), no
+// workgroup barrier.
+__device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int P, int E, int K, int u, int lane,
+                                          uint32_t* bits, int* tokp) {
+    int ev[kFewMaxPairs / kWave];
+#pragma unroll
+    for (int c = 0; c < kFewMaxPairs / kWave; ++c) {
+        ev[c] = -1;
+        if (kWave * c < P) {  // uniform
+            const int p = lane + kWave * c;
+            const int v = p < P ? idx[p] : -1;
+            ev[c] = (unsigned)v < (unsigned)E ? v : -1;
+        }
+    }
+    if (lane < kFewMaxExperts / 32) {
+        bits[lane] = 0u;
+        tokp[lane] = INT_MAX;
+    }
+#pragma unroll
+    for (int c = 0; c < kFewMaxPairs / kWave; ++c)
+        if (ev[c] >= 0) atomicOr(&bits[ev[c] >> 5], 1u << (ev[c] & 31));
+    uint32_t bw = lane < kFewMaxExperts / 32 ? bits[lane] : 0u;
+    const int cnt = __popc(bw);  // 0..32
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    int excl = 0;  // prefix sum over the lower lanes, bit by bit of cnt
+#pragma unroll
+    for (int b = 0; b < 6; ++b) excl += __popcll(__ballot((cnt >> b) & 1) & lt) << b;
+    const bool holder = u >= excl && u < excl + cnt;  // at most one lane
+    int eh = 0;
+    if (holder) {
+        for (int r = u - excl; r > 0; --r) bw &= bw - 1;
+        eh = lane * 32 + __ffs(bw) - 1;
+    }
+    const uint64_t hb = __ballot(holder);
+    if (hb == 0ull) return -1;
+    const int e = __builtin_amdgcn_readlane(eh, __ffsll((unsigned long long)hb) - 1);
+    const int magic = 65536 / K + 1;  // p / K for p < 512, K <= 64: p * magic >> 16 (error p / 65536 < 1 / K)
+#pragma unroll
+    for (int c = 0; c < kFewMaxPairs / kWave; ++c)
+        if (ev[c] == e) {
+            const int p = lane + kWave * c;
+            atomicMin(&tokp[(p * magic) >> 16], p);
+        }
+#pragma unroll
+    for (int c = 0; c < kFewMaxPairs / kWave; ++c)
+        if (ev[c] == e) {
+            const int p = lane + kWave * c, t = (p * magic) >> 16;
+            if ((tokp[t] & 0xffff) != p) atomicOr(&tokp[t], 0x10000);
+        }
+    return e;
+}
+
+// First projection: glu rows = act(A W1 (+ b1)) of one expert's rows and one weight fragment (16 glu columns for
+// gate_up, 32 for the non-gated projection). grid: (NF, u_max) few, (NF, tiles) tiles; neighbours in x read
+// neighbouring 1 KB pieces of one bundle.
+template <int MODE, int ACT, bool HAS_BIAS, bool FEW>
+__global__ __launch_bounds__(kStThreads, 4) void moe_stream_first_kernel(StreamParams prm) {
+    __shared__ float part[kStWaves][16][kWave];
+    __shared__ float s_bias[32];
+    __shared__ uint32_t s_bits[FEW ? kStWaves : 1][kFewMaxExperts / 32];
+    __shared__ int s_tokp[FEW ? kStWaves : 1][kFewMaxTokens];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lrow = lane & 31, half = lane >> 5;
+    const int fc = blockIdx.x;
+    const int nst = prm.H / kBK;
+    const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
+
+    int e, row_begin = 0, rows = 0;
+    int my_pair = INT_MAX, again = 0;  // few: this lane's token's glu row, and whether the token names e again
+    uint32_t ao;
+    if constexpr (FEW) {
+        e = few_select(prm.idx, prm.T * prm.K, prm.E, prm.K, blockIdx.y, lane, s_bits[wave], s_tokp[wave]);
+        if (e < 0) {  // the same in every wave
+            if (fc == 0 && tid == 0) prm.few_e[blockIdx.y] = -1;
+            if (tid == 0) prm.few_scaled[(long long)blockIdx.y * prm.NF + fc] = 0;
+            return;
+        }
+        int tp = INT_MAX;
+        if (lrow < prm.T) tp = s_tokp[wave][lrow];
+        if (tp != INT_MAX) {
+            my_pair = tp & 0xffff;
+            again = tp >> 16;
+        }
+        // rows of tokens that did not choose e read the first such token's row and are dropped
+        const uint64_t have = __ballot(my_pair != INT_MAX);
+        const int t = my_pair != INT_MAX ? lrow : (__ffsll((unsigned long long)have) - 1) & 31;
+        ao = (uint32_t)t * (uint32_t)(prm.H * 2) + 16u * half;
+    } else {
+        const int t = blockIdx.y;
+        if (t >= prm.meta[0]) return;
+        e = prm.tile_expert[t];
+        const int t0 = prm.tile_offsets[e], seg0 = prm.offsets[e];
+        tile_rows(t - t0, prm.tile_offsets[e + 1] - t0, prm.offsets[e + 1] - seg0, row_begin, rows);
+        row_begin += seg0;
+        const int pr = prm.sorted_pairs[row_begin + min(lrow, rows - 1)];
+        ao = (uint32_t)(pr / prm.K) * (uint32_t)(prm.H * 2) + 16u * half;
+    }
+    float bv = 0.f;  // bias of the fragment's column tid % 32 (16 gate, then 16 up)
+    if constexpr (HAS_BIAS) {
+        const int f = (tid >> 4) & 1, col = 16 * fc + (tid & 15);
+        const float* be = prm.bias + (long long)e * 2 * prm.F;
+        bv = prm.bias_interleaved ? be[2 * col + f] : be[f * prm.F + col];
+    }
+    const int nw = min(8, prm.NF - 8 * (fc >> 3));
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * nw * 1024 + 1024, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)prm.A, (short)0, prm.a_bytes, kBufferWord3);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    stream_stages<bf16x8>(rw, lane * 16u, nw * 1024, ra, ao, s0, n, acc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][r][lane] = acc[r];
+    if constexpr (HAS_BIAS) {
+        if (tid < 32) s_bias[tid] = bv;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+
+    // ---- epilogue: element r is row lane & 31, fragment column 8(r/4) + 4 half + r%4.
+    float v[16];
+    sum_parts(part, lane, v);
+    bool valid;
+    long long gr;
+    if constexpr (FEW) {
+        valid = my_pair != INT_MAX;
+        gr = my_pair;
+    } else {
+        valid = lrow < rows;
+        gr = row_begin + lrow;
+    }
+    constexpr int NV = MODE == kModePkGateUp ? 8 : 16;  // glu columns per lane
+    float g[NV];
+    float m = 0.f;  // the segment's largest |glu| (a nan is passed over)
+    if constexpr (MODE == kModePkGateUp) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            float gv = v[r], uv = v[8 + r];
+            if constexpr (HAS_BIAS) {
+                const int col = 8 * (r >> 2) + 4 * half + (r & 3);
+                gv += s_bias[col];
+                uv += s_bias[16 + col];
+            }
+            g[r] = swiglu<ACT>(gv, uv);
+            m = fmaxf(m, fabsf(g[r]));
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            g[r] = act_plain<ACT>(v[r]);
+            m = fmaxf(m, fabsf(g[r]));
+        }
+    }
+    m = max_halves(m);  // both lanes of the row
+    const int sg = glu_needs_scale(m) ? glu_scale_exp(m) : 0;  // 0 also for an all-zero segment
+    const bool scaled = valid && sg != 0;
+    if (valid) {  // lanes l and l ^ 32 hold the same row, so both run this or neither
+        uint32_t h[NV / 2];
+#pragma unroll
+        for (int r = 0; r < NV / 2; ++r)
+            h[r] = pack_f16x2(__builtin_amdgcn_ldexpf(g[2 * r], -sg), __builtin_amdgcn_ldexpf(g[2 * r + 1], -sg));
+        const int8_t se = (int8_t)(m == 0.f ? kGluAnyScale : sg);
+        if constexpr (MODE == kModePkGateUp) {
+            swap_halves(h[0], h[2]);  // lane l: columns 0-7, lane l + 32: columns 8-15
+            swap_halves(h[1], h[3]);
+            *reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 16 * fc + 8 * half) = u32x4{h[0], h[1], h[2], h[3]};
+            if (half == 0) prm.gexp[(long long)fc * prm.p_cap + gr] = se;
+        } else {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {  // lane l: columns 0-15, lane l + 32: columns 16-31
+                swap_halves(h[d], h[4 + d]);
+                swap_halves(h[2 + d], h[6 + d]);
+            }
+            u32x4* o = reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 32 * fc + 16 * half);
+            o[0] = u32x4{h[0], h[1], h[4], h[5]};
+            o[1] = u32x4{h[2], h[3], h[6], h[7]};
+            prm.gexp[(long long)(2 * fc + half) * prm.p_cap + gr] = se;
+        }
+        if constexpr (!FEW) {
+            if (scaled) {
+                if (half == 0) prm.rsig[gr] = 1;
+                prm.sync[1] = 1;
+            }
+        }
+    }
+    if constexpr (FEW) {
+        const uint64_t sb = __ballot(scaled);
+        const long long u = blockIdx.y;
+        if (lane == 0) prm.few_scaled[u * prm.NF + fc] = sb != 0ull;
+        if (fc == 0) {  // the lists that the down kernel walks
+            if (lane == 0) prm.few_e[u] = e;
+            if (lane < prm.T) {
+                float wt = 0.f;
+                for (int k = 0; k < prm.K; ++k)
+                    if (prm.idx[lane * prm.K + k] == e) wt += prm.route_w[lane * prm.K + k];
+                prm.few_row[u * prm.T + lane] = (int16_t)(valid ? my_pair | again << 14 : -1);
+                prm.few_w[u * prm.T + lane] = wt;
+            }
+        }
+    }
+}
+
+// tiles: Y[p, 32 columns of fragment c] = w_p * (glu row . W2_e) for the rows of one M-tile, as 24-bit floats at the pair's
+// own row. grid (NF, tiles).
+__global__ __launch_bounds__(kStThreads, 4) void moe_stream_down_kernel(StreamParams prm) {
+    __shared__ float part[kStWaves][16][kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lrow = lane & 31, half = lane >> 5;
+    const int fc = blockIdx.x, t = blockIdx.y;
+    if (t >= prm.meta[0]) return;
+    const int e = prm.tile_expert[t];
+    const int t0 = prm.tile_offsets[e], seg0 = prm.offsets[e];
+    int row_begin, rows;
+    tile_rows(t - t0, prm.tile_offsets[e + 1] - t0, prm.offsets[e + 1] - seg0, row_begin, rows);
+    row_begin += seg0;
+    const int nst = prm.F / kBK;
+    const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
+    const int row = min(lrow, rows - 1);
+    const long long p = prm.sorted_pairs[row_begin + row];
+    const float ws = __builtin_amdgcn_ldexpf(prm.route_w[p], prm.wexp[(long long)e * prm.NF + fc]);
+    const int nw = min(8, prm.NF - 8 * (fc >> 3));
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * nw * 1024 + 1024, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)(prm.A + (long long)row_begin * prm.F), (short)0,
+                                                                        rows * prm.F * 2, kBufferWord3);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    stream_stages<f16x8>(rw, lane * 16u, nw * 1024, ra, (uint32_t)row * (uint32_t)(prm.F * 2) + 16u * half, s0, n, acc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][r][lane] = acc[r];
+    __syncthreads();
+    if (wave != 0 || lrow >= rows) return;  // lanes l and l ^ 32 hold the same row
+    float v[16];
+    sum_parts(part, lane, v);
+    store_y(prm.Y, p, prm.H, fc, half, v, ws);
+}
+
+// few: Y[p, 32 columns of fragment c] = w_p * (glu row . W2_e) for the tokens of the u-th expert, as 24-bit floats at the
+// pair's own row. grid (NF, u_max).
+__global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(StreamParams prm) {
+    __shared__ float part[kStWaves][16][kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lrow = lane & 31, half = lane >> 5;
+    const int fc = blockIdx.x;
+    const long long u = blockIdx.y;
+    const int e = prm.few_e[u];
+    int fr = lrow < prm.T ? prm.few_row[u * prm.T + lrow] : -1;
+    int flags = 0;
+    for (int i = lane; i < prm.nf1; i += kWave) flags |= prm.few_scaled[u * prm.nf1 + i];
+    if (e < 0) return;
+    const bool any_scaled = __ballot(flags != 0) != 0ull;
+    const uint64_t have = __ballot(fr >= 0);
+    const int first = __builtin_amdgcn_readlane(fr, (__ffsll((unsigned long long)have) - 1) & 63);
+    const bool valid = fr >= 0, again = valid && (fr & 0x4000);
+    const int p = (valid ? fr : first) & 0x3fff;  // tokens without this expert read its first token's row and are dropped
+    const int nst = prm.F / kBK;
+    const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
+    int wx = prm.wexp[(long long)e * prm.NF + fc];
+    const float rw0 = prm.route_w[p];
+    const uint32_t ao = (uint32_t)p * (uint32_t)(prm.F * 2) + 16u * half;
+    const int nw = min(8, prm.NF - 8 * (fc >> 3));
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * nw * 1024 + 1024, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)prm.A, (short)0, prm.a_bytes, kBufferWord3);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (!any_scaled) {
+        stream_stages<f16x8>(rw, lane * 16u, nw * 1024, ra, ao, s0, n, acc);
+    } else {  // some segment of this expert's rows is scaled: every segment to its row's largest scale first
+        int smax = kGluAnyScale;
+        for (int g = 0; g < prm.F / 16; ++g) smax = max(smax, (int)prm.gexp[(long long)g * prm.p_cap + p]);
+        if (smax == kGluAnyScale) smax = 0;
+        wx += smax;
+        for (int ks = 4 * s0; ks < 4 * (s0 + n); ++ks) {  // a k-step is one 16-column segment
+            const f16x8 wq = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, ks * nw * 1024, 0));
+            f16x8 aq = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(ra, ao, ks * 32, 0));
+            const int d = min(0, (int)prm.gexp[(long long)ks * prm.p_cap + p] - smax);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) aq[j] = (_Float16)__builtin_amdgcn_ldexpf((float)aq[j], d);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq, aq, acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][r][lane] = acc[r];
+    __syncthreads();
+    if (wave != 0 || !valid) return;  // lanes l and l ^ 32 hold the same row
+    float v[16];
+    sum_parts(part, lane, v);
+    store_y(prm.Y, p, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(rw0, wx));
+    if (again)  // further slots of the token that name the same expert
+        for (int k = 0; k < prm.K; ++k) {
+            const int pp = lrow * prm.K + k;
+            if (pp != p && prm.idx[pp] == e)
+                store_y(prm.Y, pp, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(prm.route_w[pp], wx));
+        }
+}
+
+// few, at most kFdMaxPairs pairs: out[t, 16 columns] = bf16( sum over the experts u of w[u, t] * (glu row . W2_e + b2_e) ), which
+// saves the combine's launch. grid H / 16: a workgroup takes one half of a 32-column weight fragment for all experts; its
+// waves split the (expert, 64-column stage) list evenly and in order, each keeping its tokens' sums in registers
+// (16x16x32 MFMA, tokens as columns), and the sums are added in wave order. kFdStages stages in flight per wave.
+template <bool HAS_BIAS>
+__global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams prm) {
+    const int T = prm.T, um = prm.u_max;  // both <= kFdMaxPairs
+    __shared__ int s_e[kFdMaxPairs];
+    __shared__ int s_x[kFdMaxPairs];                // power of two of the weight fragment
+    __shared__ float s_w[kFdMaxPairs * kFdMaxPairs];  // [um, T]
+    __shared__ int s_row[kFdMaxPairs * kFdMaxPairs];  // [um, T], -1: not chosen
+    __shared__ int s_max[kFdMaxPairs];              // where segments are scaled: the largest power of two of each glu row
+    __shared__ __attribute__((aligned(16))) float red[kFdWaves][16][16];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int fc = blockIdx.x >> 1, hf = blockIdx.x & 1;  // weight fragment, its half
+    const int l16 = lane & 15, grp = lane >> 4;
+
+    const int my_e = tid < um ? prm.few_e[tid] : -1;
+    int flags = 0;
+    const int nfl = um * prm.nf1;
+    for (int i = tid; i < nfl; i += kFdThreads) flags |= prm.few_scaled[i];
+    if (tid < um * T) {
+        const int r = prm.few_row[tid];
+        s_w[tid] = prm.few_w[tid];
+        s_row[tid] = r < 0 ? -1 : r & 0x3fff;
+    }
+    if (tid < um) {
+        s_e[tid] = my_e;
+        s_x[tid] = my_e >= 0 ? prm.wexp[(long long)my_e * prm.NF + fc] : 0;
+    }
+    const int U = __syncthreads_count(my_e >= 0);  // the entries are a prefix
+    const bool any_scaled = __syncthreads_or(flags) != 0;
+    if (any_scaled) {
+        if (tid < U * T && s_row[tid] >= 0) {
+            const int p = s_row[tid];
+            int smax = kGluAnyScale;
+            for (int u = 0; u < prm.F / 16; ++u) smax = max(smax, (int)prm.gexp[(long long)u * prm.p_cap + p]);
+            s_max[p] = smax == kGluAnyScale ? 0 : smax;
+        }
+        __syncthreads();
+    }
+
+    const int S = prm.F / kBK;  // stages per expert
+    const int N = U * S;
+    const int i0 = wave * N / kFdWaves, cnt = (wave + 1) * N / kFdWaves - i0;
+    const int nw = min(8, prm.NF - 8 * (fc >> 3)), bs = nw * 1024;
+    const uint32_t wo = (uint32_t)((grp >> 1) * bs + (grp & 1) * 512 + (16 * hf + l16) * 16);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)prm.A, (short)0, prm.a_bytes, kBufferWord3);
+    const int t16 = min(l16, T - 1);
+
+    f32x4 tot = {0.f, 0.f, 0.f, 0.f}, acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int D = kFdStages;
+    u32x4 w[D][2], a[D][2];
+    float bsum = 0.f;  // this thread's output element's share of the down bias
+
+    auto run = [&](auto sc) {
+        constexpr bool SC = decltype(sc)::value;
+        int lu = cnt > 0 ? i0 / S : 0, ls = cnt > 0 ? i0 - lu * S : 0;  // stage to load next
+        int cu = lu, cs = ls;                                        // stage to multiply next
+        int left = cnt;                                              // stages not loaded yet
+        auto load = [&](int d) {
+            const int e = __builtin_amdgcn_readfirstlane(s_e[lu]);
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+                (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * bs + 1024, kBufferWord3);
+            const uint32_t r = (uint32_t)max(0, s_row[lu * T + t16]);  // a token without this expert: row 0, dropped
+            const uint32_t ro = r * (uint32_t)(prm.F * 2) + 16u * grp;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                w[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (4 * ls + 2 * i) * bs, 0));
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                a[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, ro + 64 * i, ls * kBK * 2, 0));
+            if (--left > 0 && ++ls == S) {  // past the last stage: the last one again, dropped
+                ls = 0;
+                ++lu;
+            }
+        };
+        auto mul = [&](int d, bool last) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                f16x8 aq = __builtin_bit_cast(f16x8, a[d][i]);
+                if constexpr (SC) {  // bring the segment to its row's scale
+                    const int p = max(0, s_row[cu * T + t16]);
+                    const int dd = (int)prm.gexp[(long long)(4 * cs + 2 * i + (grp >> 1)) * prm.p_cap + p] - s_max[p];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) aq[j] = (_Float16)__builtin_amdgcn_ldexpf((float)aq[j], min(dd, 0));
+                }
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[d][i]), aq, acc, 0, 0, 0);
+            }
+            if (++cs == S || last) {  // this expert's share is whole: into the tokens' sums
+                const int p = s_row[cu * T + t16];
+                int x = s_x[cu];
+                if constexpr (SC) x += s_max[max(p, 0)];
+                const float wt = s_w[cu * T + t16];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float y = tot[r] + wt * __builtin_amdgcn_ldexpf(acc[r], x);
+                    tot[r] = p >= 0 ? y : tot[r];  // a select: dropped rows may hold anything
+                    acc[r] = 0.f;
+                }
+                cs = 0;
+                ++cu;
+            }
+        };
+        if (cnt > 0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) load(d);
+        }
+        if constexpr (HAS_BIAS) {
+            const int t = tid >> 4;
+            if (t < T)
+                for (int u = 0; u < U; ++u)
+                    if (s_row[u * T + t] >= 0)
+                        bsum += s_w[u * T + t] * prm.bias[(long long)s_e[u] * prm.H + 16 * blockIdx.x + (tid & 15)];
+        }
+        for (int i = 0; i < cnt; i += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (i + d < cnt) mul(d, i + d == cnt - 1);
+                load(d);
+            }
+        }
+    };
+    if (any_scaled) run(std::true_type{});
+    else run(std::false_type{});
+    *reinterpret_cast<f32x4*>(&red[wave][l16][4 * grp]) = tot;
+    __syncthreads();
+    const int t = tid >> 4, c = tid & 15;  // tokens x 16 columns (the first 256 threads)
+    if (t < T) {
+        float s = red[0][t][c];
+#pragma unroll
+        for (int k = 1; k < kFdWaves; ++k) s += red[k][t][c];
+        if constexpr (HAS_BIAS) s += bsum;
+        prm.out[(long long)t * prm.H + 16 * blockIdx.x + c] = f32_to_bf16_bits(s);
+    }
+}
+
+int stream_tile_m() { return kStRows; }
+
+// Whether a call (that is not of the few form) takes the tiles form.
+bool tiles_supported(int T, int K, int E) {
+    return T <= kTilesMaxTokens && (long long)T * K <= (long long)kTilesMaxRows * E;
+}
+
+// Whether a call takes the few form: one 32-row block of tokens, and lists that fit the down kernel's LDS.
+bool few_supported(int T, int K, int E) {
+    const long long P = (long long)T * K;
+    return T <= kFewMaxTokens && K <= kFewMaxTopk && P <= kFewMaxPairs;
+}
+
+// Bytes of the lists that the few form passes from its first to its second launch (16-byte aligned parts).
+static size_t few_part(size_t n) { return (n + 15) / 16 * 16; }
+size_t few_workspace_bytes(int T, int F, int E, int K) {
+    const long long P = (long long)T * K;
+    if (!few_supported(T, K, E)) return 0;
+    const size_t um = (size_t)(P < E ? P : E);
+    return few_part(um * 4) + few_part(um * T * 2) + few_part(um * T * 4) + few_part(um * (F / 16));
+}
+
+hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
+                            const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
+                            hipStream_t s);
+
+template <bool FEW>
+static void launch_stream_first(const StreamParams& q, int act, dim3 grid, hipStream_t s) {
+#define CMOE_ST1(MODE, ACT, BIAS) hipLaunchKernelGGL((moe_stream_first_kernel<MODE, ACT, BIAS, FEW>), grid, dim3(kStThreads), 0, s, q)
+    if (act == kActSilu) {
+        if (q.bias) CMOE_ST1(kModePkGateUp, kActSilu, true);
+        else CMOE_ST1(kModePkGateUp, kActSilu, false);
+    } else if (act == kActGptOss) {
+        if (q.bias) CMOE_ST1(kModePkGateUp, kActGptOss, true);
+        else CMOE_ST1(kModePkGateUp, kActGptOss, false);
+    } else if (act == kActGeluTanh) CMOE_ST1(kModePkUp, kActGeluTanh, false);
+    else if (act == kActSiluPlain) CMOE_ST1(kModePkUp, kActSiluPlain, false);
+    else CMOE_ST1(kModePkUp, kActRelu, false);
+#undef CMOE_ST1
+}
+
+// gate_up -> down with the sum over slots, on stream s. Shapes were checked by the caller (few_supported).
+hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
+                      const float* route_w, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
+                      uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev) {
+    auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
+    const int P = T * K, um = std::min(P, E);
+    StreamParams q{};
+    q.A = static_cast<const uint16_t*>(x);
+    q.B = static_cast<const uint16_t*>(w1p);
+    q.bias = b1;
+    q.idx = idx;
+    q.route_w = route_w;
+    q.glu = glu;
+    q.gexp = gexp;
+    q.few_e = reinterpret_cast<int32_t*>(lists);
+    q.few_row = reinterpret_cast<int16_t*>(lists + few_part((size_t)um * 4));
+    q.few_w = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(q.few_row) + few_part((size_t)um * T * 2));
+    q.few_scaled = reinterpret_cast<unsigned char*>(q.few_w) + few_part((size_t)um * T * 4);
+    q.T = T; q.K = K; q.E = E; q.H = H; q.F = F;
+    q.NF = q.nf1 = act_is_gated(act) ? F / 16 : F / 32;
+    q.KS = H / 16;
+    q.u_max = um;
+    q.p_cap = P;
+    q.a_bytes = T * H * 2;
+    q.bias_interleaved = bias_interleaved;
+    mark(0);
+    mark(1);  // no route
+    launch_stream_first<true>(q, act, dim3(q.NF, um), s);
+    hipError_t st = hipGetLastError();
+    if (st != hipSuccess) return st;
+    mark(2);
+    q.A = glu;
+    q.a_bytes = P * F * 2;
+    q.B = static_cast<const uint16_t*>(w2p);
+    q.wexp = reinterpret_cast<const int8_t*>(static_cast<const uint16_t*>(w2p) + (long long)E * H * F);
+    q.bias = b2;
+    q.NF = H / 32;
+    q.KS = F / 16;
+    q.out = static_cast<uint16_t*>(out);
+    if (P > kFdMaxPairs) {
+        q.Y = Y;
+        hipLaunchKernelGGL(moe_few_down_rows_kernel, dim3(q.NF, um), dim3(kStThreads), 0, s, q);
+        st = hipGetLastError();
+        if (st != hipSuccess) return st;
+        mark(3);
+        st = launch_combine_h(Y, idx, static_cast<uint16_t*>(out), T, K, E, H, nullptr, nullptr, b2, route_w, s);
+        mark(4);
+        return st;
+    }
+    if (b2) hipLaunchKernelGGL((moe_few_down_kernel<true>), dim3(H / 16), dim3(kFdThreads), 0, s, q);
+    else hipLaunchKernelGGL((moe_few_down_kernel<false>), dim3(H / 16), dim3(kFdThreads), 0, s, q);
+    st = hipGetLastError();
+    mark(3);
+    mark(4);  // no combine
+    return st;
+}
+
+// The two projections of the tiles form, between the route (M-tiles of stream_tile_m() rows) and the fixup, and between the
+// fixup and the combine. max_tiles bounds the M-tile list.
+hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
+                               int bias_interleaved, int act, const int32_t* offsets, const int32_t* tile_offsets,
+                               const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles,
+                               uint16_t* glu, int8_t* gexp, int8_t* rsig, int32_t* sync, hipStream_t s) {
+    StreamParams q{};
+    q.A = static_cast<const uint16_t*>(x);
+    q.B = static_cast<const uint16_t*>(w1p);
+    q.bias = b1;
+    q.offsets = offsets; q.tile_offsets = tile_offsets; q.meta = meta; q.sorted_pairs = sorted_pairs; q.tile_expert = tile_expert;
+    q.glu = glu;
+    q.gexp = gexp;
+    q.rsig = rsig;
+    q.sync = sync;
+    q.T = T; q.K = K; q.E = E; q.H = H; q.F = F;
+    q.NF = act_is_gated(act) ? F / 16 : F / 32;
+    q.KS = H / 16;
+    q.p_cap = T * K;
+    q.a_bytes = T * H * 2;
+    q.bias_interleaved = bias_interleaved;
+    launch_stream_first<false>(q, act, dim3(q.NF, max_tiles), s);
+    return hipGetLastError();
+}
+
+hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float* route_w, int T, int H, int F, int E, int K,
+                               const int32_t* offsets, const int32_t* tile_offsets, const int32_t* meta,
+                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, unsigned char* Y,
+                               hipStream_t s) {
+    StreamParams q{};
+    q.A = glu;
+    q.B = static_cast<const uint16_t*>(w2p);
+    q.wexp = reinterpret_cast<const int8_t*>(static_cast<const uint16_t*>(w2p) + (long long)E * H * F);
+    q.route_w = route_w;
+    q.offsets = offsets; q.tile_offsets = tile_offsets; q.meta = meta; q.sorted_pairs = sorted_pairs; q.tile_expert = tile_expert;
+    q.Y = Y;
+    q.T = T; q.K = K; q.E = E; q.H = H; q.F = F;
+    q.NF = H / 32;
+    q.KS = F / 16;
+    q.p_cap = T * K;
+    hipLaunchKernelGGL(moe_stream_down_kernel, dim3(q.NF, max_tiles), dim3(kStThreads), 0, s, q);
+    return hipGetLastError();
+}
+
+}  // namespace cmoe

@@ -1,0 +1,159 @@
+"""Few rows per expert on packed weights: the streaming forms of moe_experts_packed, against the fp64 oracle.
+
+Up to 32 tokens and 512 pairs the kernels route by themselves (up to 16 pairs with the sum over slots in the down kernel,
+above that with a row per pair); up to 512 tokens with at most 8 rows per expert on average they walk the route's list in
+M-tiles of 32 rows. Cases sit on both sides of each line, at the smallest and largest sizes, with ids that are out of range
+or name an expert twice, one expert taking every token, and glu segments stored scaled.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import assert_within_tolerance, oracle_fp64, rand_case, to_device
+from oracle import eager as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _packed(c, device):
+    from cernels_amd import ops
+
+    d = to_device(c, device)
+    layout = ops.LAYOUT_CONCAT if c["layout"] == "concat" else ops.LAYOUT_INTERLEAVED
+    act = ops.ACT_SILU if c["act"] == "silu" else ops.ACT_GPTOSS
+    pk = ops.pack_experts(d["W1"], d["W2"], layout=layout, act=act, gate_up_bias=d["b1"], down_bias=d["b2"])
+    return ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], d["idx"].shape[1]).cpu()
+
+
+SILU, GPT = ("concat", "silu", False), ("interleaved", "gptoss", True)
+CASES = [
+    # T, H, F, E, K, (layout, act, bias), ids
+    (1, 64, 64, 1, 1, SILU, "plain"),          # one stage per projection: three of the four waves have none
+    (1, 192, 320, 1024, 16, SILU, "plain"),    # 16 pairs in one token, partial last bundles
+    (16, 128, 192, 3, 1, GPT, "plain"),        # 16 pairs, the fused down's last
+    (17, 128, 192, 3, 1, GPT, "plain"),        # 17: rows and combine
+    (4, 576, 64, 9, 4, GPT, "twice"),
+    (5, 320, 128, 6, 3, SILU, "twice"),        # rows form, an expert named twice by one token
+    (7, 128, 64, 12, 2, SILU, "invalid"),
+    (3, 128, 64, 4, 2, GPT, "none"),           # no valid id at all: zeros
+    (20, 128, 64, 4, 2, SILU, "none"),
+    (32, 128, 128, 512, 16, SILU, "plain"),    # 512 pairs
+    (32, 128, 128, 512, 17, SILU, "plain"),    # 544: the route's list (tiles)
+    (32, 1088, 448, 64, 8, GPT, "same"),       # every token on the same experts
+    (33, 128, 192, 64, 4, SILU, "invalid"),    # 33 tokens: tiles
+    (64, 256, 128, 32, 4, GPT, "plain"),       # 8 rows per expert: tiles' last
+    (65, 256, 128, 32, 4, GPT, "plain"),       # above: the grouped GEMMs
+    (512, 128, 64, 64, 1, SILU, "same"),       # one expert with 512 rows: 16 tiles
+    (513, 128, 64, 65, 1, SILU, "plain"),
+    (90, 192, 64, 40, 3, SILU, "twice"),
+]
+
+
+def _case(T, H, Fi, E, K, kind, ids):
+    layout, act, bias = kind
+    c = rand_case(7 * T + K, T, H, Fi, E, K, layout=layout, act=act, bias=bias, std=0.05,
+                  invalid=max(3, T // 4) if ids == "invalid" else 0)
+    if ids == "twice":
+        c["idx"][::2, K - 1] = c["idx"][::2, 0]
+    elif ids == "same":
+        c["idx"][:] = c["idx"][:1]
+    elif ids == "none":
+        c["idx"][:] = E + 5
+    return c
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"T{c[0]}H{c[1]}F{c[2]}E{c[3]}k{c[4]}{c[5][1]}-{c[6]}")
+def test_few_rows(device, case):
+    c = _case(*case)
+    print(f"[few rows {case}]", flush=True)
+    out = _packed(c, device)
+    ref = oracle_fp64(c)
+    if case[6] == "none":
+        assert not out.float().any()
+    assert_within_tolerance(out, ref, str(case))
+
+
+@pytest.mark.parametrize("gain", [3000.0, 1e-4])
+@pytest.mark.parametrize("T,E,bias", [(5, 8, True), (30, 8, True), (40, 32, False)], ids=["fused", "rows", "tiles"])
+def test_few_rows_scaled_segments(device, T, E, bias, gain):
+    """Rows whose glu leaves fp16's range (or falls to its subnormals) are stored scaled; each row group meets the bar on its
+    own scale, with columns 0-15 of two experts at zero so that scaled rows hold all-zero segments too."""
+    K = 3
+    c = rand_case(T, T, 256, 192, E, K, std=0.05, bias=bias and gain > 1)
+    for e in (0, 3):
+        c["W1"][e, :16] = 0
+    odd = torch.arange(1, T, 4)
+    x = c["x"].float()
+    x[odd] *= gain
+    c["x"] = x.bfloat16()
+    print(f"[few rows scaled T{T} gain {gain}]", flush=True)
+    out = _packed(c, device)
+    assert torch.isfinite(out.float()).all()
+    ref = oracle_fp64(c)
+    rest = torch.ones(T, dtype=torch.bool)
+    rest[odd] = False
+    assert_within_tolerance(out[odd], ref[odd], "scaled rows")
+    assert_within_tolerance(out[rest], ref[rest], "other rows")
+
+
+@pytest.mark.parametrize("T", [4, 24, 60], ids=["fused", "rows", "tiles"])
+def test_few_rows_nan_token(device, T):
+    """A token with a nan gives an all-nan row; the others, which share its experts' workgroups, stay within the bar."""
+    c = rand_case(T + 1, T, 128, 192, 32, 4)
+    bad = T // 2
+    c["x"][bad, 3] = float("nan")
+    print(f"[few rows nan T{T}]", flush=True)
+    out = _packed(c, device)
+    keep = torch.tensor([t for t in range(T) if t != bad])
+    assert torch.isnan(out[bad].float()).all()
+    assert_within_tolerance(out[keep], oracle_fp64(c, keep), "nan token")
+
+
+@pytest.mark.parametrize("T,E,act_id", [(1, 8, 0), (30, 8, 1), (40, 16, 2), (40, 16, 0)])
+def test_few_rows_nongated(device, T, E, act_id):
+    from cernels_amd import ops
+
+    g = torch.Generator().manual_seed(T + act_id)
+    H, Fi, K = 192, 320, 2
+    x = torch.randn(T, H, generator=g).bfloat16()
+    x[T // 2] *= 1000.0  # its segments are stored scaled
+    w1 = (torch.randn(E, H, Fi, generator=g) * 0.05).bfloat16()
+    w2 = (torch.randn(E, Fi, H, generator=g) * 0.05).bfloat16()
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).int()
+    wt = torch.rand(T, K, generator=g)
+    print(f"[few rows nongated T{T} act{act_id}]", flush=True)
+    out = ops.megablocks_moe(*[t.contiguous().to(device) for t in (x, w1, w2, idx, wt)], K, act_id).cpu()
+    ref = O.megablocks_fp64(x, idx, wt, w1, w2, act_id)
+    big = torch.zeros(T, dtype=torch.bool)
+    big[T // 2] = True
+    assert_within_tolerance(out[big], ref[big], "scaled row")
+    if T > 1:
+        assert_within_tolerance(out[~big], ref[~big], "other rows")
+
+
+@pytest.mark.parametrize("T", [3, 24, 60], ids=["fused", "rows", "tiles"])
+def test_few_rows_graph_replays(device, T):
+    """Captured and replayed with new inputs in the same buffers, each replay equals the eager call bit for bit (nothing is
+    kept between calls)."""
+    from cernels_amd import ops
+
+    c = rand_case(T + 2, T, 256, 192, 32, 4)
+    d = to_device(c, device)
+    pk = ops.pack_experts(d["W1"], d["W2"])
+    out = torch.empty_like(d["x"])
+    print(f"[few rows graph T{T}]", flush=True)
+    ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4, out=out)
+    for i in range(3):
+        n = to_device(rand_case(100 * i + T, T, 256, 192, 32, 4), device)
+        d["x"].copy_(n["x"])
+        d["idx"].copy_(n["idx"])
+        d["w"].copy_(n["w"])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4))
