@@ -29,6 +29,8 @@ ACT_SILU, ACT_GPTOSS = 0, 1
 ACT_GELU_TANH, ACT_SILU_PLAIN, ACT_RELU = 2, 3, 4  # non-gated (megablocks)
 GATE_UP, DOWN, UP = 0, 1, 2
 ROUTER_SOFTMAX_TOPK, ROUTER_TOPK_SOFTMAX = 0, 1
+INDEX_I32, INDEX_I64 = 0, 1
+WEIGHT_F32, WEIGHT_BF16 = 0, 1
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int32
@@ -60,6 +62,14 @@ _SIGNATURES = {
     "cernels_moe_experts_packed_staged": (
         ctypes.c_int,
         [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _S, _P, _P],
+    ),
+    "cernels_moe_experts_packed_typed": (
+        ctypes.c_int,
+        [_P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _S, _P],
+    ),
+    "cernels_moe_experts_decode_typed": (
+        ctypes.c_int,
+        [_P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _S, _P],
     ),
     "cernels_moe_router": (ctypes.c_int, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P]),
     "cernels_megablocks_moe_workspace_bytes": (_S, [_I, _I, _I, _I, _I]),

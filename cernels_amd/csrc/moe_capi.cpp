@@ -14,7 +14,8 @@ struct XcdSplit;
 hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t* offsets, int32_t* sorted_pairs,
                         int32_t* tile_offsets, int32_t* tile_expert, int32_t* meta, int32_t* counts,
                         int32_t* sched, hipStream_t stream, int8_t* row_zero = nullptr,
-                        const XcdSplit* split = nullptr);
+                        const XcdSplit* split = nullptr, int types = 0, const void* route_w = nullptr,
+                        int32_t* idx32 = nullptr, float* w32 = nullptr);
 size_t route_workspace_bytes(int T, int K, int E);
 int gemm_tile_m();
 int packed_tile_m();
@@ -35,16 +36,16 @@ int decode_max_tokens();
 size_t packed_weight_bytes(int H, int F, int E, int which);
 hipError_t launch_pack(const uint16_t* src, uint16_t* dst, int E, int H, int F, int layout, int which, hipStream_t s);
 hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2,
-                                 const int32_t* idx, const float* route_w, int T, int H, int F, int E, int K,
-                                 int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
+                                 const int32_t* idx, const void* route_w, int types, int32_t* idx32, float* w32, int T, int H,
+                                 int F, int E, int K, int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
                                  int32_t* meta, int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts,
                                  int max_tiles, uint16_t* glu, float* Y, int8_t* gexp, int8_t* rsig,
                                  int8_t* psig, unsigned char* few_lists, hipStream_t s, hipEvent_t* ev);
 int stream_tile_m();
 size_t few_workspace_bytes(int T, int F, int E, int K);
 hipError_t launch_decode(const uint16_t* x, const uint16_t* w1, const float* b1, const uint16_t* w2, const float* b2,
-                         const int32_t* idx, const float* route_w, uint16_t* glu, int32_t* order, uint16_t* out,
-                         int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev);
+                         const int32_t* idx, const void* w, int types, uint16_t* glu, int32_t* order, float* order_w,
+                         uint16_t* out, int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev);
 }  // namespace cmoe
 
 namespace {
@@ -56,7 +57,7 @@ size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 struct PrefillWs {
-    size_t offsets, tile_offsets, meta, sorted_pairs, tile_expert, route_counts, glu, Y, gexp, rsig, psig, few, total;
+    size_t offsets, tile_offsets, meta, sorted_pairs, tile_expert, route_counts, glu, Y, gexp, rsig, psig, few, idx32, w32, total;
     int capacity;
 };
 
@@ -81,12 +82,14 @@ PrefillWs prefill_ws(int T, int H, int F, int E, int K) {
     w.rsig = o;         o = align_up(o + (size_t)P);             // packed path: per glu row scale
     w.psig = o;         o = align_up(o + (size_t)P);             // packed path: the same, per pair
     w.few = o;          o = align_up(o + cmoe::few_workspace_bytes(T, F, E, K));  // packed path, few tokens: expert lists
+    w.idx32 = o;        o = align_up(o + sizeof(int32_t) * P);  // packed path: ids and weights that came as int64 / bf16
+    w.w32 = o;          o = align_up(o + sizeof(float) * P);
     w.total = o;
     return w;
 }
 
 struct DecodeWs {
-    size_t glu, order, total;
+    size_t glu, order, order_w, total, total_f32;  // total_f32: without order_w, what calls with fp32 weights use
 };
 
 DecodeWs decode_ws(int T, int H, int F, int K) {
@@ -96,6 +99,8 @@ DecodeWs decode_ws(int T, int H, int F, int K) {
     size_t o = 0;
     w.glu = o; o = align_up(o + sizeof(uint16_t) * P * F);
     w.order = o; o = align_up(o + sizeof(int32_t) * P);  // valid pairs sorted by expert, then -1
+    w.total_f32 = o;
+    w.order_w = o; o = align_up(o + sizeof(float) * P);  // bf16 weights: their fp32 values in that order
     w.total = o;
     return w;
 }
@@ -106,8 +111,15 @@ bool dims_ok(int T, int H, int F, int E, int K) {
     return T >= 0 && H > 0 && F > 0 && E > 0 && K > 0 && K <= kMaxTopk && (long long)T * K < (1LL << 31);
 }
 
-int common_checks(const void* x, const void* w1, const void* w2, const int32_t* idx, const float* wts, int T,
-                  int H, int F, int E, int K, int layout, int act, void* out, void* ws) {
+// The routing's types (moe_common.h): bit 0 int64 indices, bit 1 bf16 weights.
+int pair_types(int index_type, int weight_type) {
+    if (index_type < CERNELS_MOE_INDEX_I32 || index_type > CERNELS_MOE_INDEX_I64) return -1;
+    if (weight_type < CERNELS_MOE_WEIGHT_F32 || weight_type > CERNELS_MOE_WEIGHT_BF16) return -1;
+    return (index_type == CERNELS_MOE_INDEX_I64 ? 1 : 0) | (weight_type == CERNELS_MOE_WEIGHT_BF16 ? 2 : 0);
+}
+
+int common_checks(const void* x, const void* w1, const void* w2, const void* idx, const void* wts, int T,
+                  int H, int F, int E, int K, int layout, int act, void* out, void* ws, int types = 0) {
     if (!dims_ok(T, H, F, E, K)) return CERNELS_MOE_INVALID_ARGUMENT;
     if (layout != CERNELS_MOE_LAYOUT_CONCAT && layout != CERNELS_MOE_LAYOUT_INTERLEAVED)
         return CERNELS_MOE_INVALID_ARGUMENT;
@@ -116,7 +128,7 @@ int common_checks(const void* x, const void* w1, const void* w2, const int32_t* 
     if (!x || !w1 || !w2 || !idx || !wts || !out || !ws) return CERNELS_MOE_INVALID_ARGUMENT;
     if (!aligned16(x) || !aligned16(w1) || !aligned16(w2) || !aligned16(out) || !aligned16(ws))
         return CERNELS_MOE_MISALIGNED;
-    if ((reinterpret_cast<uintptr_t>(idx) & 3u) || (reinterpret_cast<uintptr_t>(wts) & 3u))
+    if ((reinterpret_cast<uintptr_t>(idx) & (types & 1 ? 7u : 3u)) || (reinterpret_cast<uintptr_t>(wts) & (types & 2 ? 1u : 3u)))
         return CERNELS_MOE_MISALIGNED;
     return CERNELS_MOE_OK;
 }
@@ -241,13 +253,14 @@ int cernels_moe_pack_weights(const void* src, int32_t H, int32_t F, int32_t E, i
                                         layout, which, stream));
 }
 
-int cernels_moe_experts_packed_staged(const void* x, const void* gate_up_packed, const float* gate_up_bias,
-                                      const void* down_packed, const float* down_bias, const int32_t* indices,
-                                      const float* weights, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
-                                      int32_t bias_layout, int32_t act, void* out, void* workspace,
-                                      size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events) {
+namespace {
+static int packed_impl(const void* x, const void* gate_up_packed, const float* gate_up_bias,
+                       const void* down_packed, const float* down_bias, const void* indices,
+                       const void* weights, int types, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
+                       int32_t bias_layout, int32_t act, void* out, void* workspace,
+                       size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events) {
     int st = common_checks(x, gate_up_packed, down_packed, indices, weights, T, H, F, E, K, bias_layout, act, out,
-                           workspace);
+                           workspace, types);
     if (st != CERNELS_MOE_OK || T == 0) return st;
     if (H % 64 || F % 64 || E > kMaxExperts) return CERNELS_MOE_UNSUPPORTED_SHAPE;
     if (!act_gated(act) && gate_up_bias) return CERNELS_MOE_UNSUPPORTED_SHAPE;  // non-gated: no bias
@@ -257,13 +270,35 @@ int cernels_moe_experts_packed_staged(const void* x, const void* gate_up_packed,
     if (workspace_bytes < w.total) return CERNELS_MOE_WORKSPACE_TOO_SMALL;
     char* base = static_cast<char*>(workspace);
     return hip_status(cmoe::launch_prefill_packed(
-        x, gate_up_packed, gate_up_bias, down_packed, down_bias, indices, weights, T, H, F, E, K,
+        x, gate_up_packed, gate_up_bias, down_packed, down_bias, static_cast<const int32_t*>(indices), weights, types,
+        reinterpret_cast<int32_t*>(base + w.idx32), reinterpret_cast<float*>(base + w.w32), T, H, F, E, K,
         bias_layout == CERNELS_MOE_LAYOUT_INTERLEAVED, act, out, reinterpret_cast<int32_t*>(base + w.offsets),
         reinterpret_cast<int32_t*>(base + w.tile_offsets), reinterpret_cast<int32_t*>(base + w.meta),
         reinterpret_cast<int32_t*>(base + w.sorted_pairs), reinterpret_cast<int32_t*>(base + w.tile_expert),
         reinterpret_cast<int32_t*>(base + w.route_counts), w.capacity, reinterpret_cast<uint16_t*>(base + w.glu),
         reinterpret_cast<float*>(base + w.Y), reinterpret_cast<int8_t*>(base + w.gexp), reinterpret_cast<int8_t*>(base + w.rsig),
         reinterpret_cast<int8_t*>(base + w.psig), reinterpret_cast<unsigned char*>(base + w.few), stream, stage_events));
+}
+}  // namespace
+
+int cernels_moe_experts_packed_staged(const void* x, const void* gate_up_packed, const float* gate_up_bias,
+                                      const void* down_packed, const float* down_bias, const int32_t* indices,
+                                      const float* weights, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
+                                      int32_t bias_layout, int32_t act, void* out, void* workspace,
+                                      size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events) {
+    return packed_impl(x, gate_up_packed, gate_up_bias, down_packed, down_bias, indices, weights, 0, T, H, F, E, K, bias_layout,
+                       act, out, workspace, workspace_bytes, stream, stage_events);
+}
+
+int cernels_moe_experts_packed_typed(const void* x, const void* gate_up_packed, const float* gate_up_bias,
+                                     const void* down_packed, const float* down_bias, const void* indices,
+                                     int32_t index_type, const void* weights, int32_t weight_type, int32_t T, int32_t H,
+                                     int32_t F, int32_t E, int32_t K, int32_t bias_layout, int32_t act, void* out,
+                                     void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const int types = pair_types(index_type, weight_type);
+    if (types < 0) return CERNELS_MOE_INVALID_ARGUMENT;
+    return packed_impl(x, gate_up_packed, gate_up_bias, down_packed, down_bias, indices, weights, types, T, H, F, E, K,
+                       bias_layout, act, out, workspace, workspace_bytes, stream, nullptr);
 }
 
 int cernels_moe_experts_packed(const void* x, const void* gate_up_packed, const float* gate_up_bias,
@@ -337,14 +372,30 @@ size_t cernels_moe_experts_decode_workspace_bytes(int32_t T, int32_t H, int32_t 
 
 namespace {
 // Every check of the decode entry except the workspace's size, in the entry's order.
-static int decode_checks(const void* x, const void* w1, const void* w2, const int32_t* idx, const float* wts, int T,
-                         int H, int F, int E, int K, int layout, int act, void* out, const void* ws) {
-    int st = common_checks(x, w1, w2, idx, wts, T, H, F, E, K, layout, act, out, const_cast<void*>(ws));
+static int decode_checks(const void* x, const void* w1, const void* w2, const void* idx, const void* wts, int T,
+                         int H, int F, int E, int K, int layout, int act, void* out, const void* ws, int types = 0) {
+    int st = common_checks(x, w1, w2, idx, wts, T, H, F, E, K, layout, act, out, const_cast<void*>(ws), types);
     if (st != CERNELS_MOE_OK || T == 0) return st;
     if (layout != CERNELS_MOE_LAYOUT_CONCAT || !act_gated(act)) return CERNELS_MOE_UNSUPPORTED_SHAPE;
     if (T > cmoe::decode_max_tokens() || T * K > cmoe::decode_max_pairs()) return CERNELS_MOE_UNSUPPORTED_SHAPE;
     if (H % 8 || F % 8 || E > kMaxExperts || !cmoe::decode_shape_supported(H, F)) return CERNELS_MOE_UNSUPPORTED_SHAPE;
     return CERNELS_MOE_OK;
+}
+
+static int decode_impl(const void* x, const void* w1, const float* b1, const void* w2, const float* b2, const void* idx,
+                       const void* wts, int types, int T, int H, int F, int E, int K, int layout, int act, void* out, void* ws,
+                       size_t ws_bytes, hipStream_t stream, hipEvent_t* ev) {
+    const int st = decode_checks(x, w1, w2, idx, wts, T, H, F, E, K, layout, act, out, ws, types);
+    if (st != CERNELS_MOE_OK || T == 0) return st;
+    const DecodeWs w = decode_ws(T, H, F, K);
+    const bool bf16_weights = types & 2;
+    if (ws_bytes < (bf16_weights ? w.total : w.total_f32)) return CERNELS_MOE_WORKSPACE_TOO_SMALL;
+    char* base = static_cast<char*>(ws);
+    return hip_status(cmoe::launch_decode(
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), b1, static_cast<const uint16_t*>(w2), b2,
+        static_cast<const int32_t*>(idx), wts, types, reinterpret_cast<uint16_t*>(base + w.glu),
+        reinterpret_cast<int32_t*>(base + w.order), bf16_weights ? reinterpret_cast<float*>(base + w.order_w) : nullptr,
+        static_cast<uint16_t*>(out), T, H, F, E, K, act, stream, ev));
 }
 }  // namespace
 
@@ -353,17 +404,19 @@ int cernels_moe_experts_decode_staged(const void* x, const void* gate_up_proj, c
                                       const float* weights, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
                                       int32_t layout, int32_t act, void* out, void* workspace,
                                       size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events) {
-    int st = decode_checks(x, gate_up_proj, down_proj, indices, weights, T, H, F, E, K, layout, act, out, workspace);
-    if (st != CERNELS_MOE_OK || T == 0) return st;
-    const DecodeWs w = decode_ws(T, H, F, K);
-    if (workspace_bytes < w.total) return CERNELS_MOE_WORKSPACE_TOO_SMALL;
-    char* base = static_cast<char*>(workspace);
-    return hip_status(cmoe::launch_decode(
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(gate_up_proj), gate_up_bias,
-        static_cast<const uint16_t*>(down_proj), down_bias, indices, weights,
-        reinterpret_cast<uint16_t*>(base + w.glu), reinterpret_cast<int32_t*>(base + w.order),
-        static_cast<uint16_t*>(out), T, H, F, E, K, act, stream,
-        stage_events));
+    return decode_impl(x, gate_up_proj, gate_up_bias, down_proj, down_bias, indices, weights, 0, T, H, F, E, K, layout, act, out,
+                       workspace, workspace_bytes, stream, stage_events);
+}
+
+int cernels_moe_experts_decode_typed(const void* x, const void* gate_up_proj, const float* gate_up_bias,
+                                     const void* down_proj, const float* down_bias, const void* indices,
+                                     int32_t index_type, const void* weights, int32_t weight_type, int32_t T, int32_t H,
+                                     int32_t F, int32_t E, int32_t K, int32_t layout, int32_t act, void* out,
+                                     void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const int types = pair_types(index_type, weight_type);
+    if (types < 0) return CERNELS_MOE_INVALID_ARGUMENT;
+    return decode_impl(x, gate_up_proj, gate_up_bias, down_proj, down_bias, indices, weights, types, T, H, F, E, K, layout, act,
+                       out, workspace, workspace_bytes, stream, nullptr);
 }
 
 int cernels_moe_experts_decode(const void* x, const void* gate_up_proj, const float* gate_up_bias,
@@ -387,7 +440,7 @@ int cernels_moe_experts_decode_noalloc(const void* x, const void* gate_up_proj, 
     const int st = decode_checks(x, gate_up_proj, down_proj, indices, weights, T, H, F, E, K, layout, act, out,
                                  kStandIn);
     if (st != CERNELS_MOE_OK || T == 0) return st;
-    if (decode_ws(T, H, F, K).total > cmoe::decode_noalloc_bytes()) return CERNELS_MOE_WORKSPACE_TOO_SMALL;
+    if (decode_ws(T, H, F, K).total_f32 > cmoe::decode_noalloc_bytes()) return CERNELS_MOE_WORKSPACE_TOO_SMALL;
     void* ws = nullptr;
     if (cmoe::decode_noalloc_scratch(&ws) != hipSuccess) return CERNELS_MOE_HIP_ERROR;
     return cernels_moe_experts_decode_staged(x, gate_up_proj, gate_up_bias, down_proj, down_bias, indices, weights,

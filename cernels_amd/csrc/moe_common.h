@@ -83,6 +83,18 @@ __device__ __forceinline__ float act_plain(float h) {
     }
 }
 
+// How a call's routing arrives: expert ids as int32 or int64 (kPairsI64; the low 32 bits are the id, as a cast to int32
+// takes them), routing weights as fp32 or bf16 (kPairsBf16). Routers hand over int64 and bf16; reading them as they are
+// saves two cast launches per call (about 5 us each in a stream of short kernels).
+constexpr int kPairsI64 = 1;
+constexpr int kPairsBf16 = 2;
+__device__ __forceinline__ int pair_id(const int32_t* __restrict__ idx, int types, int p) {
+    return idx[(long long)p << (types & kPairsI64)];
+}
+__device__ __forceinline__ float pair_weight(const void* __restrict__ w, int types, long long p) {
+    return types & kPairsBf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(w)[p]) : static_cast<const float*>(w)[p];
+}
+
 // Two fp32 values -> two round-to-nearest-even bf16 in one dword (low half = a).
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return (uint32_t)f32_to_bf16_bits(a) | ((uint32_t)f32_to_bf16_bits(b) << 16);

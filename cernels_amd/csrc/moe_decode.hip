@@ -125,8 +125,8 @@ __device__ __forceinline__ void wave_reduce_groups(float (&v)[N], int lane) {
 template <int ACT, bool HAS_BIAS, int MAXC, int R>
 __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1, const float* __restrict__ b1,
-    const int32_t* __restrict__ idx, uint16_t* __restrict__ glu, int32_t* __restrict__ order, int T, int H, int F,
-    int E, int K) {
+    const int32_t* __restrict__ idx, const void* __restrict__ route_w, int types, uint16_t* __restrict__ glu,
+    int32_t* __restrict__ order, float* __restrict__ order_w, int T, int H, int F, int E, int K) {
     __shared__ uint32_t bits[kDecWaves][kDecMaxExperts / 32];
     __shared__ int plist[kDecWaves][kDecMaxPairs];
     const int lane = threadIdx.x & (kWave - 1);
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
 #pragma unroll
     for (int c = 0; c < kDecMaxPairs / kWave; ++c) {
         const int p = lane + kWave * c;
-        const int v = p < P ? idx[p] : -1;
+        const int v = p < P ? pair_id(idx, types, p) : -1;
         ev[c] = ((unsigned)v < (unsigned)E) ? v : -1;
     }
     // Wave 0 of the first row group of each expert publishes that expert's pairs in the pair order the down
@@ -191,7 +191,10 @@ __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
         if (mine) {
             const int at = np + __popcll(mk & lt);
             plist[wave][at] = kWave * c + lane;
-            if (lead) order[base + at] = (e << 16) | (kWave * c + lane);
+            if (lead) {
+                order[base + at] = (e << 16) | (kWave * c + lane);
+                if (order_w) order_w[base + at] = pair_weight(route_w, types, kWave * c + lane);
+            }
         }
         np += __popcll(mk);
     }
@@ -260,8 +263,8 @@ __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
 template <bool HAS_BIAS, int MAXC, int QB, int HB>
 __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
     const uint16_t* __restrict__ glu, const uint16_t* __restrict__ w2, const float* __restrict__ b2,
-    const int32_t* __restrict__ order, const float* __restrict__ route_w, uint16_t* __restrict__ out, int T, int H,
-    int F, int K) {
+    const int32_t* __restrict__ order, const float* __restrict__ route_w, int by_order, uint16_t* __restrict__ out, int T,
+    int H, int F, int K) {
     static_assert(QB == 1 || QB == 2, "pairs per batch");
     __shared__ float part[kDnWaves][HB][kDecMaxTokens];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -326,7 +329,7 @@ __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
         for (int q = 0; q < QB; ++q) {
             if (q == 1 && !two) break;  // wave-uniform
             const int pp = q == 0 ? p0 : p1, ee = q == 0 ? e0 : e1;
-            const float wp = route_w[pp];
+            const float wp = route_w[by_order ? i + q : pp];
             const int t = pp / K;
 #pragma unroll
             for (int j = 0; j < HB; ++j) {
@@ -357,11 +360,11 @@ int decode_max_pairs() { return kDecMaxPairs; }
 int decode_max_tokens() { return kDecMaxTokens; }
 
 template <int ACT, bool HAS_BIAS, int MAXC, int R>
-static void launch_gateup_r(const uint16_t* x, const uint16_t* w1, const float* b1, const int32_t* idx, uint16_t* glu,
-                            int32_t* order, int T, int H, int F, int E, int K, hipStream_t s) {
+static void launch_gateup_r(const uint16_t* x, const uint16_t* w1, const float* b1, const int32_t* idx, const void* w,
+                            int types, uint16_t* glu, int32_t* order, float* order_w, int T, int H, int F, int E, int K, hipStream_t s) {
     dim3 grid(ceil_div(F, kDecWaves * R), min(T * K, E));
     hipLaunchKernelGGL((moe_decode_gateup_kernel<ACT, HAS_BIAS, MAXC, R>), grid, dim3(kDecThreads), 0, s, x, w1, b1,
-                       idx, glu, order, T, H, F, E, K);
+                       idx, w, types, glu, order, order_w, T, H, F, E, K);
 }
 
 static int g_dec_cu_count = 0;
@@ -382,9 +385,9 @@ static int dec_cu_count() {
 // workloads: R = 4 (eight rows, fewer and larger workgroups) was 2.5 us slower at T=8, H=1280 and
 // 1.4 us slower at T=1, H=2048; R = 1 was within noise of R = 2.
 template <int ACT, bool HAS_BIAS, int MAXC>
-static void launch_gateup_t(const uint16_t* x, const uint16_t* w1, const float* b1, const int32_t* idx, uint16_t* glu,
-                            int32_t* order, int T, int H, int F, int E, int K, hipStream_t s) {
-    launch_gateup_r<ACT, HAS_BIAS, MAXC, 2>(x, w1, b1, idx, glu, order, T, H, F, E, K, s);
+static void launch_gateup_t(const uint16_t* x, const uint16_t* w1, const float* b1, const int32_t* idx, const void* w,
+                            int types, uint16_t* glu, int32_t* order, float* order_w, int T, int H, int F, int E, int K, hipStream_t s) {
+    launch_gateup_r<ACT, HAS_BIAS, MAXC, 2>(x, w1, b1, idx, w, types, glu, order, order_w, T, H, F, E, K, s);
 }
 
 // QB (pairs per batch) is 2 while rows are short (F <= 2048) and a wave has more than one pair, else 1, to bound
@@ -393,23 +396,23 @@ static void launch_gateup_t(const uint16_t* x, const uint16_t* w1, const float* 
 // three workgroups per CU resident, so T=8's 640 workgroups (H=1280) run in one wave of residency.
 template <bool HAS_BIAS, int MAXC, int QB, int HB>
 static void launch_down_k(const uint16_t* glu, const uint16_t* w2, const float* b2, const int32_t* order,
-                          const float* route_w, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
+                          const float* route_w, int by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
     hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB>), dim3(ceil_div(H, HB)), dim3(kDnThreads), 0, s,
-                       glu, w2, b2, order, route_w, out, T, H, F, K);
+                       glu, w2, b2, order, route_w, by_order, out, T, H, F, K);
 }
 template <bool HAS_BIAS, int MAXC>
 static void launch_down_t(const uint16_t* glu, const uint16_t* w2, const float* b2, const int32_t* order,
-                          const float* route_w, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
+                          const float* route_w, int by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
     const bool one = T * K <= kDnWaves;  // at most one pair per wave
     if constexpr (MAXC <= 2) {
         if (H / 4 >= 2 * dec_cu_count()) {
-            if (one) launch_down_k<HAS_BIAS, MAXC, 1, 4>(glu, w2, b2, order, route_w, out, T, H, F, K, s);
-            else launch_down_k<HAS_BIAS, MAXC, 2, 4>(glu, w2, b2, order, route_w, out, T, H, F, K, s);
+            if (one) launch_down_k<HAS_BIAS, MAXC, 1, 4>(glu, w2, b2, order, route_w, by_order, out, T, H, F, K, s);
+            else launch_down_k<HAS_BIAS, MAXC, 2, 4>(glu, w2, b2, order, route_w, by_order, out, T, H, F, K, s);
             return;
         }
     }
-    if (one || MAXC > 4) launch_down_k<HAS_BIAS, MAXC, 1, 2>(glu, w2, b2, order, route_w, out, T, H, F, K, s);
-    else launch_down_k<HAS_BIAS, MAXC, (MAXC <= 4 ? 2 : 1), 2>(glu, w2, b2, order, route_w, out, T, H, F, K, s);
+    if (one || MAXC > 4) launch_down_k<HAS_BIAS, MAXC, 1, 2>(glu, w2, b2, order, route_w, by_order, out, T, H, F, K, s);
+    else launch_down_k<HAS_BIAS, MAXC, (MAXC <= 4 ? 2 : 1), 2>(glu, w2, b2, order, route_w, by_order, out, T, H, F, K, s);
 }
 
 // MAXC = 16-byte chunks per lane per row = ceil(len / 512); supported up to 8 (len <= 4096).
@@ -425,12 +428,12 @@ static int pick_maxc(int len) {
 }
 
 #define CMOE_DEC_GU(ACT, BIAS, C) \
-    case C: launch_gateup_t<ACT, BIAS, C>(x, w1, b1, idx, glu, order, T, H, F, E, K, s); break;
+    case C: launch_gateup_t<ACT, BIAS, C>(x, w1, b1, idx, w, types, glu, order, order_w, T, H, F, E, K, s); break;
 #define CMOE_DEC_GU_ALL(ACT, BIAS) \
     switch (cg) { CMOE_DEC_GU(ACT, BIAS, 1) CMOE_DEC_GU(ACT, BIAS, 2) CMOE_DEC_GU(ACT, BIAS, 3) \
                   CMOE_DEC_GU(ACT, BIAS, 4) CMOE_DEC_GU(ACT, BIAS, 6) CMOE_DEC_GU(ACT, BIAS, 8) default: break; }
 #define CMOE_DEC_DN(BIAS, C) \
-    case C: launch_down_t<BIAS, C>(glu, w2, b2, order, route_w, out, T, H, F, K, s); break;
+    case C: launch_down_t<BIAS, C>(glu, w2, b2, order, route_w, by_order, out, T, H, F, K, s); break;
 #define CMOE_DEC_DN_ALL(BIAS) \
     switch (cd) { CMOE_DEC_DN(BIAS, 1) CMOE_DEC_DN(BIAS, 2) CMOE_DEC_DN(BIAS, 3) CMOE_DEC_DN(BIAS, 4) \
                   CMOE_DEC_DN(BIAS, 6) CMOE_DEC_DN(BIAS, 8) default: break; }
@@ -438,9 +441,12 @@ static int pick_maxc(int len) {
 bool decode_shape_supported(int H, int F) { return pick_maxc(H) > 0 && pick_maxc(F) > 0; }
 
 hipError_t launch_decode(const uint16_t* x, const uint16_t* w1, const float* b1, const uint16_t* w2, const float* b2,
-                         const int32_t* idx, const float* route_w, uint16_t* glu, int32_t* order, uint16_t* out,
-                         int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev) {
-    // ev (optional): 3 events recorded before gate_up, after gate_up, after down.
+                         const int32_t* idx, const void* w, int types, uint16_t* glu, int32_t* order, float* order_w,
+                         uint16_t* out, int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev) {
+    // ev (optional): 3 events recorded before gate_up, after gate_up, after down. order_w (required for bf16 weights): the
+    // down GEMV then reads the weights from there, fp32 in the pair order that gate_up writes.
+    const float* route_w = order_w ? order_w : static_cast<const float*>(w);
+    const int by_order = order_w != nullptr;
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     if (E > kDecMaxExperts) return hipErrorInvalidValue;
     const int cg = pick_maxc(H), cd = pick_maxc(F);

@@ -431,13 +431,14 @@ hipError_t launch_down(const GemmParams& prm, int layout, bool has_bias, int max
 }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
-                            const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
-                            hipStream_t s);
+                            const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
+                            hipStream_t s, int types = 0);
 
 hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t* offsets, int32_t* sorted_pairs,
                         int32_t* tile_offsets, int32_t* tile_expert, int32_t* meta, int32_t* counts,
                         int32_t* sched, hipStream_t stream, int8_t* row_zero = nullptr,
-                        const XcdSplit* split = nullptr);
+                        const XcdSplit* split = nullptr, int types = 0, const void* route_w = nullptr,
+                        int32_t* idx32 = nullptr, float* w32 = nullptr);
 
 // route -> gate_up GEMM -> down GEMM -> combine, all on stream s. Shapes were checked by the caller
 // (H % 64 == 0, F % 64 == 0, E <= 1024, T >= 1).

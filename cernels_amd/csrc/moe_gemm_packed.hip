@@ -892,7 +892,8 @@ static hipError_t launch_pk_t(const PkParams& prm, int max_tiles, hipStream_t s)
 hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t* offsets, int32_t* sorted_pairs,
                         int32_t* tile_offsets, int32_t* tile_expert, int32_t* meta, int32_t* counts,
                         int32_t* sched, hipStream_t stream, int8_t* row_zero = nullptr,
-                        const XcdSplit* split = nullptr);
+                        const XcdSplit* split = nullptr, int types = 0, const void* route_w = nullptr,
+                        int32_t* idx32 = nullptr, float* w32 = nullptr);
 // out[t, :] = bf16( sum over valid slots k of Y[t*K + k, :] * 2^psig + w[t, k] * b2[e] ), slots in k
 // order, Y in the 24-bit float form both down GEMMs write (the packed one: w * glu W2, without the bias;
 // psig only when some glu row was stored scaled, i.e. sync non-null and sync[1] set; the stored-layout one:
@@ -904,7 +905,7 @@ __global__ __launch_bounds__(1024) void moe_combine_h_kernel(const unsigned char
                                                             int T, int K, int E, int H,
                                                             const int32_t* __restrict__ sync,
                                                             const int8_t* __restrict__ psig,
-                                                            const float* __restrict__ bias, const float* __restrict__ route_w) {
+                                                            const float* __restrict__ bias, const void* __restrict__ route_w, int types) {
     const int t = blockIdx.x;
     const bool scaled = sync != nullptr && sync[1] != 0;  // some glu row was stored scaled: its Y row is scaled by 2^-psig
     for (int c = threadIdx.x; c < H / 8; c += blockDim.x) {
@@ -915,7 +916,7 @@ __global__ __launch_bounds__(1024) void moe_combine_h_kernel(const unsigned char
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int k = k0 + j;
-                ev[j] = k < K ? idx[t * K + k] : -1;
+                ev[j] = k < K ? pair_id(idx, types, t * K + k) : -1;
                 if ((unsigned)ev[j] < (unsigned)E) {
                     const unsigned char* src = Yb + (((long long)t * K + k) * H + 8 * c) * 3;
                     __builtin_memcpy(&q[j][0], src, 12);
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(1024) void moe_combine_h_kernel(const unsigned char
                     y1 *= sc;
                 }
                 if (bias) {  // the slot's share of the down bias, w * b[e]
-                    const float w = route_w[(long long)t * K + k];
+                    const float w = pair_weight(route_w, types, (long long)t * K + k);
                     const f32x4* bb = reinterpret_cast<const f32x4*>(bias + (long long)e * H + 8 * c);
                     y0 += w * bb[0];
                     y1 += w * bb[1];
@@ -1011,13 +1012,13 @@ static int pick_fw(long long P, int E, int NF, int Kd, int cus) {
 }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
-                            const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
-                            hipStream_t s);
+                            const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
+                            hipStream_t s, int types = 0);
 
 bool few_supported(int T, int K, int E);
 bool tiles_supported(int T, int K, int E);
 hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
-                      const float* route_w, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
+                      const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
                       uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev);
 int stream_tile_m();
 hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
@@ -1033,22 +1034,25 @@ hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float
 // forms of moe_stream.hip instead (its header states where the lines lie and why). Shapes were checked
 // by the caller (H % 64 == 0, F % 64 == 0, E <= 1024, T >= 1).
 hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2,
-                                 const int32_t* idx, const float* route_w, int T, int H, int F, int E, int K,
-                                 int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
+                                 const int32_t* idx_in, const void* w_in, int types, int32_t* idx32, float* w32, int T, int H,
+                                 int F, int E, int K, int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
                                  int32_t* meta, int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts,
                                  int max_tiles, uint16_t* glu, float* Y, int8_t* gexp, int8_t* rsig,
                                  int8_t* psig, unsigned char* few_lists, hipStream_t s, hipEvent_t* ev) {
     if (few_supported(T, K, E))
-        return launch_few(x, w1p, b1, w2p, b2, idx, route_w, T, H, F, E, K, bias_interleaved, act, out, glu, gexp,
+        return launch_few(x, w1p, b1, w2p, b2, idx_in, w_in, types, T, H, F, E, K, bias_interleaved, act, out, glu, gexp,
                           reinterpret_cast<unsigned char*>(Y), few_lists, s, ev);
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
+    // what the kernels after the route read: the caller's arrays, or the int32 / fp32 ones that the route leaves
+    const int32_t* idx = types ? idx32 : idx_in;
+    const float* route_w = types ? w32 : static_cast<const float*>(w_in);
     if (tiles_supported(T, K, E)) {  // moe_stream.hip
         const int bm = stream_tile_m();
         const long long P = (long long)T * K;
         const int tiles = (int)((P + bm - 1) / bm + std::min<long long>(P, E));
         mark(0);
-        hipError_t st = launch_route(idx, T, K, E, bm, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
-                                     meta + 8, s, rsig, nullptr);
+        hipError_t st = launch_route(idx_in, T, K, E, bm, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
+                                     meta + 8, s, rsig, nullptr, types, w_in, idx32, w32);
         if (st != hipSuccess) return st;
         mark(1);
         st = launch_stream_gemm1(x, w1p, b1, T, H, F, E, K, bias_interleaved, act, offsets, tile_offsets, meta, sorted_pairs,
@@ -1083,8 +1087,8 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     XcdSplit split{{fw1, fw2}, {nt1, nt2}, {slots1, slots2}, meta + 32};
     mark(0);
     hipError_t st =
-        launch_route(idx, T, K, E, kPkBM, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
-                     meta + 8, s, rsig, cost_split ? &split : nullptr);
+        launch_route(idx_in, T, K, E, kPkBM, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
+                     meta + 8, s, rsig, cost_split ? &split : nullptr, types, w_in, idx32, w32);
     if (st != hipSuccess) return st;
     mark(1);
     PkParams g1{};
@@ -1157,11 +1161,11 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
 }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
-                            const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
-                            hipStream_t s) {
+                            const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
+                            hipStream_t s, int types) {
     if (T == 0) return hipSuccess;
     hipLaunchKernelGGL(moe_combine_h_kernel, dim3(T), dim3(std::min(1024, ceil_div(H / 8, kWave) * kWave)), 0, s, Y,
-                       idx, out, T, K, E, H, sync, psig, b2, route_w);
+                       idx, out, T, K, E, H, sync, psig, b2, route_w, types);
     return hipGetLastError();
 }
 

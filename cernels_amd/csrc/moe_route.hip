@@ -85,9 +85,10 @@ __device__ __forceinline__ int div_by_t(int q, int T, float rT) {
     return k + (r >= T ? 1 : 0) - (r < 0 ? 1 : 0);
 }
 
+template <int IS = 1>  // ints per id: 2 for int64
 __device__ __forceinline__ int expert_at(const int32_t* __restrict__ idx, int q, int T, int K, int E, float rT) {
     const int k = div_by_t(q, T, rT), t = q - k * T;
-    const int v = idx[t * K + k];
+    const int v = idx[(long long)(t * K + k) * IS];
     return ((unsigned)v < (unsigned)E) ? v : -1;
 }
 
@@ -305,8 +306,12 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_count_scan_kernel(
 constexpr int kRtChunks = 8;           // 16-byte idx chunks per thread and round of the histogram pass
 constexpr int kRtOneCells = 39 * 1024;  // LDS cells: ntiles * E histograms + 16 * E wave cursors (156 KiB)
 
+// IS: ints per id (2: int64). With idx32 the workgroups also leave the ids as int32 and the weights as fp32 there and
+// in w32, one tile of pairs in memory order each, for the kernels that follow.
+template <int IS>
 __global__ __launch_bounds__(kRouteThreads) void moe_route_one_kernel(
-    const int32_t* __restrict__ idx, int T, int K, int E, int BM, int ntiles, int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ idx, const void* __restrict__ route_w, int types, int32_t* __restrict__ idx32,
+    float* __restrict__ w32, int T, int K, int E, int BM, int ntiles, int32_t* __restrict__ offsets,
     int32_t* __restrict__ sorted_pairs, int32_t* __restrict__ tile_offsets, int32_t* __restrict__ tile_expert,
     int32_t* __restrict__ meta, int32_t* __restrict__ sched, int8_t* __restrict__ row_zero, XcdSplit split) {
     extern __shared__ int32_t rt_lds[];
@@ -320,13 +325,19 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_one_kernel(
     const float rT = 1.0f / (float)T;
     for (int i = tid; i < (ntiles + kRouteWaves) * E; i += kRouteThreads) rt_lds[i] = 0;
     const int q = blockIdx.x * kRtTile + w * kWave + lane;
-    const int eq = q < P ? expert_at(idx, q, T, K, E, rT) : -1;
+    const int eq = q < P ? expert_at<IS>(idx, q, T, K, E, rT) : -1;
+    const int pm = blockIdx.x * kRtTile + tid;
+    if (idx32 && pm < P) {
+        idx32[pm] = idx[(long long)pm * IS];
+        w32[pm] = pair_weight(route_w, types, pm);
+    }
     __syncthreads();
     const double rK = 1.0 / (double)K;
-    const int nchunks = ceil_div(P, 4);
-    // idx in 16-byte chunks through a buffer descriptor (P * 4 < 2^31 on this path): one load
+    constexpr int PC = 4 / IS;  // pairs per chunk
+    const int nchunks = ceil_div(P, PC);
+    // idx in 16-byte chunks through a buffer descriptor (P * 8 < 2^31 on this path): one load
     // instruction per chunk, the tail of the last chunk reads 0 and is masked by i + v < P
-    const __amdgpu_buffer_rsrc_t ridx = __builtin_amdgcn_make_buffer_rsrc((void*)idx, (short)0, P * 4, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t ridx = __builtin_amdgcn_make_buffer_rsrc((void*)idx, (short)0, P * 4 * IS, kBufferWord3);
     for (int c0 = tid; c0 < nchunks; c0 += kRtChunks * kRouteThreads) {
         u32x4 ev[kRtChunks];
 #pragma unroll
@@ -335,14 +346,14 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_one_kernel(
                                                   ridx, (uint32_t)(c0 + u * kRouteThreads) * 16u, 0, 0));
 #pragma unroll
         for (int u = 0; u < kRtChunks; ++u) {
-            const int i = 4 * (c0 + u * kRouteThreads);
+            const int i = PC * (c0 + u * kRouteThreads);
             if (i >= P) continue;
             int t = (int)((double)i * rK), k = i - t * K;
             t += (k >= K ? 1 : 0) - (k < 0 ? 1 : 0);
             k = i - t * K;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int e = (int)ev[u][v];
+            for (int v = 0; v < PC; ++v) {
+                const int e = (int)ev[u][v * IS];
                 if (i + v < P && (unsigned)e < (unsigned)E) atomicAdd(&h[((k * T + t) / kRtTile) * E + e], 1);
                 if (++k == K) {
                     k = 0;
@@ -410,27 +421,53 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_one_kernel(
     }
 }
 
+// The ids as int32 and the weights as fp32, for the routes of more than one launch.
+__global__ __launch_bounds__(kRtThreads) void moe_pairs_kernel(const int32_t* __restrict__ idx, const void* __restrict__ route_w,
+                                                               int types, int P, int32_t* __restrict__ idx32,
+                                                               float* __restrict__ w32) {
+    const int p = blockIdx.x * kRtThreads + threadIdx.x;
+    if (p >= P) return;
+    idx32[p] = pair_id(idx, types, p);
+    w32[p] = pair_weight(route_w, types, p);
+}
+
 int route_tiles(int T, int K) { return ceil_div(T * K, kRtTile); }
 size_t route_workspace_bytes(int T, int K, int E) { return (size_t)max(route_tiles(T, K), 1) * E * sizeof(int32_t); }
 
+template <int IS>
+static hipError_t launch_route_one(const int32_t* idx, const void* route_w, int types, int32_t* idx32, float* w32, int T, int K,
+                                   int E, int BM, int nt, int32_t* offsets, int32_t* sorted_pairs, int32_t* tile_offsets,
+                                   int32_t* tile_expert, int32_t* meta, int32_t* sched, hipStream_t stream, int8_t* row_zero,
+                                   const XcdSplit& sp) {
+    static bool lds_attr = false;  // dynamic LDS above 64 KiB must be allowed once per process
+    if (!lds_attr) {
+        const hipError_t st = hipFuncSetAttribute((const void*)moe_route_one_kernel<IS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  kRtOneCells * (int)sizeof(int32_t));
+        if (st != hipSuccess) return st;
+        lds_attr = true;
+    }
+    hipLaunchKernelGGL(moe_route_one_kernel<IS>, dim3(nt + 1), dim3(kRouteThreads),
+                       (size_t)(nt + kRouteWaves) * E * sizeof(int32_t), stream, idx, route_w, types, idx32, w32, T, K, E, BM, nt,
+                       offsets, sorted_pairs, tile_offsets, tile_expert, meta, sched, row_zero, sp);
+    return hipGetLastError();
+}
+
+// types, route_w, idx32, w32: with types != 0 the route also writes the pairs' ids and weights as int32 and fp32.
 hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t* offsets, int32_t* sorted_pairs,
                         int32_t* tile_offsets, int32_t* tile_expert, int32_t* meta, int32_t* counts,
-                        int32_t* sched, hipStream_t stream, int8_t* row_zero, const XcdSplit* split) {
+                        int32_t* sched, hipStream_t stream, int8_t* row_zero, const XcdSplit* split, int types,
+                        const void* route_w, int32_t* idx32, float* w32) {
     const int nt = route_tiles(T, K);
     const XcdSplit sp = split ? *split : XcdSplit{};
-    if (nt > 0 && (long long)(nt + kRouteWaves) * E <= kRtOneCells) {
-        static bool lds_attr = false;  // dynamic LDS above 64 KiB must be allowed once per process
-        if (!lds_attr) {
-            const hipError_t st = hipFuncSetAttribute((const void*)moe_route_one_kernel,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                      kRtOneCells * (int)sizeof(int32_t));
-            if (st != hipSuccess) return st;
-            lds_attr = true;
-        }
-        hipLaunchKernelGGL(moe_route_one_kernel, dim3(nt + 1), dim3(kRouteThreads),
-                           (size_t)(nt + kRouteWaves) * E * sizeof(int32_t), stream, idx, T, K, E, BM, nt, offsets,
-                           sorted_pairs, tile_offsets, tile_expert, meta, sched, row_zero, sp);
-        return hipGetLastError();
+    if (types == 0) idx32 = nullptr;
+    if (nt > 0 && (long long)(nt + kRouteWaves) * E <= kRtOneCells)
+        return (types & kPairsI64 ? launch_route_one<2> : launch_route_one<1>)(idx, route_w, types, idx32, w32, T, K, E, BM, nt,
+                                                                               offsets, sorted_pairs, tile_offsets, tile_expert,
+                                                                               meta, sched, stream, row_zero, sp);
+    if (types != 0 && nt > 0) {
+        hipLaunchKernelGGL(moe_pairs_kernel, dim3(ceil_div(T * K, kRtThreads)), dim3(kRtThreads), 0, stream, idx, route_w, types,
+                           T * K, idx32, w32);
+        idx = idx32;
     }
     if ((long long)nt * E <= kRtFusedCells) {
         hipLaunchKernelGGL(moe_route_count_scan_kernel, dim3(1), dim3(kRouteThreads), 0, stream, idx, T, K, E, BM, nt,

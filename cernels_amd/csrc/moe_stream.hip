@@ -54,7 +54,8 @@ struct StreamParams {
     const uint16_t* B;            // packed weights of this projection
     const float* bias;            // first: [E, 2F]; few down: [E, H]; or null
     const int32_t* idx;           // few: [T, K]
-    const float* route_w;         // [T, K]
+    const void* route_w;          // [T, K]
+    int types;                    // of idx and route_w (kPairsI64, kPairsBf16); tiles: 0
     const int32_t* sorted_pairs;  // tiles: the route's lists
     const int32_t* offsets;
     const int32_t* tile_offsets;
@@ -150,7 +151,7 @@ __device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, in
 // few: the u-th smallest distinct expert of the indices (-1: fewer than u + 1), and in tokp[t] the first pair of token t
 // that names it, with bit 16 set if further pairs of t do (INT_MAX: none). One wave by itself: its own LDS words (a wave's LDS operations run in order), no
 // workgroup barrier.
-__device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int P, int E, int K, int u, int lane,
+__device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int types, int P, int E, int K, int u, int lane,
                                           uint32_t* bits, int* tokp) {
     int ev[kFewMaxPairs / kWave];
 #pragma unroll
@@ -158,7 +159,7 @@ __device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int P
         ev[c] = -1;
         if (kWave * c < P) {  // uniform
             const int p = lane + kWave * c;
-            const int v = p < P ? idx[p] : -1;
+            const int v = p < P ? pair_id(idx, types, p) : -1;
             ev[c] = (unsigned)v < (unsigned)E ? v : -1;
         }
     }
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_stream_first_kernel(StreamP
     int my_pair = INT_MAX, again = 0;  // few: this lane's token's glu row, and whether the token names e again
     uint32_t ao;
     if constexpr (FEW) {
-        e = few_select(prm.idx, prm.T * prm.K, prm.E, prm.K, blockIdx.y, lane, s_bits[wave], s_tokp[wave]);
+        e = few_select(prm.idx, prm.types, prm.T * prm.K, prm.E, prm.K, blockIdx.y, lane, s_bits[wave], s_tokp[wave]);
         if (e < 0) {  // the same in every wave
             if (fc == 0 && tid == 0) prm.few_e[blockIdx.y] = -1;
             if (tid == 0) prm.few_scaled[(long long)blockIdx.y * prm.NF + fc] = 0;
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_stream_first_kernel(StreamP
             if (lane < prm.T) {
                 float wt = 0.f;
                 for (int k = 0; k < prm.K; ++k)
-                    if (prm.idx[lane * prm.K + k] == e) wt += prm.route_w[lane * prm.K + k];
+                    if (pair_id(prm.idx, prm.types, lane * prm.K + k) == e) wt += pair_weight(prm.route_w, prm.types, lane * prm.K + k);
                 prm.few_row[u * prm.T + lane] = (int16_t)(valid ? my_pair | again << 14 : -1);
                 prm.few_w[u * prm.T + lane] = wt;
             }
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_stream_down_kernel(StreamPa
     const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
     const int row = min(lrow, rows - 1);
     const long long p = prm.sorted_pairs[row_begin + row];
-    const float ws = __builtin_amdgcn_ldexpf(prm.route_w[p], prm.wexp[(long long)e * prm.NF + fc]);
+    const float ws = __builtin_amdgcn_ldexpf(static_cast<const float*>(prm.route_w)[p], prm.wexp[(long long)e * prm.NF + fc]);
     const int nw = min(8, prm.NF - 8 * (fc >> 3));
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * nw * 1024 + 1024, kBufferWord3);
@@ -410,7 +411,7 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
     const int nst = prm.F / kBK;
     const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
     int wx = prm.wexp[(long long)e * prm.NF + fc];
-    const float rw0 = prm.route_w[p];
+    const float rw0 = pair_weight(prm.route_w, prm.types, p);
     const uint32_t ao = (uint32_t)p * (uint32_t)(prm.F * 2) + 16u * half;
     const int nw = min(8, prm.NF - 8 * (fc >> 3));
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -445,8 +446,8 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
     if (again)  // further slots of the token that name the same expert
         for (int k = 0; k < prm.K; ++k) {
             const int pp = lrow * prm.K + k;
-            if (pp != p && prm.idx[pp] == e)
-                store_y(prm.Y, pp, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(prm.route_w[pp], wx));
+            if (pp != p && pair_id(prm.idx, prm.types, pp) == e)
+                store_y(prm.Y, pp, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(pair_weight(prm.route_w, prm.types, pp), wx));
         }
 }
 
@@ -611,8 +612,8 @@ size_t few_workspace_bytes(int T, int F, int E, int K) {
 }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
-                            const int32_t* sync, const int8_t* psig, const float* b2, const float* route_w,
-                            hipStream_t s);
+                            const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
+                            hipStream_t s, int types);
 
 template <bool FEW>
 static void launch_stream_first(const StreamParams& q, int act, dim3 grid, hipStream_t s) {
@@ -631,7 +632,7 @@ static void launch_stream_first(const StreamParams& q, int act, dim3 grid, hipSt
 
 // gate_up -> down with the sum over slots, on stream s. Shapes were checked by the caller (few_supported).
 hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
-                      const float* route_w, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
+                      const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
                       uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev) {
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     const int P = T * K, um = std::min(P, E);
@@ -641,6 +642,7 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
     q.bias = b1;
     q.idx = idx;
     q.route_w = route_w;
+    q.types = types;
     q.glu = glu;
     q.gexp = gexp;
     q.few_e = reinterpret_cast<int32_t*>(lists);
@@ -674,7 +676,7 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
         st = hipGetLastError();
         if (st != hipSuccess) return st;
         mark(3);
-        st = launch_combine_h(Y, idx, static_cast<uint16_t*>(out), T, K, E, H, nullptr, nullptr, b2, route_w, s);
+        st = launch_combine_h(Y, idx, static_cast<uint16_t*>(out), T, K, E, H, nullptr, nullptr, b2, route_w, s, types);
         mark(4);
         return st;
     }

@@ -20,7 +20,7 @@ _ATTR = "_cernels_packed"
 
 
 def _key(params):
-    return tuple(None if p is None else (p.data_ptr(), p._version, tuple(p.shape), str(p.device)) for p in params)
+    return tuple(None if p is None else (p.data_ptr(), p._version, p.shape, p.device) for p in params)
 
 
 def invalidate(module) -> None:

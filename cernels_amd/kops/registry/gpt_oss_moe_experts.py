@@ -8,8 +8,6 @@ expert weights made on first use and cached on the module. Layout: ``gate_up_pro
 gate/up columns, ``down_proj[e]`` is [F, H].
 """
 
-import torch
-
 from cernels_amd import ops
 from cernels_amd.kops.registry._local import load
 from cernels_amd.kops.registry._packed import packed_experts
@@ -26,9 +24,7 @@ def kernel(x, mlp):
         raise RuntimeError("mlp module not available (meta device)")
     bsz, seqlen, hidden = x.shape
     xf = x.reshape(-1, hidden).contiguous()
-    with torch.no_grad():
-        load("gpt_oss_moe_experts")  # fail loudly if the native library is missing
-        r = mlp.router  # GptOssTopKRouter semantics (modeling_gpt_oss.py:126-130), fused
-        indices, scores = ops.moe_router(xf, r.weight, r.bias, int(r.top_k), ops.ROUTER_TOPK_SOFTMAX)
-        out = ops.moe_experts_packed(xf, _weights(mlp.experts), indices, scores, int(r.top_k))
+    load("gpt_oss_moe_experts")  # fail loudly if the native library is missing
+    r = mlp.router  # GptOssTopKRouter semantics (modeling_gpt_oss.py:126-130), fused
+    out = ops.moe_block(xf, r.weight, r.bias, int(r.top_k), ops.ROUTER_TOPK_SOFTMAX, _weights(mlp.experts))
     return out.reshape(bsz, seqlen, hidden)

@@ -10,8 +10,6 @@ reference loader's name table (gelu -> 0, silu/swish -> 1, relu -> 2; anything u
 megablocks' default ``partial(F.gelu, approximate="tanh")``, -> gelu).
 """
 
-import torch
-
 from cernels_amd import ops
 from cernels_amd.kops.registry._local import load
 from cernels_amd.kops.registry._packed import packed_megablocks
@@ -34,9 +32,6 @@ def kernel(x, moe):
     if norm not in (None, 0, 1, 1.0):
         raise RuntimeError(f"moe_normalize_expert_weights={norm} is not supported (only none or the 1-norm)")
     xf = x.reshape(-1, x.shape[-1]).contiguous()
-    with torch.no_grad():
-        load("megablocks_moe")  # fail loudly if the native library is missing
-        indices, weights = ops.moe_router(xf, moe.router.layer.weight, None, topk, ops.ROUTER_SOFTMAX_TOPK,
-                                          renorm=bool(norm))
-        packed = packed_megablocks(moe.experts.mlp, ops.MEGABLOCKS_ACTS[act_id_of(args)])
-        return ops.moe_experts_packed(xf, packed, indices, weights, topk)
+    load("megablocks_moe")  # fail loudly if the native library is missing
+    packed = packed_megablocks(moe.experts.mlp, ops.MEGABLOCKS_ACTS[act_id_of(args)])
+    return ops.moe_block(xf, moe.router.layer.weight, None, topk, ops.ROUTER_SOFTMAX_TOPK, packed, renorm=bool(norm))

@@ -14,8 +14,6 @@ Weights are packed on first use and cached on the block. Layout: ``gate_up_proj[
 ``down_proj[e]`` is [H, F].
 """
 
-import torch
-
 from cernels_amd import ops
 from cernels_amd.kops.registry._local import load
 from cernels_amd.kops.registry._packed import packed_block
@@ -26,11 +24,9 @@ def kernel(x, block):
         raise RuntimeError("block module not available (meta device)")
     bsz, seqlen, hidden = x.shape
     xf = x.reshape(-1, hidden).contiguous()
-    with torch.no_grad():
-        load("qwen3_next_moe_experts")  # fail loudly if the native library is missing
-        gate = block.gate  # Qwen3NextTopKRouter semantics (modeling_qwen3_next.py:766-775), fused
-        packed, router_w, S = packed_block(block)
-        indices, scores = ops.moe_router(xf, router_w, None, int(gate.top_k), ops.ROUTER_SOFTMAX_TOPK,
-                                         renorm=bool(getattr(gate, "norm_topk_prob", True)), shared_slots=S)
-        out = ops.moe_experts_packed(xf, packed, indices, scores, int(gate.top_k) + S)
+    load("qwen3_next_moe_experts")  # fail loudly if the native library is missing
+    gate = block.gate  # Qwen3NextTopKRouter semantics (modeling_qwen3_next.py:766-775), fused
+    packed, router_w, S = packed_block(block)
+    out = ops.moe_block(xf, router_w, None, int(gate.top_k), ops.ROUTER_SOFTMAX_TOPK, packed,
+                        renorm=bool(getattr(gate, "norm_topk_prob", True)), shared_slots=S)
     return out.reshape(bsz, seqlen, hidden)

@@ -33,9 +33,61 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+# The native entries read a router's own types; anything else is converted before the call.
+_INDEX_TYPES = {torch.int32: _native.INDEX_I32, torch.int64: _native.INDEX_I64}
+_WEIGHT_TYPES = {torch.float32: _native.WEIGHT_F32, torch.bfloat16: _native.WEIGHT_BF16}
+_BF16 = torch.bfloat16
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: _stream(torch.device("cuda", i)))
+
+
+def _launch(what: str, device_index: int, fn, *args) -> None:
+    """One native call on the current stream of the tensors' device, which is made current where it is not."""
+    if torch.cuda.current_device() == device_index:
+        st = fn(*args, _raw_stream(device_index))
+    else:
+        with torch.cuda.device(device_index):
+            st = fn(*args, _raw_stream(device_index))
+    check(st, what)
+
+
+def routing(top_k_index: torch.Tensor, top_k_weights: torch.Tensor):
+    """A router's ids and weights as the native entries take them: ids int64 or int32 and weights bf16 or fp32 as they are,
+    other types cast to int32 and fp32."""
+    idx, w = top_k_index, top_k_weights
+    if idx.dtype not in _INDEX_TYPES or w.dtype not in _WEIGHT_TYPES or not (idx.is_contiguous() and w.is_contiguous()):
+        with torch.no_grad():
+            idx = (idx if idx.dtype in _INDEX_TYPES else idx.to(torch.int32)).contiguous()
+            w = (w if w.dtype in _WEIGHT_TYPES else w.float()).contiguous()
+    return idx, w
+
+
 def _require(cond: bool, msg: str) -> None:
     if not cond:
         raise RuntimeError(msg)
+
+
+def _usable(t, dtype, device_index: int, shape) -> bool:
+    return t.dtype is dtype and t.get_device() == device_index and t.shape == shape and t.is_contiguous()
+
+
+def _dims(x, gate_up_proj, down_proj, indices, weights, topk, layout, gate_up_bias, down_bias):
+    """(T, H, F, E) of inputs that hold to the contract, else None: the caller then runs _check_inputs, which says what is
+    wrong. indices and weights may have any type that the native entries read."""
+    try:
+        T, H = x.shape
+        E, n1, n2 = gate_up_proj.shape
+        F = (n1 if layout == LAYOUT_CONCAT else n2) // 2
+        dev = x.get_device()
+        ok = (dev >= 0 and x.dtype is _BF16 and x.is_contiguous()
+              and _usable(gate_up_proj, _BF16, dev, (E, 2 * F, H) if layout == LAYOUT_CONCAT else (E, H, 2 * F))
+              and _usable(down_proj, _BF16, dev, (E, H, F) if layout == LAYOUT_CONCAT else (E, F, H))
+              and indices.dtype in _INDEX_TYPES and _usable(indices, indices.dtype, dev, (T, topk))
+              and weights.dtype in _WEIGHT_TYPES and _usable(weights, weights.dtype, dev, (T, topk))
+              and (gate_up_bias is None or _usable(gate_up_bias, torch.float32, dev, (E, 2 * F)))
+              and (down_bias is None or _usable(down_bias, torch.float32, dev, (E, H))))
+    except (AttributeError, TypeError, ValueError):
+        return None
+    return (T, H, F, E) if ok else None
 
 
 def _check_inputs(x, gate_up_proj, down_proj, indices, weights, topk, layout, gate_up_bias=None, down_bias=None):
@@ -84,8 +136,14 @@ def moe_experts(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Routed experts forward through the native library (prefill grouped GEMM or decode GEMV)."""
-    T, H, F, E = _check_inputs(x, gate_up_proj, down_proj, indices, weights, topk, layout, gate_up_bias, down_bias)
     K = int(topk)
+    dims = None
+    if decode and out is None and isinstance(indices, torch.Tensor) and indices.dtype is torch.int32 \
+            and isinstance(weights, torch.Tensor) and weights.dtype is torch.float32:
+        dims = _dims(x, gate_up_proj, down_proj, indices, weights, K, layout, gate_up_bias, down_bias)
+    if dims is not None:
+        return _decode(dims, x, gate_up_proj, down_proj, indices, weights, K, layout, act, gate_up_bias, down_bias)
+    T, H, F, E = _check_inputs(x, gate_up_proj, down_proj, indices, weights, topk, layout, gate_up_bias, down_bias)
     L = _native.lib()
     if out is None:
         out = torch.empty((T, H), dtype=torch.bfloat16, device=x.device)
@@ -111,6 +169,32 @@ def moe_experts(
         )
         check(st, name)
     return out
+
+
+def _decode(dims, x, gate_up_proj, down_proj, indices, weights, K, layout, act, gate_up_bias=None, down_bias=None):
+    T, H, F, E = dims
+    L = _native.lib()
+    out = torch.empty((T, H), dtype=_BF16, device=x.device)
+    if T == 0:
+        return out
+    nbytes = L.cernels_moe_experts_decode_workspace_bytes(T, H, F, E, K)
+    _require(nbytes > 0, f"cernels_moe_experts_decode: invalid dimensions T={T} H={H} F={F} E={E} K={K}")
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _launch("cernels_moe_experts_decode", x.get_device(), L.cernels_moe_experts_decode_typed, x.data_ptr(),
+            gate_up_proj.data_ptr(), _ptr(gate_up_bias), down_proj.data_ptr(), _ptr(down_bias), indices.data_ptr(),
+            _INDEX_TYPES[indices.dtype], weights.data_ptr(), _WEIGHT_TYPES[weights.dtype], T, H, F, E, K, layout, act,
+            out.data_ptr(), ws.data_ptr(), nbytes)
+    return out
+
+
+def experts_decode(x, gate_up_proj, down_proj, top_k_index, top_k_weights):
+    """The decode entry on a router's ids and weights in their own types (``routing``); concat layout, SiLU."""
+    idx, w = routing(top_k_index, top_k_weights)
+    K = int(idx.size(1))
+    dims = _dims(x, gate_up_proj, down_proj, idx, w, K, LAYOUT_CONCAT, None, None)
+    if dims is None:  # says what is wrong
+        return moe_experts(x, gate_up_proj, down_proj, idx.to(torch.int32), w.float(), K, decode=True)
+    return _decode(dims, x, gate_up_proj, down_proj, idx, w, K, LAYOUT_CONCAT, ACT_SILU)
 
 
 class PackedExperts:
@@ -200,9 +284,90 @@ def pack_experts(gate_up_proj, down_proj, *, layout=LAYOUT_CONCAT, act=ACT_SILU,
     return PackedExperts(gu, dn, H, F, E, act, layout, f32(gate_up_bias), f32(down_bias))
 
 
+def _packed_ok(x, packed, dev: int) -> bool:
+    """Whether ``packed`` holds the buffers of its own sizes on x's device: the kernels read packed_weight_bytes of each."""
+    try:
+        H, F, E = packed.H, packed.F, packed.E
+        gu_which = _native.GATE_UP if packed.act in (ACT_SILU, ACT_GPTOSS) else _native.UP
+        size = _native.lib().cernels_moe_packed_weight_bytes
+        n1, n2 = size(H, F, E, gu_which), size(H, F, E, _native.DOWN)
+        return (dev >= 0 and x.dtype is _BF16 and x.is_contiguous() and x.dim() == 2 and x.shape[1] == H and n1 > 0
+                and _usable(packed.gate_up, torch.uint8, dev, (n1,)) and _usable(packed.down, torch.uint8, dev, (n2,))
+                and (packed.gate_up_bias is None or _usable(packed.gate_up_bias, torch.float32, dev, (E, 2 * F)))
+                and (packed.down_bias is None or _usable(packed.down_bias, torch.float32, dev, (E, H))))
+    except (AttributeError, TypeError, ValueError):
+        return False
+
+
+def _packed(x, packed, idx, w, K, dev):
+    """The packed experts call where everything holds to the contract, else None."""
+    if not (isinstance(packed, PackedExperts) and _packed_ok(x, packed, dev) and _usable(idx, idx.dtype, dev, (x.shape[0], K))
+            and _usable(w, w.dtype, dev, (x.shape[0], K))):
+        return None
+    T, H, F, E = x.shape[0], packed.H, packed.F, packed.E
+    out = torch.empty((T, H), dtype=_BF16, device=x.device)
+    if T == 0:
+        return out
+    L = _native.lib()
+    nbytes = L.cernels_moe_experts_workspace_bytes(T, H, F, E, K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _launch("cernels_moe_experts_packed", dev, L.cernels_moe_experts_packed_typed, x.data_ptr(), packed.gate_up.data_ptr(),
+            _ptr(packed.gate_up_bias), packed.down.data_ptr(), _ptr(packed.down_bias), idx.data_ptr(),
+            _INDEX_TYPES[idx.dtype], w.data_ptr(), _WEIGHT_TYPES[w.dtype], T, H, F, E, K, packed.bias_layout, packed.act,
+            out.data_ptr(), ws.data_ptr(), nbytes)
+    return out
+
+
+def experts_packed(x, packed: PackedExperts, top_k_index, top_k_weights):
+    """moe_experts_packed on a router's ids and weights in their own types (``routing``)."""
+    idx, w = routing(top_k_index, top_k_weights)
+    K = int(idx.size(1))
+    out = _packed(x, packed, idx, w, K, x.get_device())
+    return out if out is not None else moe_experts_packed(x, packed, idx.to(torch.int32), w.float(), K)  # says what is wrong
+
+
+def moe_block(x, router_weight, router_bias, top_k: int, mode: int, packed: PackedExperts, renorm: bool = True,
+              shared_slots: int = 0):
+    """Router and packed experts of one block, as moe_router then moe_experts_packed: the routing passes from one native call
+    to the next in one scratch buffer with the experts' workspace."""
+    K, S, dev = int(top_k), int(shared_slots), x.get_device()
+    rw = router_weight
+    ok = isinstance(packed, PackedExperts) and _packed_ok(x, packed, dev) and rw.dim() == 2
+    if ok:
+        ER = rw.shape[0]
+        E = ER - (1 if S > 0 else 0)
+        ok = (E >= 1 and E + S == packed.E and _usable(rw, _BF16, dev, (ER, x.shape[1]))
+              and (router_bias is None or _usable(router_bias, _BF16, dev, (ER,))))
+    if not ok:  # says what is wrong, or takes what the two ops take apart
+        idx, w = moe_router(x, rw, router_bias, K, mode, renorm=renorm, shared_slots=S)
+        return moe_experts_packed(x, packed, idx, w, K + S)
+    T, H, F = x.shape[0], packed.H, packed.F
+    out = torch.empty((T, H), dtype=_BF16, device=x.device)
+    if T == 0:
+        return out
+    L = _native.lib()
+    nbytes = L.cernels_moe_experts_workspace_bytes(T, H, F, packed.E, K + S)
+    o_w = (4 * T * (K + S) + 255) // 256 * 256
+    o_logits = 2 * o_w
+    o_ws = o_logits + (2 * T * ER + 255) // 256 * 256
+    scratch = torch.empty(o_ws + nbytes, dtype=torch.uint8, device=x.device)
+    base, xp = scratch.data_ptr(), x.data_ptr()
+    _launch("cernels_moe_router", dev, L.cernels_moe_router, xp, rw.data_ptr(), _ptr(router_bias), T, H, E, K, int(mode),
+            int(bool(renorm)), S, base, base + o_w, base + o_logits)
+    _launch("cernels_moe_experts_packed", dev, L.cernels_moe_experts_packed, xp, packed.gate_up.data_ptr(),
+            _ptr(packed.gate_up_bias), packed.down.data_ptr(), _ptr(packed.down_bias), base, base + o_w, T, H, F, packed.E,
+            K + S, packed.bias_layout, packed.act, out.data_ptr(), base + o_ws, nbytes)
+    return out
+
+
 def moe_experts_packed(x: torch.Tensor, packed: PackedExperts, indices: torch.Tensor, weights: torch.Tensor,
                        topk: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """Routed experts prefill on packed weights (same result contract as moe_experts)."""
+    if out is None and all(isinstance(t, torch.Tensor) for t in (x, indices, weights)) \
+            and indices.dtype is torch.int32 and weights.dtype is torch.float32:
+        out = _packed(x, packed, indices, weights, int(topk), x.get_device())
+        if out is not None:
+            return out
     _require(isinstance(packed, PackedExperts), "packed must come from pack_experts")
     _require(isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
              and x.dim() == 2, "x must be a contiguous bf16 CUDA tensor [T, H]")

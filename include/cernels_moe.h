@@ -136,6 +136,16 @@ int cernels_moe_experts_packed_staged(const void* x, const void* gate_up_packed,
                                       int32_t bias_layout, int32_t act, void* out, void* workspace,
                                       size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events);
 
+/* The same with the routing in the types a transformers router returns: indices int32 or int64 (the id is the low 32
+ * bits, as a cast to int32 takes it; 8-byte aligned), weights fp32 or bf16 (2-byte aligned). Same workspace. */
+enum cernels_moe_index_type { CERNELS_MOE_INDEX_I32 = 0, CERNELS_MOE_INDEX_I64 = 1 };
+enum cernels_moe_weight_type { CERNELS_MOE_WEIGHT_F32 = 0, CERNELS_MOE_WEIGHT_BF16 = 1 };
+int cernels_moe_experts_packed_typed(const void* x, const void* gate_up_packed, const float* gate_up_bias,
+                                     const void* down_packed, const float* down_bias, const void* indices,
+                                     int32_t index_type, const void* weights, int32_t weight_type, int32_t T, int32_t H,
+                                     int32_t F, int32_t E, int32_t K, int32_t bias_layout, int32_t act, void* out,
+                                     void* workspace, size_t workspace_bytes, hipStream_t stream);
+
 /* ---- decode: fused gather-GEMV over the distinct selected experts -------------------------------
  * Two launches, no atomics on the output, no host sync. Layout CONCAT only.
  * Limits: T <= cernels_moe_decode_max_tokens(), T*K <= cernels_moe_decode_max_pairs(),
@@ -148,6 +158,14 @@ int cernels_moe_experts_decode(const void* x, const void* gate_up_proj, const fl
                                const float* weights, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
                                int32_t layout, int32_t act, void* out, void* workspace,
                                size_t workspace_bytes, hipStream_t stream);
+
+/* The same with the routing in a router's types (as cernels_moe_experts_packed_typed); the workspace is the one
+ * cernels_moe_experts_decode_workspace_bytes states. */
+int cernels_moe_experts_decode_typed(const void* x, const void* gate_up_proj, const float* gate_up_bias,
+                                     const void* down_proj, const float* down_bias, const void* indices,
+                                     int32_t index_type, const void* weights, int32_t weight_type, int32_t T, int32_t H,
+                                     int32_t F, int32_t E, int32_t K, int32_t layout, int32_t act, void* out,
+                                     void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 /* Decode with 3 stage events (before gate_up, after gate_up, after down) when not NULL. */
 int cernels_moe_experts_decode_staged(const void* x, const void* gate_up_proj, const float* gate_up_bias,
