@@ -1011,6 +1011,37 @@ static int pick_fw(long long P, int E, int NF, int Kd, int cus) {
     return best_w;
 }
 
+// M-tiles of kPkBM rows that an expert of r rows on average has on average: rows per expert spread as sqrt(r) under
+// routing without skew, so next to a multiple of kPkBM part of the experts need one tile more.
+static double expected_tiles(double r) {
+    double t = 1;
+    for (int j = 1; j * kPkBM < r + 4 * std::sqrt(r); ++j) t += 0.5 * std::erfc((j * kPkBM + 0.5 - r) / std::sqrt(2 * r));
+    return t;
+}
+
+// Whether a call takes the items of moe_mid_kernel (moe_stream.hip) in place of the persistent ones here. Two lines:
+// - Up to 90 rows per expert on average, with items for the two workgroups a CU holds in both GEMMs: one loads while the other
+//   multiplies or stores, and an expert that skewed routing makes popular is split into more, shorter items. Both GEMMs,
+//   persistent -> items (us): 128 experts of H 2048 F 768, 12.5 / 31 / 87 rows 225 -> 212, 239 -> 230, 271 -> 262; 513 experts
+//   of F 512, 43 rows 663 -> 662, 88 rows 763 -> 723 and with Zipf 1.2 skew 540 -> 473. At 112 rows (289 -> 308) and with
+//   fewer items (8 experts of F 5632, 25 rows: 95 -> 107) they lose.
+// - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM's
+//   estimate is 1.2 for items of up to 4 fragments (half of a workgroup's waves idle), else 0.95 ceil(R) / R for R rounds, and
+//   1 for at most one round (nothing to split); the mean, weighted by work, has to pass 1.08. Over 150 shapes of 8 to 513
+//   experts the mid items measured 1.00 to 1.30 times as fast wherever it does (8 experts of F 5632, 1024 rows, non-gated: 533
+//   -> 421; 64 of H 1280 F 896, 384 rows: 259 -> 230; 21 of H 1920 F 1024, 325 rows: 145 -> 108), and 0.78 to 1.12 times
+//   where it does not (32 of H = F = 2880, 188 rows: 397 -> 435, 1024 rows: 1502 -> 1605).
+static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, int fw1, int fw2, int cus) {
+    const double r = (double)P / E;
+    if (r <= 90) return (long long)E * ceil_div(std::min(nf1, nf2), kPkWaves) >= 2LL * cus;
+    auto estimate = [&](int nf, int fw) {
+        const double R = E * expected_tiles(r) * ceil_div(nf, fw) / cus;
+        return R <= 1 ? 1.0 : fw <= 4 ? 1.2 : 0.95 * std::ceil(R - 0.02) / R;
+    };
+    const double w1 = (double)nf1 * H, w2 = (double)nf2 * F;
+    return w1 * estimate(nf1, fw1) + w2 * estimate(nf2, fw2) > 1.08 * (w1 + w2);
+}
+
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
                             const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
                             hipStream_t s, int types = 0);
@@ -1021,13 +1052,14 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
                       const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
                       uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev);
 int stream_tile_m();
+int mid_tile_m();
 hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
                                int bias_interleaved, int act, const int32_t* offsets, const int32_t* tile_offsets,
                                const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles,
-                               uint16_t* glu, int8_t* gexp, int8_t* rsig, int32_t* sync, hipStream_t s);
+                               bool mid, uint16_t* glu, int8_t* gexp, int8_t* rsig, int32_t* sync, hipStream_t s);
 hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float* route_w, int T, int H, int F, int E, int K,
                                const int32_t* offsets, const int32_t* tile_offsets, const int32_t* meta,
-                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, unsigned char* Y,
+                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, bool mid, unsigned char* Y,
                                hipStream_t s);
 
 // route -> packed gate_up GEMM -> packed down GEMM -> combine, all on stream s; few rows per expert take the streaming
@@ -1046,8 +1078,13 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     // what the kernels after the route read: the caller's arrays, or the int32 / fp32 ones that the route leaves
     const int32_t* idx = types ? idx32 : idx_in;
     const float* route_w = types ? w32 : static_cast<const float*>(w_in);
-    if (tiles_supported(T, K, E)) {  // moe_stream.hip
-        const int bm = stream_tile_m();
+    const int nf1 = act_is_gated(act) ? F / 16 : F / 32, nf2 = H / 32;
+    const int fw1 = pick_fw((long long)T * K, E, nf1, H, pk_cu_count());
+    const int fw2 = pick_fw((long long)T * K, E, nf2, F, pk_cu_count());
+    const bool tiles_form = tiles_supported(T, K, E);
+    const bool mid = !tiles_form && mid_supported((long long)T * K, E, nf1, nf2, H, F, fw1, fw2, pk_cu_count());
+    if (tiles_form || mid) {  // moe_stream.hip
+        const int bm = mid ? mid_tile_m() : stream_tile_m();
         const long long P = (long long)T * K;
         const int tiles = (int)((P + bm - 1) / bm + std::min<long long>(P, E));
         mark(0);
@@ -1056,7 +1093,7 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
         if (st != hipSuccess) return st;
         mark(1);
         st = launch_stream_gemm1(x, w1p, b1, T, H, F, E, K, bias_interleaved, act, offsets, tile_offsets, meta, sorted_pairs,
-                                 tile_expert, tiles, glu, gexp, rsig, meta + 24, s);
+                                 tile_expert, tiles, mid, glu, gexp, rsig, meta + 24, s);
         if (st != hipSuccess) return st;
         hipLaunchKernelGGL(moe_glu_fixup_kernel, dim3(32), dim3(256), 0, s, glu, gexp, rsig, psig, sorted_pairs, meta + 24,
                            meta, T * K, F);
@@ -1064,7 +1101,7 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
         if (st != hipSuccess) return st;
         mark(2);
         st = launch_stream_gemm2(glu, w2p, route_w, T, H, F, E, K, offsets, tile_offsets, meta, sorted_pairs, tile_expert,
-                                 tiles, reinterpret_cast<unsigned char*>(Y), s);
+                                 tiles, mid, reinterpret_cast<unsigned char*>(Y), s);
         if (st != hipSuccess) return st;
         mark(3);
         st = launch_combine_h(reinterpret_cast<const unsigned char*>(Y), idx, static_cast<uint16_t*>(out), T, K, E, H,
@@ -1076,9 +1113,6 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     // the XCDs (meta[32..40] gate_up, meta[41..49] down). Where even the most M-tiles the route can
     // make (ceil(P / 256) + min(P, E)) would give each workgroup fewer than 8 rounds of items, the
     // split is the equal one for both GEMMs (moe_split.h) and the GEMMs compute it themselves.
-    const int nf1 = act_is_gated(act) ? F / 16 : F / 32, nf2 = H / 32;
-    const int fw1 = pick_fw((long long)T * K, E, nf1, H, pk_cu_count());
-    const int fw2 = pick_fw((long long)T * K, E, nf2, F, pk_cu_count());
     const int nt1 = ceil_div(nf1, fw1), nt2 = ceil_div(nf2, fw2);
     const int slots1 = pk_grid(max_tiles, nt1) / 8, slots2 = pk_grid(max_tiles, nt2) / 8;
     const long long P = (long long)T * K, mt_max = (P + kPkBM - 1) / kPkBM + std::min<long long>(P, E);

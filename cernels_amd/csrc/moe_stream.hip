@@ -131,9 +131,70 @@ __device__ __forceinline__ void sum_parts(const float (*part)[16][kWave], int la
     }
 }
 
+// One 32-row block's glu of one weight fragment: element r of v is row lane & 31 (valid: an existing one, glu row gr),
+// fragment column 8(r/4) + 4 half + r%4; bias: the fragment's 16 gate, then 16 up values (HAS_BIAS). Stores the fp16
+// segment and its power of two; true on lanes whose segment is scaled.
+template <int MODE, int ACT, bool HAS_BIAS, typename V>
+__device__ __forceinline__ bool store_glu(const StreamParams& prm, const V& v, bool valid, long long gr, int fc, int half,
+                                          const float* bias) {
+    constexpr int NV = MODE == kModePkGateUp ? 8 : 16;  // glu columns per lane
+    float g[NV];
+    float m = 0.f;  // the segment's largest |glu| (a nan is passed over)
+    if constexpr (MODE == kModePkGateUp) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            float gv = v[r], uv = v[8 + r];
+            if constexpr (HAS_BIAS) {
+                const int col = 8 * (r >> 2) + 4 * half + (r & 3);
+                gv += bias[col];
+                uv += bias[16 + col];
+            }
+            g[r] = swiglu<ACT>(gv, uv);
+            m = fmaxf(m, fabsf(g[r]));
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            g[r] = act_plain<ACT>(v[r]);
+            m = fmaxf(m, fabsf(g[r]));
+        }
+    }
+    m = max_halves(m);  // both lanes of the row
+    const int sg = glu_needs_scale(m) ? glu_scale_exp(m) : 0;  // 0 also for an all-zero segment
+    const bool scaled = valid && sg != 0;
+    if (__ballot(scaled) != 0ull) {  // rare
+#pragma unroll
+        for (int r = 0; r < NV; ++r) g[r] = __builtin_amdgcn_ldexpf(g[r], -sg);
+    }
+    if (valid) {  // lanes l and l ^ 32 hold the same row, so both run this or neither
+        uint32_t h[NV / 2];
+#pragma unroll
+        for (int r = 0; r < NV / 2; ++r) h[r] = pack_f16x2(g[2 * r], g[2 * r + 1]);
+        const int8_t se = (int8_t)(m == 0.f ? kGluAnyScale : sg);
+        if constexpr (MODE == kModePkGateUp) {
+            swap_halves(h[0], h[2]);  // lane l: columns 0-7, lane l + 32: columns 8-15
+            swap_halves(h[1], h[3]);
+            *reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 16 * fc + 8 * half) = u32x4{h[0], h[1], h[2], h[3]};
+            if (half == 0) prm.gexp[(long long)fc * prm.p_cap + gr] = se;
+        } else {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {  // lane l: columns 0-15, lane l + 32: columns 16-31
+                swap_halves(h[d], h[4 + d]);
+                swap_halves(h[2 + d], h[6 + d]);
+            }
+            u32x4* o = reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 32 * fc + 16 * half);
+            o[0] = u32x4{h[0], h[1], h[4], h[5]};
+            o[1] = u32x4{h[2], h[3], h[6], h[7]};
+            prm.gexp[(long long)(2 * fc + half) * prm.p_cap + gr] = se;
+        }
+    }
+    return scaled;
+}
+
 // Y row of pair p, 32 columns of fragment fc, as 24-bit floats: a lane holds columns 8i + 4 half + 0..3 of its row (both
 // half-waves active for it); after the exchange lane l stores columns 0-15 and lane l + 32 columns 16-31.
-__device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, int fc, int half, const float (&v)[16], float ws) {
+template <typename V>
+__device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, int fc, int half, const V& v, float ws) {
     f24x4 q[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = pack_f24x4(v[4 * i] * ws, v[4 * i + 1] * ws, v[4 * i + 2] * ws, v[4 * i + 3] * ws);
@@ -281,58 +342,11 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_stream_first_kernel(StreamP
         valid = lrow < rows;
         gr = row_begin + lrow;
     }
-    constexpr int NV = MODE == kModePkGateUp ? 8 : 16;  // glu columns per lane
-    float g[NV];
-    float m = 0.f;  // the segment's largest |glu| (a nan is passed over)
-    if constexpr (MODE == kModePkGateUp) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            float gv = v[r], uv = v[8 + r];
-            if constexpr (HAS_BIAS) {
-                const int col = 8 * (r >> 2) + 4 * half + (r & 3);
-                gv += s_bias[col];
-                uv += s_bias[16 + col];
-            }
-            g[r] = swiglu<ACT>(gv, uv);
-            m = fmaxf(m, fabsf(g[r]));
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            g[r] = act_plain<ACT>(v[r]);
-            m = fmaxf(m, fabsf(g[r]));
-        }
-    }
-    m = max_halves(m);  // both lanes of the row
-    const int sg = glu_needs_scale(m) ? glu_scale_exp(m) : 0;  // 0 also for an all-zero segment
-    const bool scaled = valid && sg != 0;
-    if (valid) {  // lanes l and l ^ 32 hold the same row, so both run this or neither
-        uint32_t h[NV / 2];
-#pragma unroll
-        for (int r = 0; r < NV / 2; ++r)
-            h[r] = pack_f16x2(__builtin_amdgcn_ldexpf(g[2 * r], -sg), __builtin_amdgcn_ldexpf(g[2 * r + 1], -sg));
-        const int8_t se = (int8_t)(m == 0.f ? kGluAnyScale : sg);
-        if constexpr (MODE == kModePkGateUp) {
-            swap_halves(h[0], h[2]);  // lane l: columns 0-7, lane l + 32: columns 8-15
-            swap_halves(h[1], h[3]);
-            *reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 16 * fc + 8 * half) = u32x4{h[0], h[1], h[2], h[3]};
-            if (half == 0) prm.gexp[(long long)fc * prm.p_cap + gr] = se;
-        } else {
-#pragma unroll
-            for (int d = 0; d < 2; ++d) {  // lane l: columns 0-15, lane l + 32: columns 16-31
-                swap_halves(h[d], h[4 + d]);
-                swap_halves(h[2 + d], h[6 + d]);
-            }
-            u32x4* o = reinterpret_cast<u32x4*>(prm.glu + gr * prm.F + 32 * fc + 16 * half);
-            o[0] = u32x4{h[0], h[1], h[4], h[5]};
-            o[1] = u32x4{h[2], h[3], h[6], h[7]};
-            prm.gexp[(long long)(2 * fc + half) * prm.p_cap + gr] = se;
-        }
-        if constexpr (!FEW) {
-            if (scaled) {
-                if (half == 0) prm.rsig[gr] = 1;
-                prm.sync[1] = 1;
-            }
+    const bool scaled = store_glu<MODE, ACT, HAS_BIAS>(prm, v, valid, gr, fc, half, s_bias);
+    if constexpr (!FEW) {
+        if (scaled) {
+            if (half == 0) prm.rsig[gr] = 1;
+            prm.sync[1] = 1;
         }
     }
     if constexpr (FEW) {
@@ -589,6 +603,207 @@ __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams p
     }
 }
 
+// ---- mid: the packed GEMMs as one workgroup per item, two workgroups per CU ------------------------------------------------
+// The persistent GEMMs of moe_gemm_packed.hip run one 8-wave workgroup per CU on items of up to 256 rows x 8 fragments. That
+// is the best use of the matrix units while every CU has full items, but a CU multiplies nothing while its one workgroup
+// stores an item and fills the pipe of the next, a last round that few items share costs as much as a full one, and items of
+// fewer than 8 fragments leave waves idle. Here an item is a workgroup of its own, 128 rows x 8 fragments, and a CU holds two
+// (64 KB LDS and 128 VGPRs for 8 waves each): the stores of one run under the MFMAs of the other. Which calls take it:
+// mid_supported() in moe_gemm_packed.hip. Activations go through LDS (copied there by buffer_load .. lds, double buffered),
+// weights straight to registers two 64-column groups ahead. First + second GEMM, persistent -> here (us): 8 non-gated experts
+// of H 2048 F 5632, 1024 rows each, 251 + 282 -> 196 + 225 (1.80 PFLOP/s); 513 experts of H 2048 F 512, 88 rows with Zipf 1.2
+// skew, 304 + 236 -> 251 + 222; 128 of F 768, 21 rows, 146 + 85 -> 140 + 80 (5.9 TB/s of weights). Tried and slower over 60 to
+// 150 shapes: items of 192 rows x 4 fragments, three per CU (-2% on average, up to 10% where rows cross 192), 256 x 4 (spills),
+// 128 x 8 with four waves of two fragments (0-2%, 3% faster under skew); no s_setprio around the MFMAs 0.6%; no order of MFMAs
+// and LDS reads 1%; five LDS reads ahead in place of three +0.3%, within the spread.
+constexpr int kMidMB = 4, kMidBM = 32 * kMidMB;  // rows of an item
+constexpr int kMidWaves = 8, kMidThreads = kMidWaves * kWave;
+constexpr int kMidGroups = 2;  // 64-column groups of an activation stage (32 KB)
+
+// The k-loop of one wave: one weight fragment (rw) times NMB row blocks. Group g (64 columns) of the reduction sits in
+// subtile g % kMidGroups of LDS buffer (g / kMidGroups) & 1; a stage is kMidGroups groups. Weight groups are loaded two groups ahead into slot
+// g & 1, and a stage's activations while the stage before it is multiplied; past the end both load the last group again.
+// buf(i): LDS buffer i, as an array of its own (a wait that the compiler adds before a read then covers the copies into that
+// array only).
+template <typename OpT, int NMB, typename Buf, typename CopyA>
+__device__ __forceinline__ void mid_loop(__amdgpu_buffer_rsrc_t rw, uint32_t wo, int bs, __amdgpu_buffer_rsrc_t ra, int nG,
+                                         int lane, Buf&& buf, CopyA&& copy_a, f32x16 (&acc)[kMidMB]) {
+    constexpr int GS = kMidGroups;
+    u32x4 w[2][4];
+    auto load_w = [&](int d, int g) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            w[d][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (4 * g + q) * bs, 0));
+    };
+    auto mul = [&](int d, const unsigned char* sub) {
+        constexpr int NK = 4 * NMB, R = NMB < 3 ? 2 * NMB : 3;
+        auto rd = [&](int k) {
+            return *reinterpret_cast<const OpT*>(sub + lds_off((k % NMB) * 32 + (lane & 31), 2 * (k / NMB) + (lane >> 5)));
+        };
+        OpT af[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) af[k] = rd(k);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+            const OpT wq = __builtin_bit_cast(OpT, w[d][k / NMB]);
+            f32x16& c = acc[k % NMB];
+            if constexpr (std::is_same_v<OpT, f16x8>) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq, af[k % R], c, 0, 0, 0);
+            else c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq, af[k % R], c, 0, 0, 0);
+            if (k + R < NK) af[k % R] = rd(k + R);
+        }
+        // each activation fragment's MFMA, then the LDS read that refills its registers, in that order
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (k + R < NK) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
+    };
+    load_w(0, 0);
+    load_w(1, min(1, nG - 1));
+    auto stage = [&](int g0, auto bc) {
+        constexpr int B = decltype(bc)::value;
+        // A stage issues its copies, then 4 GS weight loads, in this order (the clobbers keep it, and no load is ever dead):
+        // with at most 4 GS operations in flight this wave's copies of the stage before have landed. After the barrier
+        // every wave's have, and every wave's reads of the other buffer are done.
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070 | 4 * GS);  // vmcnt(4 GS), lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        copy_a(ra, g0 + GS, std::integral_constant<int, 1 - B>{});
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int p = 0; p < GS; ++p) {
+            const int g = g0 + p, d = p & 1;
+            if (g < nG) mul(d, buf(bc) + p * kMidBM * 128);
+            asm volatile("" ::: "memory");
+            load_w(d, min(g + 2, nG - 1));
+        }
+    };
+    // whole rounds of two stages: groups past the end are skipped (an early exit after the first stage, or a peeled tail,
+    // made the compiler move weight registers whose loads were in flight)
+    for (int g0 = 0; g0 < nG; g0 += 2 * GS) {
+        stage(g0, std::integral_constant<int, 0>{});
+        stage(g0 + GS, std::integral_constant<int, 1>{});
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) asm volatile("" ::"v"(w[d][q]));  // the loads past the end have a use
+}
+
+template <int MODE, int ACT, bool HAS_BIAS>
+__global__ __launch_bounds__(kMidThreads, 4) void moe_mid_kernel(StreamParams prm, int n_tiles) {
+    constexpr int GS = kMidGroups, FW = kMidWaves;
+    constexpr bool kDown = MODE == kModePkDown;
+    using OpT = std::conditional_t<kDown, f16x8, bf16x8>;
+    __shared__ __attribute__((aligned(16))) unsigned char sA0[GS * kMidBM * 128];
+    __shared__ __attribute__((aligned(16))) unsigned char sA1[GS * kMidBM * 128];
+    __shared__ float s_bias[FW][32];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lrow = lane & 31, half = lane >> 5;
+    // items of XCD x: one contiguous range of the list (M-tiles of an N-tile are neighbours)
+    const int total = prm.meta[0] * n_tiles, per = ceil_div(total, 8);
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    if (slot >= per || xcd * per + slot >= total) return;
+    const WorkItem it = decode_item(xcd * per + slot, n_tiles, prm.tile_expert, prm.tile_offsets, prm.offsets);
+    const int Kd = kDown ? prm.F : prm.H, nG = Kd / kBK;
+    const bool active = FW * it.n_idx + wave < prm.NF;  // a wave past the last fragment multiplies the last one again, unstored
+    const int fc = min(FW * it.n_idx + wave, prm.NF - 1);
+    const int nmb = ceil_div(it.rows, 32);
+
+    // activation copies: thread t takes chunk position t & 7 of rows t >> 3 and 64 + (t >> 3) of every subtile
+    constexpr int RP = kMidThreads / 8, NR = kMidBM / RP;
+    const int r0 = tid >> 3;
+    uint32_t ao[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int row = min(r0 + RP * i, it.rows - 1);
+        const int chunk = (tid & 7) ^ swz(r0);
+        uint32_t src;
+        if constexpr (kDown) src = row;
+        else src = prm.sorted_pairs[it.row_begin + row] / prm.K;
+        ao[i] = src * (uint32_t)(Kd * 2) + 16u * chunk;
+    }
+    const void* abase = kDown ? (const void*)(prm.A + (long long)it.row_begin * Kd) : (const void*)prm.A;
+    const __amdgpu_buffer_rsrc_t ra =
+        __builtin_amdgcn_make_buffer_rsrc((void*)abase, (short)0, kDown ? it.rows * Kd * 2 : prm.a_bytes, kBufferWord3);
+    using lds_bytes = __attribute__((address_space(3))) unsigned char*;
+    auto sbuf = [&](auto bc) -> unsigned char* {
+        if constexpr (decltype(bc)::value == 0) return sA0;
+        else return sA1;
+    };
+    auto sbuf_lds = [&](auto bc) { return (lds_bytes)sbuf(bc); };
+    auto copy_a = [&](__amdgpu_buffer_rsrc_t r, int g0, auto bc) {
+#pragma unroll
+        for (int p = 0; p < GS; ++p)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const uint32_t o = ao[i];
+                const int col = min(g0 + p, nG - 1) * kBK * 2, at = (p * kMidBM + RP * i + 8 * wave) * 128;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(sbuf_lds(bc) + at), 16, o, col,
+                                                         0, 0);
+            }
+    };
+    copy_a(ra, 0, std::integral_constant<int, 0>{});
+    if constexpr (HAS_BIAS) {
+        const int gu = (lane >> 4) & 1, col = 16 * fc + (lane & 15);
+        const float* be = prm.bias + (long long)it.e * 2 * prm.F;
+        if (lane < 32) s_bias[wave][lane] = prm.bias_interleaved ? be[2 * col + gu] : be[gu * prm.F + col];
+    }
+    const int nw = min(8, prm.NF - 8 * (fc >> 3));
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(prm.B + packed_frag(it.e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * nw * 1024 + 1024, kBufferWord3);
+    f32x16 acc[kMidMB];
+#pragma unroll
+    for (int mb = 0; mb < kMidMB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
+    auto loop = [&](auto nc) {
+        constexpr int NMB = decltype(nc)::value;
+        mid_loop<OpT, NMB>(rw, lane * 16u, nw * 1024, ra, nG, lane, sbuf, copy_a, acc);
+    };
+    switch (nmb) {
+        case 1: loop(std::integral_constant<int, 1>{}); break;
+        case 2: loop(std::integral_constant<int, 2>{}); break;
+        case 3: loop(std::integral_constant<int, 3>{}); break;
+        case 4: loop(std::integral_constant<int, 4>{}); break;
+        default: break;  // none (as the default, case 4 spills 58 registers)
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the copies past the last stage land before the LDS is gone
+    if (!active) return;
+#pragma unroll
+    for (int mb = 0; mb < kMidMB; ++mb) {
+        if (mb >= nmb) break;
+        const int row = 32 * mb + lrow;
+        const bool valid = row < it.rows;
+        const long long gr = it.row_begin + row;
+        if constexpr (kDown) {
+            const long long p = prm.sorted_pairs[it.row_begin + min(row, it.rows - 1)];
+            const float rwt = static_cast<const float*>(prm.route_w)[p];
+            const float ws = __builtin_amdgcn_ldexpf(rwt, prm.wexp[(long long)it.e * prm.NF + fc]);
+            if (valid) store_y(prm.Y, p, prm.H, fc, half, acc[mb], ws);
+        } else {
+            if (store_glu<MODE, ACT, HAS_BIAS>(prm, acc[mb], valid, gr, fc, half, s_bias[wave])) {
+                if (half == 0) prm.rsig[gr] = 1;
+                prm.sync[1] = 1;
+            }
+        }
+    }
+}
+
+template <int MODE, int ACT, bool HAS_BIAS>
+static void launch_mid_t(const StreamParams& q, int max_tiles, hipStream_t s) {
+    const int nt = ceil_div(q.NF, kMidWaves);
+    hipLaunchKernelGGL((moe_mid_kernel<MODE, ACT, HAS_BIAS>), dim3(8 * ceil_div(max_tiles * nt, 8)), dim3(kMidThreads), 0, s, q, nt);
+}
+
+int mid_tile_m() { return kMidBM; }
+
 int stream_tile_m() { return kStRows; }
 
 // Whether a call (that is not of the few form) takes the tiles form.
@@ -688,11 +903,11 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
     return st;
 }
 
-// The two projections of the tiles form, between the route (M-tiles of stream_tile_m() rows) and the fixup, and between the
-// fixup and the combine. max_tiles bounds the M-tile list.
+// The two projections of the tiles form (mid: of moe_mid_kernel), between the route (M-tiles of stream_tile_m() or mid_tile_m()
+// rows) and the fixup, and between the fixup and the combine. max_tiles bounds the M-tile list.
 hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
                                int bias_interleaved, int act, const int32_t* offsets, const int32_t* tile_offsets,
-                               const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles,
+                               const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, bool mid,
                                uint16_t* glu, int8_t* gexp, int8_t* rsig, int32_t* sync, hipStream_t s) {
     StreamParams q{};
     q.A = static_cast<const uint16_t*>(x);
@@ -709,13 +924,25 @@ hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, 
     q.p_cap = T * K;
     q.a_bytes = T * H * 2;
     q.bias_interleaved = bias_interleaved;
+    if (mid) {
+        if (act == kActSilu) {
+            if (b1) launch_mid_t<kModePkGateUp, kActSilu, true>(q, max_tiles, s);
+            else launch_mid_t<kModePkGateUp, kActSilu, false>(q, max_tiles, s);
+        } else if (act == kActGptOss) {
+            if (b1) launch_mid_t<kModePkGateUp, kActGptOss, true>(q, max_tiles, s);
+            else launch_mid_t<kModePkGateUp, kActGptOss, false>(q, max_tiles, s);
+        } else if (act == kActGeluTanh) launch_mid_t<kModePkUp, kActGeluTanh, false>(q, max_tiles, s);
+        else if (act == kActSiluPlain) launch_mid_t<kModePkUp, kActSiluPlain, false>(q, max_tiles, s);
+        else launch_mid_t<kModePkUp, kActRelu, false>(q, max_tiles, s);
+        return hipGetLastError();
+    }
     launch_stream_first<false>(q, act, dim3(q.NF, max_tiles), s);
     return hipGetLastError();
 }
 
 hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float* route_w, int T, int H, int F, int E, int K,
                                const int32_t* offsets, const int32_t* tile_offsets, const int32_t* meta,
-                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, unsigned char* Y,
+                               const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, bool mid, unsigned char* Y,
                                hipStream_t s) {
     StreamParams q{};
     q.A = glu;
@@ -728,6 +955,10 @@ hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float
     q.NF = H / 32;
     q.KS = F / 16;
     q.p_cap = T * K;
+    if (mid) {
+        launch_mid_t<kModePkDown, kActSilu, false>(q, max_tiles, s);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(moe_stream_down_kernel, dim3(q.NF, max_tiles), dim3(kStThreads), 0, s, q);
     return hipGetLastError();
 }
