@@ -249,6 +249,12 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
     // GEMM2: power of two of each wave's weight fragment (entry t holds fragment t % 8: every table
     // thread stores one, which keeps the table store free of a branch of its own)
     __shared__ int s_wx[2][kPkBM];
+    // GEMM2: epilogue staging, per wave: one 32-row block of its fragment's Y, 96 bytes a row, from which consecutive lanes
+    // store consecutive bytes. Straight from the accumulator's lanes a store touches 64 lines of 16 bytes each, which kept an
+    // item's epilogue busy for 7 us (128 rows x 8 fragments, all CUs at once); through LDS 11 or 12 runs of up to 96 bytes, 4 us.
+    // The first projections' rows (32 and 64 bytes a fragment) stay as they are.
+    constexpr int kYRow = 96;
+    __shared__ __attribute__((aligned(16))) unsigned char s_out[MODE == kModePkDown ? kPkWaves : 1][32 * kYRow];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
 
@@ -811,7 +817,6 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                     const int row = mb * 32 + lrow;
                     if (row < rows) {  // lanes l and l ^ 32 hold the same row, so both run this or neither
                         const float ws = wsc * s_w[tb][row];  // exact: wsc is a power of two
-                        const long long p = s_pair[tb][row];
                         f24x4 q[4];
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
@@ -822,10 +827,17 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                             swap_halves(q[0].d[d], q[2].d[d]);
                             swap_halves(q[1].d[d], q[3].d[d]);
                         }
-                        u32x4* yrow = reinterpret_cast<u32x4*>(Yb + (p * prm.H + 32 * fc + 16 * half) * 3);
-                        yrow[0] = u32x4{q[0].d[0], q[0].d[1], q[0].d[2], q[2].d[0]};
-                        yrow[1] = u32x4{q[2].d[1], q[2].d[2], q[1].d[0], q[1].d[1]};
-                        yrow[2] = u32x4{q[1].d[2], q[3].d[0], q[3].d[1], q[3].d[2]};
+                        u32x4* o = reinterpret_cast<u32x4*>(s_out[wave] + lrow * kYRow + 48 * half);
+                        o[0] = u32x4{q[0].d[0], q[0].d[1], q[0].d[2], q[2].d[0]};
+                        o[1] = u32x4{q[2].d[1], q[2].d[2], q[1].d[0], q[1].d[1]};
+                        o[2] = u32x4{q[1].d[2], q[3].d[0], q[3].d[1], q[3].d[2]};
+                    }
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const int c = 64 * i + lid, rr = mb * 32 + c / 6;
+                        const u32x4 v = *reinterpret_cast<const u32x4*>(s_out[wave] + 16 * c);
+                        if (rr < rows)
+                            *reinterpret_cast<u32x4*>(Yb + ((long long)s_pair[tb][rr] * prm.H + 32 * fc) * 3 + 16 * (c % 6)) = v;
                     }
                 }
             }
