@@ -191,10 +191,10 @@ __device__ __forceinline__ bool store_glu(const StreamParams& prm, const V& v, b
     return scaled;
 }
 
-// Y row of pair p, 32 columns of fragment fc, as 24-bit floats: a lane holds columns 8i + 4 half + 0..3 of its row (both
-// half-waves active for it); after the exchange lane l stores columns 0-15 and lane l + 32 columns 16-31.
+// 32 columns of a Y row as 24-bit floats: a lane holds columns 8i + 4 half + 0..3 (both half-waves active for the row); after
+// the exchange lane l has columns 0-15 and lane l + 32 columns 16-31, 48 bytes each, at y.
 template <typename V>
-__device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, int fc, int half, const V& v, float ws) {
+__device__ __forceinline__ void pack_y(const V& v, float ws, u32x4* y) {
     f24x4 q[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = pack_f24x4(v[4 * i] * ws, v[4 * i + 1] * ws, v[4 * i + 2] * ws, v[4 * i + 3] * ws);
@@ -203,10 +203,15 @@ __device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, in
         swap_halves(q[0].d[d], q[2].d[d]);
         swap_halves(q[1].d[d], q[3].d[d]);
     }
-    u32x4* y = reinterpret_cast<u32x4*>(Y + (p * H + 32 * fc + 16 * half) * 3);
     y[0] = u32x4{q[0].d[0], q[0].d[1], q[0].d[2], q[2].d[0]};
     y[1] = u32x4{q[2].d[1], q[2].d[2], q[1].d[0], q[1].d[1]};
     y[2] = u32x4{q[1].d[2], q[3].d[0], q[3].d[1], q[3].d[2]};
+}
+
+// The same, straight to the Y row of pair p (fragment fc).
+template <typename V>
+__device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, int fc, int half, const V& v, float ws) {
+    pack_y(v, ws, reinterpret_cast<u32x4*>(Y + (p * H + 32 * fc + 16 * half) * 3));
 }
 
 // few: the u-th smallest distinct expert of the indices (-1: fewer than u + 1), and in tokp[t] the first pair of token t
@@ -611,13 +616,14 @@ __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams p
 // (64 KB LDS and 128 VGPRs for 8 waves each): the stores of one run under the MFMAs of the other. Which calls take it:
 // mid_supported() in moe_gemm_packed.hip. Activations go through LDS (copied there by buffer_load .. lds, double buffered),
 // weights straight to registers two 64-column groups ahead. First + second GEMM, persistent -> here (us): 8 non-gated experts
-// of H 2048 F 5632, 1024 rows each, 251 + 282 -> 196 + 225 (1.80 PFLOP/s); 513 experts of H 2048 F 512, 88 rows with Zipf 1.2
+// of H 2048 F 5632, 1024 rows each, 251 + 282 -> 190 + 215 (0.71 -> 0.93 PFLOP/s); 513 experts of H 2048 F 512, 88 rows with Zipf 1.2
 // skew, 304 + 236 -> 251 + 222; 128 of F 768, 21 rows, 146 + 85 -> 140 + 80 (5.9 TB/s of weights). Tried and slower over 60 to
 // 150 shapes: items of 192 rows x 4 fragments, three per CU (-2% on average, up to 10% where rows cross 192), 256 x 4 (spills),
 // 128 x 8 with four waves of two fragments (0-2%, 3% faster under skew); no s_setprio around the MFMAs 0.6%; no order of MFMAs
 // and LDS reads 1%; five LDS reads ahead in place of three +0.3%, within the spread.
 constexpr int kMidMB = 4, kMidBM = 32 * kMidMB;  // rows of an item
 constexpr int kMidWaves = 8, kMidThreads = kMidWaves * kWave;
+constexpr int kYRow = 96;  // bytes of a fragment's 32 columns of a Y row
 constexpr int kMidGroups = 2;  // 64-column groups of an activation stage (32 KB)
 
 // The k-loop of one wave: one weight fragment (rw) times NMB row blocks. Group g (64 columns) of the reduction sits in
@@ -774,8 +780,23 @@ __global__ __launch_bounds__(kMidThreads, 4) void moe_mid_kernel(StreamParams pr
         case 4: loop(std::integral_constant<int, 4>{}); break;
         default: break;  // none (as the default, case 4 spills 58 registers)
     }
+    // Down: rows of Y leave through LDS, 32 rows x 96 bytes of a wave's fragment at a time (in the first activation buffer), so
+    // that consecutive lanes store consecutive bytes; straight from the accumulators a store is 64 pieces of 16 bytes, which
+    // the L2 takes one by one. Down GEMM, without -> with (us): 513 experts of H 2048 F 512, 88 rows 294 -> 277; 8 of F 5632,
+    // 1024 rows 223 -> 215, 550 rows 142 -> 136; 64 of H 1280 F 896, 469 rows 122 -> 112; 128 of F 768, 62 rows 94 -> 91.
+    __shared__ int s_pair[kMidBM];
+    __shared__ float s_w[kMidBM];
+    if constexpr (kDown) {
+        if (tid < it.rows) {
+            const int p = prm.sorted_pairs[it.row_begin + tid];
+            s_pair[tid] = p;
+            s_w[tid] = static_cast<const float*>(prm.route_w)[p];
+        }
+    }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the copies past the last stage land before the LDS is gone
+    if constexpr (kDown) __syncthreads();
     if (!active) return;
+    [[maybe_unused]] const float wsc = kDown ? __builtin_amdgcn_ldexpf(1.f, prm.wexp[(long long)it.e * prm.NF + fc]) : 1.f;
 #pragma unroll
     for (int mb = 0; mb < kMidMB; ++mb) {
         if (mb >= nmb) break;
@@ -783,10 +804,16 @@ __global__ __launch_bounds__(kMidThreads, 4) void moe_mid_kernel(StreamParams pr
         const bool valid = row < it.rows;
         const long long gr = it.row_begin + row;
         if constexpr (kDown) {
-            const long long p = prm.sorted_pairs[it.row_begin + min(row, it.rows - 1)];
-            const float rwt = static_cast<const float*>(prm.route_w)[p];
-            const float ws = __builtin_amdgcn_ldexpf(rwt, prm.wexp[(long long)it.e * prm.NF + fc]);
-            if (valid) store_y(prm.Y, p, prm.H, fc, half, acc[mb], ws);
+            static_assert(kMidWaves * 32 * kYRow <= kMidGroups * kMidBM * 128);
+            unsigned char* st = sA0 + wave * 32 * kYRow;
+            if (valid) pack_y(acc[mb], s_w[row] * wsc, reinterpret_cast<u32x4*>(st + lrow * kYRow + 48 * half));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int c = 64 * i + lane, rr = 32 * mb + c / 6;
+                const u32x4 v = *reinterpret_cast<const u32x4*>(st + 16 * c);
+                if (rr < it.rows)
+                    *reinterpret_cast<u32x4*>(prm.Y + ((long long)s_pair[rr] * prm.H + 32 * fc) * 3 + 16 * (c % 6)) = v;
+            }
         } else {
             if (store_glu<MODE, ACT, HAS_BIAS>(prm, acc[mb], valid, gr, fc, half, s_bias[wave])) {
                 if (half == 0) prm.rsig[gr] = 1;
