@@ -617,7 +617,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams p
 // mid_supported() in moe_gemm_packed.hip. Activations go through LDS (copied there by buffer_load .. lds, double buffered),
 // weights straight to registers two 64-column groups ahead. First + second GEMM, persistent -> here (us): 8 non-gated experts
 // of H 2048 F 5632, 1024 rows each, 251 + 282 -> 190 + 215 (0.71 -> 0.93 PFLOP/s); 513 experts of H 2048 F 512, 88 rows with Zipf 1.2
-// skew, 304 + 236 -> 251 + 222; 128 of F 768, 21 rows, 146 + 85 -> 140 + 80 (5.9 TB/s of weights). Tried and slower over 60 to
+// skew, 304 + 236 -> 251 + 222; 128 of F 768, 21 rows, 146 + 85 -> 140 + 80 (5.5 TB/s of weights). Tried and slower over 60 to
 // 150 shapes: items of 192 rows x 4 fragments, three per CU (-2% on average, up to 10% where rows cross 192), 256 x 4 (spills),
 // 128 x 8 with four waves of two fragments (0-2%, 3% faster under skew); no s_setprio around the MFMAs 0.6%; no order of MFMAs
 // and LDS reads 1%; five LDS reads ahead in place of three +0.3%, within the spread.
