@@ -668,6 +668,7 @@ __device__ __forceinline__ void mid_loop(__amdgpu_buffer_rsrc_t rw, uint32_t wo,
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(0);
     };
+    asm volatile("" ::: "memory");  // the caller's copies of the first stage are issued before these loads (see stage)
     load_w(0, 0);
     load_w(1, min(1, nG - 1));
     auto stage = [&](int g0, auto bc) {
