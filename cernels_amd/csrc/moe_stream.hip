@@ -70,7 +70,6 @@ struct StreamParams {
     const int8_t* wexp;           // down: [E, NF] power of two of each weight fragment
     int32_t* few_e;               // few: [U_max] the u-th smallest expert chosen, -1 past the last
     int16_t* few_row;             // few: [U_max, T] glu row (pair) of (expert u, token t), bit 14 if t names u again, -1: not chosen
-    float* few_w;                 // few: [U_max, T] routing weight (summed over slots that name the expert twice)
     uint8_t* few_scaled;          // few: [U_max, NF of the first projection] some segment is scaled
     int T, K, E, H, F, NF, KS, u_max, nf1;
     int p_cap, a_bytes, bias_interleaved;
@@ -360,13 +359,7 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_stream_first_kernel(StreamP
         if (lane == 0) prm.few_scaled[u * prm.NF + fc] = sb != 0ull;
         if (fc == 0) {  // the lists that the down kernel walks
             if (lane == 0) prm.few_e[u] = e;
-            if (lane < prm.T) {
-                float wt = 0.f;
-                for (int k = 0; k < prm.K; ++k)
-                    if (pair_id(prm.idx, prm.types, lane * prm.K + k) == e) wt += pair_weight(prm.route_w, prm.types, lane * prm.K + k);
-                prm.few_row[u * prm.T + lane] = (int16_t)(valid ? my_pair | again << 14 : -1);
-                prm.few_w[u * prm.T + lane] = wt;
-            }
+            if (lane < prm.T) prm.few_row[u * prm.T + lane] = (int16_t)(valid ? my_pair | again << 14 : -1);
         }
     }
 }
@@ -470,19 +463,22 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
         }
 }
 
-// few, at most kFdMaxPairs pairs: out[t, 16 columns] = bf16( sum over the experts u of w[u, t] * (glu row . W2_e + b2_e) ), which
-// saves the combine's launch. grid H / 16: a workgroup takes one half of a 32-column weight fragment for all experts; its
-// waves split the (expert, 64-column stage) list evenly and in order, each keeping its tokens' sums in registers
-// (16x16x32 MFMA, tokens as columns), and the sums are added in wave order. kFdStages stages in flight per wave.
+// few, at most kFdMaxPairs pairs: out[t, 16 columns] = bf16( sum over the slots k of t of w_k * (glu row . W2_e + b2_e) ), in slot
+// order, which saves the combine's launch. grid H / 16: a workgroup takes one half of a 32-column weight fragment for all
+// experts. An expert's 64-column stages are cut into kFdWaves shares whose bounds depend on F alone; wave w takes share
+// (w + u) % kFdWaves of the u-th expert (shares differ by a stage), one expert after the other with kFdStages stages in flight,
+// and leaves its partial sums in LDS (16x16x32 MFMA, tokens as columns). A thread per pair and column then adds the shares in
+// order. So a row depends on its token and that token's slots alone: not on the other tokens of the call, nor on how the
+// experts are numbered.
 template <bool HAS_BIAS>
 __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams prm) {
-    const int T = prm.T, um = prm.u_max;  // both <= kFdMaxPairs
+    const int T = prm.T, um = prm.u_max, P = prm.T * prm.K;  // all <= kFdMaxPairs
     __shared__ int s_e[kFdMaxPairs];
-    __shared__ int s_x[kFdMaxPairs];                // power of two of the weight fragment
-    __shared__ float s_w[kFdMaxPairs * kFdMaxPairs];  // [um, T]
-    __shared__ int s_row[kFdMaxPairs * kFdMaxPairs];  // [um, T], -1: not chosen
-    __shared__ int s_max[kFdMaxPairs];              // where segments are scaled: the largest power of two of each glu row
-    __shared__ __attribute__((aligned(16))) float red[kFdWaves][16][16];
+    __shared__ int s_id[kFdMaxPairs];                 // pairs' experts, -1: out of range
+    __shared__ int s_row[kFdMaxPairs * kFdMaxPairs];  // [um, T] glu row, -1: not chosen
+    __shared__ int s_max[kFdMaxPairs];                // where segments are scaled: the largest power of two of each glu row
+    __shared__ __attribute__((aligned(16))) float s_part[kFdWaves][kFdMaxPairs][16];  // share, glu row, column
+    __shared__ float s_y[kFdMaxPairs][16];            // slots' weighted rows
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int fc = blockIdx.x >> 1, hf = blockIdx.x & 1;  // weight fragment, its half
@@ -494,14 +490,14 @@ __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams p
     for (int i = tid; i < nfl; i += kFdThreads) flags |= prm.few_scaled[i];
     if (tid < um * T) {
         const int r = prm.few_row[tid];
-        s_w[tid] = prm.few_w[tid];
         s_row[tid] = r < 0 ? -1 : r & 0x3fff;
     }
-    if (tid < um) {
-        s_e[tid] = my_e;
-        s_x[tid] = my_e >= 0 ? prm.wexp[(long long)my_e * prm.NF + fc] : 0;
+    if (tid < um) s_e[tid] = my_e;
+    if (tid < P) {
+        const int e = pair_id(prm.idx, prm.types, tid);
+        s_id[tid] = (unsigned)e < (unsigned)prm.E ? e : -1;
     }
-    const int U = __syncthreads_count(my_e >= 0);  // the entries are a prefix
+    const int U = __builtin_amdgcn_readfirstlane(__syncthreads_count(my_e >= 0));  // the entries are a prefix
     const bool any_scaled = __syncthreads_or(flags) != 0;
     if (any_scaled) {
         if (tid < U * T && s_row[tid] >= 0) {
@@ -514,97 +510,115 @@ __global__ __launch_bounds__(kFdThreads) void moe_few_down_kernel(StreamParams p
     }
 
     const int S = prm.F / kBK;  // stages per expert
-    const int N = U * S;
-    const int i0 = wave * N / kFdWaves, cnt = (wave + 1) * N / kFdWaves - i0;
+    auto share_of = [&](int u) { return (wave + u) % kFdWaves; };
+    auto bound = [&](int j) { return j * S / kFdWaves; };
+    int cnt = 0;  // this wave's stages
+    for (int u = 0; u < U; ++u) cnt += bound(share_of(u) + 1) - bound(share_of(u));
     const int nw = min(8, prm.NF - 8 * (fc >> 3)), bs = nw * 1024;
     const uint32_t wo = (uint32_t)((grp >> 1) * bs + (grp & 1) * 512 + (16 * hf + l16) * 16);
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)prm.A, (short)0, prm.a_bytes, kBufferWord3);
     const int t16 = min(l16, T - 1);
 
-    f32x4 tot = {0.f, 0.f, 0.f, 0.f}, acc = {0.f, 0.f, 0.f, 0.f};
+    // the epilogue's pair and column of this thread (the first 16 P threads)
+    const int q = tid >> 4, c = tid & 15;
+    const int eq = q < P ? s_id[q] : -1, e0 = max(eq, 0);
+    int first = q;  // the glu row of the pair: the token's first pair that names the expert
+    if (eq >= 0)
+        for (int k = q / prm.K * prm.K; k < first; ++k)
+            if (s_id[k] == eq) first = k;
+    const int wx = prm.wexp[(long long)e0 * prm.NF + fc];
+    const float wq = pair_weight(prm.route_w, prm.types, min(q, P - 1));
+    float bq = 0.f;
+    if constexpr (HAS_BIAS) bq = prm.bias[(long long)e0 * prm.H + 16 * blockIdx.x + c];
+
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     constexpr int D = kFdStages;
     u32x4 w[D][2], a[D][2];
-    float bsum = 0.f;  // this thread's output element's share of the down bias
 
     auto run = [&](auto sc) {
         constexpr bool SC = decltype(sc)::value;
-        int lu = cnt > 0 ? i0 / S : 0, ls = cnt > 0 ? i0 - lu * S : 0;  // stage to load next
-        int cu = lu, cs = ls;                                        // stage to multiply next
-        int left = cnt;                                              // stages not loaded yet
+        // a walk over this wave's stages: stage s of [.., end) of expert u; empty shares are passed over
+        struct Walk { int u, s, end; };
+        auto settle = [&](Walk& k) {
+            while (k.s == k.end && k.u + 1 < U) {
+                ++k.u;
+                k.s = bound(share_of(k.u));
+                k.end = bound(share_of(k.u) + 1);
+            }
+        };
+        Walk ld{0, bound(share_of(0)), bound(share_of(0) + 1)};  // stage to load next
+        settle(ld);
+        Walk mu = ld;    // stage to multiply next
+        int left = cnt;  // stages not loaded yet
         auto load = [&](int d) {
-            const int e = __builtin_amdgcn_readfirstlane(s_e[lu]);
+            const int e = __builtin_amdgcn_readfirstlane(s_e[ld.u]);
             const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
                 (void*)(prm.B + packed_frag(e, fc, 0, prm.NF, prm.KS) * kPkFrag), (short)0, (prm.KS - 1) * bs + 1024, kBufferWord3);
-            const uint32_t r = (uint32_t)max(0, s_row[lu * T + t16]);  // a token without this expert: row 0, dropped
+            const uint32_t r = (uint32_t)max(0, s_row[ld.u * T + t16]);  // a token without this expert: row 0, dropped
             const uint32_t ro = r * (uint32_t)(prm.F * 2) + 16u * grp;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-                w[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (4 * ls + 2 * i) * bs, 0));
+                w[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (4 * ld.s + 2 * i) * bs, 0));
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-                a[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, ro + 64 * i, ls * kBK * 2, 0));
-            if (--left > 0 && ++ls == S) {  // past the last stage: the last one again, dropped
-                ls = 0;
-                ++lu;
+                a[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, ro + 64 * i, ld.s * kBK * 2, 0));
+            if (--left > 0) {  // past the last stage: the last one again, dropped
+                ++ld.s;
+                settle(ld);
             }
         };
-        auto mul = [&](int d, bool last) {
+        auto mul = [&](int d) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 f16x8 aq = __builtin_bit_cast(f16x8, a[d][i]);
                 if constexpr (SC) {  // bring the segment to its row's scale
-                    const int p = max(0, s_row[cu * T + t16]);
-                    const int dd = (int)prm.gexp[(long long)(4 * cs + 2 * i + (grp >> 1)) * prm.p_cap + p] - s_max[p];
+                    const int p = max(0, s_row[mu.u * T + t16]);
+                    const int dd = (int)prm.gexp[(long long)(4 * mu.s + 2 * i + (grp >> 1)) * prm.p_cap + p] - s_max[p];
 #pragma unroll
                     for (int j = 0; j < 8; ++j) aq[j] = (_Float16)__builtin_amdgcn_ldexpf((float)aq[j], min(dd, 0));
                 }
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[d][i]), aq, acc, 0, 0, 0);
             }
-            if (++cs == S || last) {  // this expert's share is whole: into the tokens' sums
-                const int p = s_row[cu * T + t16];
-                int x = s_x[cu];
-                if constexpr (SC) x += s_max[max(p, 0)];
-                const float wt = s_w[cu * T + t16];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float y = tot[r] + wt * __builtin_amdgcn_ldexpf(acc[r], x);
-                    tot[r] = p >= 0 ? y : tot[r];  // a select: dropped rows may hold anything
-                    acc[r] = 0.f;
-                }
-                cs = 0;
-                ++cu;
+            if (++mu.s == mu.end) {  // the share is whole
+                const int p = l16 < T ? s_row[mu.u * T + l16] : -1;
+                if (p >= 0) *reinterpret_cast<f32x4*>(&s_part[share_of(mu.u)][p][4 * grp]) = acc;
+                acc = f32x4{0.f, 0.f, 0.f, 0.f};
+                settle(mu);
             }
         };
         if (cnt > 0) {
 #pragma unroll
             for (int d = 0; d < D; ++d) load(d);
         }
-        if constexpr (HAS_BIAS) {
-            const int t = tid >> 4;
-            if (t < T)
-                for (int u = 0; u < U; ++u)
-                    if (s_row[u * T + t] >= 0)
-                        bsum += s_w[u * T + t] * prm.bias[(long long)s_e[u] * prm.H + 16 * blockIdx.x + (tid & 15)];
-        }
         for (int i = 0; i < cnt; i += D) {
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                if (i + d < cnt) mul(d, i + d == cnt - 1);
+                if (i + d < cnt) mul(d);
                 load(d);
             }
         }
     };
     if (any_scaled) run(std::true_type{});
     else run(std::false_type{});
-    *reinterpret_cast<f32x4*>(&red[wave][l16][4 * grp]) = tot;
     __syncthreads();
-    const int t = tid >> 4, c = tid & 15;  // tokens x 16 columns (the first 256 threads)
-    if (t < T) {
-        float s = red[0][t][c];
+    if (eq >= 0) {
+        float v = 0.f;
 #pragma unroll
-        for (int k = 1; k < kFdWaves; ++k) s += red[k][t][c];
-        if constexpr (HAS_BIAS) s += bsum;
-        prm.out[(long long)t * prm.H + 16 * blockIdx.x + c] = f32_to_bf16_bits(s);
+        for (int k = 0; k < kFdWaves; ++k) {
+            const float part = s_part[k][first][c];
+            v += bound(k) < bound(k + 1) ? part : 0.f;  // an empty share holds nothing
+        }
+        float y = v * __builtin_amdgcn_ldexpf(wq, wx);
+        if (any_scaled) y = __builtin_amdgcn_ldexpf(y, s_max[first]);
+        if constexpr (HAS_BIAS) y += wq * bq;
+        s_y[q][c] = y;
+    }
+    __syncthreads();
+    if (q < T) {  // now a token and column
+        float s = 0.f;
+        for (int k = 0; k < prm.K; ++k)
+            if (s_id[q * prm.K + k] >= 0) s += s_y[q * prm.K + k][c];
+        prm.out[(long long)q * prm.H + 16 * blockIdx.x + c] = f32_to_bf16_bits(s);
     }
 }
 
@@ -851,7 +865,7 @@ size_t few_workspace_bytes(int T, int F, int E, int K) {
     const long long P = (long long)T * K;
     if (!few_supported(T, K, E)) return 0;
     const size_t um = (size_t)(P < E ? P : E);
-    return few_part(um * 4) + few_part(um * T * 2) + few_part(um * T * 4) + few_part(um * (F / 16));
+    return few_part(um * 4) + few_part(um * T * 2) + few_part(um * (F / 16));
 }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
@@ -890,8 +904,7 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
     q.gexp = gexp;
     q.few_e = reinterpret_cast<int32_t*>(lists);
     q.few_row = reinterpret_cast<int16_t*>(lists + few_part((size_t)um * 4));
-    q.few_w = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(q.few_row) + few_part((size_t)um * T * 2));
-    q.few_scaled = reinterpret_cast<unsigned char*>(q.few_w) + few_part((size_t)um * T * 4);
+    q.few_scaled = reinterpret_cast<unsigned char*>(q.few_row) + few_part((size_t)um * T * 2);
     q.T = T; q.K = K; q.E = E; q.H = H; q.F = F;
     q.NF = q.nf1 = act_is_gated(act) ? F / 16 : F / 32;
     q.KS = H / 16;

@@ -157,3 +157,29 @@ def test_few_rows_graph_replays(device, T):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4))
+
+
+@pytest.mark.parametrize("T,K,part", [(4, 4, 1), (5, 3, 1), (24, 4, 6), (64, 4, 40)], ids=["fused", "fused-k3", "rows", "tiles"])
+def test_few_rows_do_not_depend_on_the_other_tokens(device, T, K, part):
+    """A token's row is the same bit for bit whether the call holds the other tokens or not (both calls of one form), some of
+    which are stored scaled, and however the experts are numbered: its slots are summed in their own order, each from a
+    reduction that is cut at places that only the layer's sizes fix. F gives 13 stages, which no number of waves divides."""
+    from cernels_amd import ops
+
+    c = rand_case(T + K, T, 192, 832, 32, K, layout="interleaved", act="gptoss", bias=True, std=0.05)
+    c["idx"][0, K - 1] = c["idx"][0, 0]  # an expert named twice
+    c["x"][T - 1] = (c["x"][T - 1].float() * 3000.0).bfloat16()
+    d = to_device(c, device)
+    kw = dict(layout=ops.LAYOUT_INTERLEAVED, act=ops.ACT_GPTOSS)
+    pk = ops.pack_experts(d["W1"], d["W2"], gate_up_bias=d["b1"], down_bias=d["b2"], **kw)
+    print(f"[few rows neighbours T{T} K{K}]", flush=True)
+    whole = ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], K)
+    for t in range(0, T - part + 1, part):
+        r = slice(t, t + part)
+        some = ops.moe_experts_packed(d["x"][r].contiguous(), pk, d["idx"][r].contiguous(), d["w"][r].contiguous(), K)
+        assert torch.equal(some, whole[r]), f"tokens {t}..{t + part - 1}"
+    perm = torch.randperm(32, generator=torch.Generator().manual_seed(1)).to(device)  # expert e moves to place perm[e]
+    inv = torch.argsort(perm)
+    pk2 = ops.pack_experts(d["W1"][inv].contiguous(), d["W2"][inv].contiguous(), gate_up_bias=d["b1"][inv].contiguous(),
+                           down_bias=d["b2"][inv].contiguous(), **kw)
+    assert torch.equal(ops.moe_experts_packed(d["x"], pk2, perm[d["idx"].long()].int(), d["w"], K), whole)
