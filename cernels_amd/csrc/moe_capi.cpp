@@ -36,13 +36,10 @@ int decode_max_tokens();
 size_t packed_weight_bytes(int H, int F, int E, int which);
 hipError_t launch_pack(const uint16_t* src, uint16_t* dst, int E, int H, int F, int layout, int which, hipStream_t s);
 hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2,
-                                 const int32_t* idx, const void* route_w, int types, int32_t* idx32, float* w32, int T, int H,
-                                 int F, int E, int K, int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
-                                 int32_t* meta, int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts,
-                                 int max_tiles, uint16_t* glu, float* Y, int8_t* gexp, int8_t* rsig,
-                                 int8_t* psig, unsigned char* few_lists, hipStream_t s, hipEvent_t* ev);
-int stream_tile_m();
-size_t few_workspace_bytes(int T, int F, int E, int K);
+                                 const int32_t* idx, const void* route_w, int types, int T, int H, int F, int E, int K,
+                                 int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets, int32_t* meta,
+                                 int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts, int max_tiles, uint16_t* glu,
+                                 float* Y, int8_t* gexp, int8_t* rsig, int8_t* psig, hipStream_t s, hipEvent_t* ev);
 hipError_t launch_decode(const uint16_t* x, const uint16_t* w1, const float* b1, const uint16_t* w2, const float* b2,
                          const int32_t* idx, const void* w, int types, uint16_t* glu, int32_t* order, float* order_w,
                          uint16_t* out, int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev);
@@ -57,10 +54,13 @@ size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 struct PrefillWs {
-    size_t offsets, tile_offsets, meta, sorted_pairs, tile_expert, route_counts, glu, Y, gexp, rsig, psig, few, idx32, w32, total;
+    size_t offsets, tile_offsets, meta, sorted_pairs, tile_expert, route_counts, glu, Y, gexp, rsig, psig, total;
     int capacity;
 };
 
+// Every part grows with T, K and E (a workspace sized for a caller's largest call serves the smaller ones), so no part is
+// there for one form of the packed path alone: what its forms need beyond this lies in the half of glu that they leave free
+// (packed_spare in moe_gemm_packed.hip).
 PrefillWs prefill_ws(int T, int H, int F, int E, int K) {
     PrefillWs w{};
     const long long P = (long long)T * K;
@@ -72,18 +72,13 @@ PrefillWs prefill_ws(int T, int H, int F, int E, int K) {
     w.meta = o;         o = align_up(o + sizeof(int32_t) * 64);  // [0..1] route totals, [8..31] GEMM counters, flags,
                                                                  // [32..49] per-XCD item ranges (packed)
     w.sorted_pairs = o; o = align_up(o + sizeof(int32_t) * P);
-    const int bs = cmoe::stream_tile_m();  // the packed path's smaller M-tiles (few rows per expert)
-    const long long tiles = std::max<long long>(w.capacity, (P + bs - 1) / bs + (P < E ? P : E));
-    w.tile_expert = o;  o = align_up(o + sizeof(int32_t) * (size_t)(tiles > 0 ? tiles : 1));
+    w.tile_expert = o;  o = align_up(o + sizeof(int32_t) * (size_t)(w.capacity > 0 ? w.capacity : 1));
     w.route_counts = o; o = align_up(o + cmoe::route_workspace_bytes(T, K, E));
     w.glu = o;          o = align_up(o + sizeof(uint16_t) * 2 * P * F);  // stored layout: bf16 pairs; packed: fp16
     w.Y = o;            o = align_up(o + 3 * P * H);  // 24-bit floats (both paths)
     w.gexp = o;         o = align_up(o + (size_t)P * (F / 16));  // packed path: exponent per 16-column glu segment
     w.rsig = o;         o = align_up(o + (size_t)P);             // packed path: per glu row scale
     w.psig = o;         o = align_up(o + (size_t)P);             // packed path: the same, per pair
-    w.few = o;          o = align_up(o + cmoe::few_workspace_bytes(T, F, E, K));  // packed path, few tokens: expert lists
-    w.idx32 = o;        o = align_up(o + sizeof(int32_t) * P);  // packed path: ids and weights that came as int64 / bf16
-    w.w32 = o;          o = align_up(o + sizeof(float) * P);
     w.total = o;
     return w;
 }
@@ -271,13 +266,12 @@ static int packed_impl(const void* x, const void* gate_up_packed, const float* g
     char* base = static_cast<char*>(workspace);
     return hip_status(cmoe::launch_prefill_packed(
         x, gate_up_packed, gate_up_bias, down_packed, down_bias, static_cast<const int32_t*>(indices), weights, types,
-        reinterpret_cast<int32_t*>(base + w.idx32), reinterpret_cast<float*>(base + w.w32), T, H, F, E, K,
-        bias_layout == CERNELS_MOE_LAYOUT_INTERLEAVED, act, out, reinterpret_cast<int32_t*>(base + w.offsets),
+        T, H, F, E, K, bias_layout == CERNELS_MOE_LAYOUT_INTERLEAVED, act, out, reinterpret_cast<int32_t*>(base + w.offsets),
         reinterpret_cast<int32_t*>(base + w.tile_offsets), reinterpret_cast<int32_t*>(base + w.meta),
         reinterpret_cast<int32_t*>(base + w.sorted_pairs), reinterpret_cast<int32_t*>(base + w.tile_expert),
         reinterpret_cast<int32_t*>(base + w.route_counts), w.capacity, reinterpret_cast<uint16_t*>(base + w.glu),
         reinterpret_cast<float*>(base + w.Y), reinterpret_cast<int8_t*>(base + w.gexp), reinterpret_cast<int8_t*>(base + w.rsig),
-        reinterpret_cast<int8_t*>(base + w.psig), reinterpret_cast<unsigned char*>(base + w.few), stream, stage_events));
+        reinterpret_cast<int8_t*>(base + w.psig), stream, stage_events));
 }
 }  // namespace
 

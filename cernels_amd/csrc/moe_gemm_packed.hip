@@ -1074,22 +1074,42 @@ hipError_t launch_stream_gemm2(const uint16_t* glu, const void* w2p, const float
                                const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles, bool mid, unsigned char* Y,
                                hipStream_t s);
 
+// What the packed path's forms keep in the second half of the workspace's glu part. That part is sized for the stored layout's
+// bf16 pairs, 4 P F bytes; the packed path's fp16 takes 2 P F and leaves at least 128 bytes per pair (F >= 64). The ids, the
+// weights and the list of 32-row tiles take 8 P + 4 (P / 32 + 1 + P); the few-token lists (few_part in moe_stream.hip, P >= 1 pairs of
+// at most 32 tokens) at most P (68 + F / 16) + 45, below 2 P F.
+struct PackedSpare {
+    unsigned char* few_lists;  // few tokens: expert lists (no route, so nothing of the rest)
+    int32_t* idx32;            // ids and weights that came as int64 or bf16
+    float* w32;
+    int32_t* tile_expert;      // 32-row M-tiles
+};
+static PackedSpare packed_spare(uint16_t* glu, int T, int F, int K) {
+    const long long P = (long long)T * K;
+    PackedSpare sp;
+    sp.few_lists = reinterpret_cast<unsigned char*>(glu + P * F);
+    sp.idx32 = reinterpret_cast<int32_t*>(glu + P * F);
+    sp.w32 = reinterpret_cast<float*>(sp.idx32 + P);
+    sp.tile_expert = reinterpret_cast<int32_t*>(sp.w32 + P);
+    return sp;
+}
+
 // route -> packed gate_up GEMM -> packed down GEMM -> combine, all on stream s; few rows per expert take the streaming
 // forms of moe_stream.hip instead (its header states where the lines lie and why). Shapes were checked
 // by the caller (H % 64 == 0, F % 64 == 0, E <= 1024, T >= 1).
 hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2,
-                                 const int32_t* idx_in, const void* w_in, int types, int32_t* idx32, float* w32, int T, int H,
-                                 int F, int E, int K, int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets,
-                                 int32_t* meta, int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts,
-                                 int max_tiles, uint16_t* glu, float* Y, int8_t* gexp, int8_t* rsig,
-                                 int8_t* psig, unsigned char* few_lists, hipStream_t s, hipEvent_t* ev) {
+                                 const int32_t* idx_in, const void* w_in, int types, int T, int H, int F, int E, int K,
+                                 int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets, int32_t* meta,
+                                 int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts, int max_tiles, uint16_t* glu,
+                                 float* Y, int8_t* gexp, int8_t* rsig, int8_t* psig, hipStream_t s, hipEvent_t* ev) {
+    const PackedSpare spare = packed_spare(glu, T, F, K);
     if (few_supported(T, K, E))
         return launch_few(x, w1p, b1, w2p, b2, idx_in, w_in, types, T, H, F, E, K, bias_interleaved, act, out, glu, gexp,
-                          reinterpret_cast<unsigned char*>(Y), few_lists, s, ev);
+                          reinterpret_cast<unsigned char*>(Y), spare.few_lists, s, ev);
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     // what the kernels after the route read: the caller's arrays, or the int32 / fp32 ones that the route leaves
-    const int32_t* idx = types ? idx32 : idx_in;
-    const float* route_w = types ? w32 : static_cast<const float*>(w_in);
+    const int32_t* idx = types ? spare.idx32 : idx_in;
+    const float* route_w = types ? spare.w32 : static_cast<const float*>(w_in);
     const int nf1 = act_is_gated(act) ? F / 16 : F / 32, nf2 = H / 32;
     const int fw1 = pick_fw((long long)T * K, E, nf1, H, pk_cu_count());
     const int fw2 = pick_fw((long long)T * K, E, nf2, F, pk_cu_count());
@@ -1099,9 +1119,10 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
         const int bm = mid ? mid_tile_m() : stream_tile_m();
         const long long P = (long long)T * K;
         const int tiles = (int)((P + bm - 1) / bm + std::min<long long>(P, E));
+        if (tiles_form) tile_expert = spare.tile_expert;  // the workspace's own list holds tiles of 128 rows and more
         mark(0);
         hipError_t st = launch_route(idx_in, T, K, E, bm, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
-                                     meta + 8, s, rsig, nullptr, types, w_in, idx32, w32);
+                                     meta + 8, s, rsig, nullptr, types, w_in, spare.idx32, spare.w32);
         if (st != hipSuccess) return st;
         mark(1);
         st = launch_stream_gemm1(x, w1p, b1, T, H, F, E, K, bias_interleaved, act, offsets, tile_offsets, meta, sorted_pairs,
@@ -1134,7 +1155,7 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     mark(0);
     hipError_t st =
         launch_route(idx_in, T, K, E, kPkBM, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
-                     meta + 8, s, rsig, cost_split ? &split : nullptr, types, w_in, idx32, w32);
+                     meta + 8, s, rsig, cost_split ? &split : nullptr, types, w_in, spare.idx32, spare.w32);
     if (st != hipSuccess) return st;
     mark(1);
     PkParams g1{};

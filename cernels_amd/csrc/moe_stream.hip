@@ -859,14 +859,9 @@ bool few_supported(int T, int K, int E) {
     return T <= kFewMaxTokens && K <= kFewMaxTopk && P <= kFewMaxPairs;
 }
 
-// Bytes of the lists that the few form passes from its first to its second launch (16-byte aligned parts).
+// Parts of the lists that the few form passes from its first to its second launch, at `lists`: um experts, um x T glu rows,
+// um x nf1 flags, each to a multiple of 16 bytes.
 static size_t few_part(size_t n) { return (n + 15) / 16 * 16; }
-size_t few_workspace_bytes(int T, int F, int E, int K) {
-    const long long P = (long long)T * K;
-    if (!few_supported(T, K, E)) return 0;
-    const size_t um = (size_t)(P < E ? P : E);
-    return few_part(um * 4) + few_part(um * T * 2) + few_part(um * (F / 16));
-}
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
                             const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,

@@ -58,6 +58,20 @@ def test_workspace_sizes(L):
     assert L.cernels_moe_route_tile_capacity(1, 8, 128, 128) == 1 + 8
 
 
+@pytest.mark.parametrize("H,F,E,K", [(64, 64, 1024, 16), (512, 384, 256, 8), (64, 64, 8, 1), (64, 128, 513, 11),
+                                     (2880, 2880, 32, 4), (2048, 768, 128, 8), (128, 64, 4, 64)])
+def test_workspace_grows_with_every_size(L, H, F, E, K):
+    """A workspace sized for a caller's largest call serves every smaller one, whichever form of the path the smaller one
+    takes: the size never falls as T, K, E, F or H grows (over the token counts where the packed path changes form)."""
+    size = L.cernels_moe_experts_workspace_bytes
+    tokens = [*range(1, 130), *range(500, 530), 1024, 4096]
+    by_t = [size(t, H, F, E, K) for t in tokens]
+    assert all(a <= b for a, b in zip(by_t, by_t[1:])), [t for t, a, b in zip(tokens[1:], by_t, by_t[1:]) if b < a]
+    for t in (1, 16, 17, 32, 33, 64, 512):
+        for grown in ((t, H, F, E, K + 1), (t, H, F, E + 1, K), (t, H, F + 64, E, K), (t, H + 64, F, E, K)):
+            assert size(t, H, F, E, K) <= size(*grown), (t, grown)
+
+
 def _fake(n=0x10000):
     return ctypes.c_void_p(n)
 

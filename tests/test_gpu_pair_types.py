@@ -78,3 +78,32 @@ def test_loaders_refuse_what_they_refused(device):
         ops.moe_experts(d["x"], d["W1"], d["W2"], idx, d["w"], 2, decode=True)  # the op itself keeps to int32
     with pytest.raises(RuntimeError):
         ops.moe_experts_packed(d["x"], ops.pack_experts(d["W1"], d["W2"]), idx, d["w"], 2)
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (16, 1, 1), (32, 512, 16), (33, 40, 4), (512, 1024, 16), (700, 520, 16), (300, 4, 3),
+                                   (5000, 1024, 6)])
+def test_packed_typed_stays_in_its_workspace(device, T, E, K):
+    """Each form of the packed path, with ids and weights to convert, in a workspace of exactly the stated size (the smallest
+    layer, where the parts that share space lie closest): the bytes behind it stay as they were, the result is the op's."""
+    import ctypes
+
+    from cernels_amd import _native, ops
+
+    H = Fi = 64
+    c = rand_case(T + K, T, H, Fi, E, K)
+    d = to_device(c, device)
+    pk = ops.pack_experts(d["W1"], d["W2"])
+    idx, w = c["idx"].long().to(device), c["w"].bfloat16().to(device)
+    L = _native.lib()
+    n = L.cernels_moe_experts_workspace_bytes(T, H, Fi, E, K)
+    ws = torch.full((n + 4096,), 0x5A, dtype=torch.uint8, device=device)
+    out = torch.empty(T, H, dtype=torch.bfloat16, device=device)
+    print(f"[workspace T{T} E{E} K{K}]", flush=True)
+    st = L.cernels_moe_experts_packed_typed(
+        d["x"].data_ptr(), pk.gate_up.data_ptr(), None, pk.down.data_ptr(), None, idx.data_ptr(), _native.INDEX_I64, w.data_ptr(),
+        _native.WEIGHT_BF16, T, H, Fi, E, K, 0, _native.ACT_SILU, out.data_ptr(), ws.data_ptr(), ctypes.c_size_t(n),
+        torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    assert bool((ws[n:] == 0x5A).all())
+    assert torch.equal(out, ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], K))
+    assert_within_tolerance(out.cpu()[:64], oracle_fp64(c, slice(0, 64)), f"T{T} E{E} K{K}")
