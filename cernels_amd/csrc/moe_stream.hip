@@ -422,7 +422,8 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
     const int p = (valid ? fr : first) & 0x3fff;  // tokens without this expert read its first token's row and are dropped
     const int nst = prm.F / kBK;
     const int s0 = wave * nst / kStWaves, n = (wave + 1) * nst / kStWaves - s0;
-    int wx = prm.wexp[(long long)e * prm.NF + fc];
+    const int wx = prm.wexp[(long long)e * prm.NF + fc];
+    int smax = 0;  // power of two of the glu row
     const float rw0 = pair_weight(prm.route_w, prm.types, p);
     const uint32_t ao = (uint32_t)p * (uint32_t)(prm.F * 2) + 16u * half;
     const int nw = min(8, prm.NF - 8 * (fc >> 3));
@@ -435,10 +436,9 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
     if (!any_scaled) {
         stream_stages<f16x8>(rw, lane * 16u, nw * 1024, ra, ao, s0, n, acc);
     } else {  // some segment of this expert's rows is scaled: every segment to its row's largest scale first
-        int smax = kGluAnyScale;
+        smax = kGluAnyScale;
         for (int g = 0; g < prm.F / 16; ++g) smax = max(smax, (int)prm.gexp[(long long)g * prm.p_cap + p]);
         if (smax == kGluAnyScale) smax = 0;
-        wx += smax;
         for (int ks = 4 * s0; ks < 4 * (s0 + n); ++ks) {  // a k-step is one 16-column segment
             const f16x8 wq = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, ks * nw * 1024, 0));
             f16x8 aq = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(ra, ao, ks * 32, 0));
@@ -454,12 +454,24 @@ __global__ __launch_bounds__(kStThreads, 4) void moe_few_down_rows_kernel(Stream
     if (wave != 0 || !valid) return;  // lanes l and l ^ 32 hold the same row
     float v[16];
     sum_parts(part, lane, v);
-    store_y(prm.Y, p, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(rw0, wx));
+    // The weight and the fragment's power come first, the row's power last, as on the general path: w 2^(wx + smax) in one factor
+    // would be subnormal for rows of tiny glu (smax down to -126) whose products are not.
+    auto store = [&](int pp, float w) {
+        const float ws = __builtin_amdgcn_ldexpf(w, wx);
+        if (!any_scaled) {
+            store_y(prm.Y, pp, prm.H, fc, half, v, ws);
+            return;
+        }
+        float y[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] = __builtin_amdgcn_ldexpf(v[r] * ws, smax);
+        store_y(prm.Y, pp, prm.H, fc, half, y, 1.f);
+    };
+    store(p, rw0);
     if (again)  // further slots of the token that name the same expert
         for (int k = 0; k < prm.K; ++k) {
             const int pp = lrow * prm.K + k;
-            if (pp != p && pair_id(prm.idx, prm.types, pp) == e)
-                store_y(prm.Y, pp, prm.H, fc, half, v, __builtin_amdgcn_ldexpf(pair_weight(prm.route_w, prm.types, pp), wx));
+            if (pp != p && pair_id(prm.idx, prm.types, pp) == e) store(pp, pair_weight(prm.route_w, prm.types, pp));
         }
 }
 

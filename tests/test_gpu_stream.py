@@ -75,11 +75,12 @@ def test_few_rows(device, case):
     assert_within_tolerance(out, ref, str(case))
 
 
-@pytest.mark.parametrize("gain", [3000.0, 1e-4])
+@pytest.mark.parametrize("gain", [3000.0, 1e-4, 2.0 ** -57])
 @pytest.mark.parametrize("T,E,bias", [(5, 8, True), (30, 8, True), (40, 32, False)], ids=["fused", "rows", "tiles"])
 def test_few_rows_scaled_segments(device, T, E, bias, gain):
     """Rows whose glu leaves fp16's range (or falls to its subnormals) are stored scaled; each row group meets the bar on its
-    own scale, with columns 0-15 of two experts at zero so that scaled rows hold all-zero segments too."""
+    own scale, with columns 0-15 of two experts at zero so that scaled rows hold all-zero segments too. At 2^-57 glu lies near
+    2^-115: the product of the row's, the fragment's and the routing weight's powers is subnormal, the results are not."""
     K = 3
     c = rand_case(T, T, 256, 192, E, K, std=0.05, bias=bias and gain > 1)
     for e in (0, 3):
