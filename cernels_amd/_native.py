@@ -30,6 +30,7 @@ ACT_GELU_TANH, ACT_SILU_PLAIN, ACT_RELU = 2, 3, 4  # non-gated (megablocks)
 GATE_UP, DOWN, UP = 0, 1, 2
 ROUTER_SOFTMAX_TOPK, ROUTER_TOPK_SOFTMAX = 0, 1
 INDEX_I32, INDEX_I64 = 0, 1
+PACKED_FORMS = ("grouped", "grouped_split", "few_sum", "few_rows", "tiles", "items")
 WEIGHT_F32, WEIGHT_BF16 = 0, 1
 
 _P = ctypes.c_void_p
@@ -42,6 +43,7 @@ _SIGNATURES = {
     "cernels_moe_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "cernels_moe_route_tile_capacity": (_S, [_I, _I, _I, _I]),
     "cernels_moe_route_workspace_bytes": (_S, [_I, _I, _I]),
+    "cernels_moe_route_launches": (_I, [_I, _I, _I]),
     "cernels_moe_route": (ctypes.c_int, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _S, _P]),
     "cernels_moe_experts_workspace_bytes": (_S, [_I, _I, _I, _I, _I]),
     "cernels_moe_experts": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _S, _P]),
@@ -55,6 +57,7 @@ _SIGNATURES = {
     ),
     "cernels_moe_packed_weight_bytes": (_S, [_I, _I, _I, _I]),
     "cernels_moe_pack_weights": (ctypes.c_int, [_P, _I, _I, _I, _I, _I, _P, _P]),
+    "cernels_moe_experts_packed_form": (_I, [_I, _I, _I, _I, _I, _I]),
     "cernels_moe_experts_packed": (
         ctypes.c_int,
         [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _S, _P],

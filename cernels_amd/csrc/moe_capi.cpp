@@ -40,6 +40,8 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
                                  int bias_interleaved, int act, void* out, int32_t* offsets, int32_t* tile_offsets, int32_t* meta,
                                  int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts, int max_tiles, uint16_t* glu,
                                  float* Y, int8_t* gexp, int8_t* rsig, int8_t* psig, hipStream_t s, hipEvent_t* ev);
+int packed_form(int T, int H, int F, int E, int K, int act, int max_tiles);
+int route_launches(int T, int K, int E);
 hipError_t launch_decode(const uint16_t* x, const uint16_t* w1, const float* b1, const uint16_t* w2, const float* b2,
                          const int32_t* idx, const void* w, int types, uint16_t* glu, int32_t* order, float* order_w,
                          uint16_t* out, int T, int H, int F, int E, int K, int act, hipStream_t s, hipEvent_t* ev);
@@ -162,6 +164,11 @@ size_t cernels_moe_route_tile_capacity(int32_t T, int32_t K, int32_t E, int32_t 
     return (size_t)(cap > 0 ? cap : 1);
 }
 
+int32_t cernels_moe_route_launches(int32_t T, int32_t K, int32_t E) {
+    if (T < 0 || K <= 0 || K > kMaxTopk || E <= 0 || E > kMaxExperts || (long long)T * K >= (1LL << 31)) return -1;
+    return cmoe::route_launches(T, K, E);
+}
+
 int cernels_moe_route(const int32_t* indices, int32_t T, int32_t K, int32_t E, int32_t tile_m,
                       int32_t* expert_offsets, int32_t* sorted_pairs, int32_t* tile_offsets, int32_t* tile_expert,
                       int32_t* meta, void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -246,6 +253,12 @@ int cernels_moe_pack_weights(const void* src, int32_t H, int32_t F, int32_t E, i
     if (!aligned16(src) || !aligned16(dst)) return CERNELS_MOE_MISALIGNED;
     return hip_status(cmoe::launch_pack(static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), E, H, F,
                                         layout, which, stream));
+}
+
+int32_t cernels_moe_experts_packed_form(int32_t T, int32_t H, int32_t F, int32_t E, int32_t K, int32_t act) {
+    if (!dims_ok(T, H, F, E, K) || T == 0 || H % 64 || F % 64 || E > kMaxExperts) return -1;
+    if (act < CERNELS_MOE_ACT_SILU || act > CERNELS_MOE_ACT_RELU) return -1;
+    return cmoe::packed_form(T, H, F, E, K, act, prefill_ws(T, H, F, E, K).capacity);
 }
 
 namespace {

@@ -1059,6 +1059,7 @@ hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t
                             hipStream_t s, int types = 0);
 
 bool few_supported(int T, int K, int E);
+bool few_sums(int T, int K);
 bool tiles_supported(int T, int K, int E);
 hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
                       const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
@@ -1094,6 +1095,46 @@ static PackedSpare packed_spare(uint16_t* glu, int T, int F, int K) {
     return sp;
 }
 
+// Which form a call takes, from its sizes alone, and the launch shapes of the grouped GEMMs: fragments per item, N-tiles and
+// workgroups per XCD of both. max_tiles bounds the M-tile list of 256 rows.
+struct PackedPlan {
+    int form, nf1, nf2, fw1, fw2, nt1, nt2, slots1, slots2;
+};
+static PackedPlan packed_plan(int T, int H, int F, int E, int K, int act, int max_tiles) {
+    const long long P = (long long)T * K;
+    PackedPlan pl{};
+    pl.nf1 = act_is_gated(act) ? F / 16 : F / 32;
+    pl.nf2 = H / 32;
+    if (few_supported(T, K, E)) {
+        pl.form = few_sums(T, K) ? kFormFewSum : kFormFewRows;
+        return pl;
+    }
+    if (tiles_supported(T, K, E)) {
+        pl.form = kFormTiles;
+        return pl;
+    }
+    pl.fw1 = pick_fw(P, E, pl.nf1, H, pk_cu_count());
+    pl.fw2 = pick_fw(P, E, pl.nf2, F, pk_cu_count());
+    if (mid_supported(P, E, pl.nf1, pl.nf2, H, F, pl.fw1, pl.fw2, pk_cu_count())) {
+        pl.form = kFormItems;
+        return pl;
+    }
+    // The route splits each GEMM's items over the XCDs (meta[32..40] gate_up, meta[41..49] down). Where even the most M-tiles
+    // the route can make (ceil(P / 256) + min(P, E)) would give each workgroup fewer than 8 rounds of items, the split is the
+    // equal one for both GEMMs (moe_split.h) and the GEMMs compute it themselves.
+    pl.nt1 = ceil_div(pl.nf1, pl.fw1);
+    pl.nt2 = ceil_div(pl.nf2, pl.fw2);
+    pl.slots1 = pk_grid(max_tiles, pl.nt1) / 8;
+    pl.slots2 = pk_grid(max_tiles, pl.nt2) / 8;
+    const long long mt_max = (P + kPkBM - 1) / kPkBM + std::min<long long>(P, E);
+    auto max_rounds = [&](int nt, int slots) { return (mt_max * nt + 8LL * slots - 1) / (8LL * slots); };
+    pl.form = std::max(max_rounds(pl.nt1, pl.slots1), max_rounds(pl.nt2, pl.slots2)) >= 8 ? kFormGroupedSplit : kFormGrouped;
+    return pl;
+}
+int packed_form(int T, int H, int F, int E, int K, int act, int max_tiles) {
+    return packed_plan(T, H, F, E, K, act, max_tiles).form;
+}
+
 // route -> packed gate_up GEMM -> packed down GEMM -> combine, all on stream s; few rows per expert take the streaming
 // forms of moe_stream.hip instead (its header states where the lines lie and why). Shapes were checked
 // by the caller (H % 64 == 0, F % 64 == 0, E <= 1024, T >= 1).
@@ -1103,23 +1144,20 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
                                  int32_t* sorted_pairs, int32_t* tile_expert, int32_t* route_counts, int max_tiles, uint16_t* glu,
                                  float* Y, int8_t* gexp, int8_t* rsig, int8_t* psig, hipStream_t s, hipEvent_t* ev) {
     const PackedSpare spare = packed_spare(glu, T, F, K);
-    if (few_supported(T, K, E))
+    const PackedPlan pl = packed_plan(T, H, F, E, K, act, max_tiles);
+    if (pl.form == kFormFewSum || pl.form == kFormFewRows)
         return launch_few(x, w1p, b1, w2p, b2, idx_in, w_in, types, T, H, F, E, K, bias_interleaved, act, out, glu, gexp,
                           reinterpret_cast<unsigned char*>(Y), spare.few_lists, s, ev);
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     // what the kernels after the route read: the caller's arrays, or the int32 / fp32 ones that the route leaves
     const int32_t* idx = types ? spare.idx32 : idx_in;
     const float* route_w = types ? spare.w32 : static_cast<const float*>(w_in);
-    const int nf1 = act_is_gated(act) ? F / 16 : F / 32, nf2 = H / 32;
-    const int fw1 = pick_fw((long long)T * K, E, nf1, H, pk_cu_count());
-    const int fw2 = pick_fw((long long)T * K, E, nf2, F, pk_cu_count());
-    const bool tiles_form = tiles_supported(T, K, E);
-    const bool mid = !tiles_form && mid_supported((long long)T * K, E, nf1, nf2, H, F, fw1, fw2, pk_cu_count());
-    if (tiles_form || mid) {  // moe_stream.hip
+    if (pl.form == kFormTiles || pl.form == kFormItems) {  // moe_stream.hip
+        const bool mid = pl.form == kFormItems;
         const int bm = mid ? mid_tile_m() : stream_tile_m();
         const long long P = (long long)T * K;
         const int tiles = (int)((P + bm - 1) / bm + std::min<long long>(P, E));
-        if (tiles_form) tile_expert = spare.tile_expert;  // the workspace's own list holds tiles of 128 rows and more
+        if (!mid) tile_expert = spare.tile_expert;  // the workspace's own list holds tiles of 128 rows and more
         mark(0);
         hipError_t st = launch_route(idx_in, T, K, E, bm, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
                                      meta + 8, s, rsig, nullptr, types, w_in, spare.idx32, spare.w32);
@@ -1142,16 +1180,8 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
         mark(4);
         return st;
     }
-    // Launch shapes of both GEMMs, from the shape alone; the route then splits each one's items over
-    // the XCDs (meta[32..40] gate_up, meta[41..49] down). Where even the most M-tiles the route can
-    // make (ceil(P / 256) + min(P, E)) would give each workgroup fewer than 8 rounds of items, the
-    // split is the equal one for both GEMMs (moe_split.h) and the GEMMs compute it themselves.
-    const int nt1 = ceil_div(nf1, fw1), nt2 = ceil_div(nf2, fw2);
-    const int slots1 = pk_grid(max_tiles, nt1) / 8, slots2 = pk_grid(max_tiles, nt2) / 8;
-    const long long P = (long long)T * K, mt_max = (P + kPkBM - 1) / kPkBM + std::min<long long>(P, E);
-    auto max_rounds = [&](int nt, int slots) { return (mt_max * nt + 8LL * slots - 1) / (8LL * slots); };
-    const bool cost_split = max(max_rounds(nt1, slots1), max_rounds(nt2, slots2)) >= 8;
-    XcdSplit split{{fw1, fw2}, {nt1, nt2}, {slots1, slots2}, meta + 32};
+    const bool cost_split = pl.form == kFormGroupedSplit;
+    XcdSplit split{{pl.fw1, pl.fw2}, {pl.nt1, pl.nt2}, {pl.slots1, pl.slots2}, meta + 32};
     mark(0);
     hipError_t st =
         launch_route(idx_in, T, K, E, kPkBM, offsets, sorted_pairs, tile_offsets, tile_expert, meta, route_counts,
@@ -1171,10 +1201,10 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     g1.route_w = route_w;
     g1.out = glu;
     g1.Kd = H;
-    g1.NF = nf1;
+    g1.NF = pl.nf1;
     g1.KS = H / 16;
-    g1.fw = fw1;
-    g1.n_tiles = nt1;
+    g1.fw = pl.fw1;
+    g1.n_tiles = pl.nt1;
     g1.F = F;
     g1.H = H;
     g1.topk = K;
@@ -1210,11 +1240,11 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     g2.out = Y;  // written as 24-bit floats (3/4 of the fp32 buffer)
     g2.wexp = reinterpret_cast<const int8_t*>(static_cast<const uint16_t*>(w2p) + (long long)E * H * F);
     g2.Kd = F;
-    g2.NF = nf2;
+    g2.NF = pl.nf2;
     g2.KS = F / 16;
-    g2.fw = fw2;
+    g2.fw = pl.fw2;
     g2.counters = meta + 16;
-    g2.n_tiles = nt2;
+    g2.n_tiles = pl.nt2;
     g2.bounds = cost_split ? meta + 41 : nullptr;
     g2.bias = nullptr;  // the down bias is added by the combine
     g2.tail = 0;

@@ -12,7 +12,6 @@ constexpr int kPkFrag = 512;  // bf16 elements of one fragment (1 KB)
 constexpr float kGluSmall = 0.00390625f;
 constexpr int kGluAnyScale = -128;
 
-
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kModePkGateUp = 0;
@@ -33,6 +32,14 @@ __host__ __device__ inline long long packed_frag(int e, int c, int ks, int NF, i
     const int t = c >> 3, w = c & 7, nw = min(8, NF - 8 * t);
     return (long long)e * NF * KS + 8LL * KS * t + (long long)ks * nw + w;
 }
+
+// The forms of the packed path (mirrors cernels_moe_packed_form in include/cernels_moe.h).
+constexpr int kFormGrouped = 0;       // persistent grouped GEMMs, equal item ranges per XCD
+constexpr int kFormGroupedSplit = 1;  // the same, with the cost-balanced ranges that the route writes
+constexpr int kFormFewSum = 2;        // few tokens, the sum over slots in the down kernel
+constexpr int kFormFewRows = 3;       // few tokens, a Y row per pair and the combine
+constexpr int kFormTiles = 4;         // streaming kernels over 32-row M-tiles
+constexpr int kFormItems = 5;         // a workgroup per item of 128 rows
 
 // Whether a glu segment whose largest |value| is m is stored scaled, and the power of two s it is then scaled by:
 // m * 2^-s in [2^14, 2^15); s >= 1 for m >= 2^15 (inf or nan: s = 1), s <= -23 for 0 < m < 2^-8 (clamped at -126, so

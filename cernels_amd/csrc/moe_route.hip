@@ -434,6 +434,16 @@ __global__ __launch_bounds__(kRtThreads) void moe_pairs_kernel(const int32_t* __
 int route_tiles(int T, int K) { return ceil_div(T * K, kRtTile); }
 size_t route_workspace_bytes(int T, int K, int E) { return (size_t)max(route_tiles(T, K), 1) * E * sizeof(int32_t); }
 
+// Whether the histograms of a route fit the LDS of the one-launch kernel, or of the count + scan kernel.
+static bool route_fits_one(int nt, int E) { return nt > 0 && (long long)(nt + kRouteWaves) * E <= kRtOneCells; }
+static bool route_fits_count_scan(int nt, int E) { return (long long)nt * E <= kRtFusedCells; }
+
+// Launches of a route on int32 ids: one; count + scan in one, scatter; or count, scan, scatter.
+int route_launches(int T, int K, int E) {
+    const int nt = route_tiles(T, K);
+    return route_fits_one(nt, E) ? 1 : (route_fits_count_scan(nt, E) ? 1 : 2) + (nt > 0);
+}
+
 template <int IS>
 static hipError_t launch_route_one(const int32_t* idx, const void* route_w, int types, int32_t* idx32, float* w32, int T, int K,
                                    int E, int BM, int nt, int32_t* offsets, int32_t* sorted_pairs, int32_t* tile_offsets,
@@ -460,7 +470,7 @@ hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t
     const int nt = route_tiles(T, K);
     const XcdSplit sp = split ? *split : XcdSplit{};
     if (types == 0) idx32 = nullptr;
-    if (nt > 0 && (long long)(nt + kRouteWaves) * E <= kRtOneCells)
+    if (route_fits_one(nt, E))
         return (types & kPairsI64 ? launch_route_one<2> : launch_route_one<1>)(idx, route_w, types, idx32, w32, T, K, E, BM, nt,
                                                                                offsets, sorted_pairs, tile_offsets, tile_expert,
                                                                                meta, sched, stream, row_zero, sp);
@@ -469,7 +479,7 @@ hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t
                            T * K, idx32, w32);
         idx = idx32;
     }
-    if ((long long)nt * E <= kRtFusedCells) {
+    if (route_fits_count_scan(nt, E)) {
         hipLaunchKernelGGL(moe_route_count_scan_kernel, dim3(1), dim3(kRouteThreads), 0, stream, idx, T, K, E, BM, nt,
                            counts, offsets, tile_offsets, tile_expert, meta, sched, sp);
     } else {

@@ -871,6 +871,9 @@ bool few_supported(int T, int K, int E) {
     return T <= kFewMaxTokens && K <= kFewMaxTopk && P <= kFewMaxPairs;
 }
 
+// Whether the few form's down kernel sums over the slots itself (kFdMaxPairs).
+bool few_sums(int T, int K) { return (long long)T * K <= kFdMaxPairs; }
+
 // Parts of the lists that the few form passes from its first to its second launch, at `lists`: um experts, um x T glu rows,
 // um x nf1 flags, each to a multiple of 16 bytes.
 static size_t few_part(size_t n) { return (n + 15) / 16 * 16; }
@@ -933,7 +936,7 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
     q.NF = H / 32;
     q.KS = F / 16;
     q.out = static_cast<uint16_t*>(out);
-    if (P > kFdMaxPairs) {
+    if (!few_sums(T, K)) {
         q.Y = Y;
         hipLaunchKernelGGL(moe_few_down_rows_kernel, dim3(q.NF, um), dim3(kStThreads), 0, s, q);
         st = hipGetLastError();

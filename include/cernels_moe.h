@@ -74,6 +74,8 @@ const char* cernels_moe_status_string(int status);
  * Limits: 1 <= E <= 1024, 1 <= K <= 4096, T*K < 2^31, tile_m >= 1. */
 size_t cernels_moe_route_tile_capacity(int32_t T, int32_t K, int32_t E, int32_t tile_m);
 size_t cernels_moe_route_workspace_bytes(int32_t T, int32_t K, int32_t E);
+/* Kernel launches of one route (1, 2 or 3; -1 for sizes outside the limits): which of its three forms the sizes take. */
+int32_t cernels_moe_route_launches(int32_t T, int32_t K, int32_t E);
 int cernels_moe_route(const int32_t* indices, int32_t T, int32_t K, int32_t E, int32_t tile_m,
                       int32_t* expert_offsets, int32_t* sorted_pairs, int32_t* tile_offsets,
                       int32_t* tile_expert, int32_t* meta, void* workspace, size_t workspace_bytes,
@@ -135,6 +137,19 @@ int cernels_moe_experts_packed_staged(const void* x, const void* gate_up_packed,
                                       const float* weights, int32_t T, int32_t H, int32_t F, int32_t E, int32_t K,
                                       int32_t bias_layout, int32_t act, void* out, void* workspace,
                                       size_t workspace_bytes, hipStream_t stream, hipEvent_t* stage_events);
+
+/* Which kernels a packed call of these sizes takes on the current device (-1 for sizes or an act that the entry refuses):
+ * persistent grouped GEMMs with equal or with cost-balanced item ranges per XCD; the few-token kernels with the sum over slots
+ * in the second one, or with a row per pair; streaming kernels over 32-row tiles; one workgroup per item of 128 rows. */
+enum cernels_moe_packed_form {
+    CERNELS_MOE_FORM_GROUPED = 0,
+    CERNELS_MOE_FORM_GROUPED_SPLIT = 1,
+    CERNELS_MOE_FORM_FEW_SUM = 2,
+    CERNELS_MOE_FORM_FEW_ROWS = 3,
+    CERNELS_MOE_FORM_TILES = 4,
+    CERNELS_MOE_FORM_ITEMS = 5
+};
+int32_t cernels_moe_experts_packed_form(int32_t T, int32_t H, int32_t F, int32_t E, int32_t K, int32_t act);
 
 /* The same with the routing in the types a transformers router returns: indices int32 or int64 (the id is the low 32
  * bits, as a cast to int32 takes it; 8-byte aligned), weights fp32 or bf16 (2-byte aligned). Same workspace. */

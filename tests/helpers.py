@@ -61,6 +61,23 @@ def run_gpu(c, device, decode=False, dev_tensors=None):
                            gate_up_bias=d["b1"], down_bias=d["b2"], decode=decode)
 
 
+def packed_form(T, H, Fi, E, K, act="silu"):
+    """Which kernels a packed call of these sizes takes (``_native.PACKED_FORMS``); act: "silu", "gptoss" or a megablocks
+    act_id. Tests of one form assert it, so that a moved line cannot turn them into tests of another."""
+    from cernels_amd import _native, ops
+
+    a = {"silu": ops.ACT_SILU, "gptoss": ops.ACT_GPTOSS, **ops.MEGABLOCKS_ACTS}[act]
+    form = _native.lib().cernels_moe_experts_packed_form(T, H, Fi, E, K, a)
+    assert form >= 0, (T, H, Fi, E, K, act)
+    return _native.PACKED_FORMS[form]
+
+
+def form_of(c):
+    """``packed_form`` of a case of ``rand_case``."""
+    (E, n1, n2), (T, H), K = c["W1"].shape, c["x"].shape, c["idx"].shape[1]
+    return packed_form(T, H, (n1 if c["layout"] == "concat" else n2) // 2, E, K, c["act"])
+
+
 def to_device(c, device):
     mv = lambda t, dt=None: None if t is None else (t.to(dt) if dt else t).contiguous().to(device)  # noqa: E731
     return dict(x=mv(c["x"]), W1=mv(c["W1"]), W2=mv(c["W2"]), idx=mv(c["idx"], torch.int32),

@@ -72,6 +72,23 @@ def test_workspace_grows_with_every_size(L, H, F, E, K):
             assert size(t, H, F, E, K) <= size(*grown), (t, grown)
 
 
+def test_packed_forms_on_their_lines(L):
+    """Which kernels a packed call takes, on both sides of each line (256 CUs, also the library's figure without a GPU)."""
+    lines = [
+        ((1, 64, 64, 8, 16), "few_sum"), ((1, 64, 64, 8, 17), "few_rows"), ((32, 64, 64, 512, 16), "few_rows"),
+        ((32, 64, 64, 512, 17), "tiles"), ((33, 64, 64, 512, 16), "tiles"), ((8, 64, 64, 8, 64), "few_rows"),
+        ((1, 64, 64, 1024, 64), "few_rows"), ((1, 64, 64, 1024, 65), "tiles"), ((512, 64, 64, 64, 1), "tiles"),
+        ((513, 64, 64, 65, 1), "grouped"), ((64, 64, 64, 32, 4), "tiles"), ((65, 64, 64, 32, 4), "grouped"),
+        ((1440, 2048, 768, 128, 8), "items"), ((1441, 2048, 768, 128, 8), "grouped"), ((4096, 2880, 2880, 32, 4), "grouped_split"),
+    ]
+    for sizes, form in lines:
+        assert _native.PACKED_FORMS[L.cernels_moe_experts_packed_form(*sizes, 0)] == form, sizes
+    for bad in ((0, 64, 64, 8, 2, 0), (4, 96, 64, 8, 2, 0), (4, 64, 64, 1025, 2, 0), (4, 64, 64, 8, 2, 9), (4, 64, 64, 8, 0, 0)):
+        assert L.cernels_moe_experts_packed_form(*bad) == -1
+    assert [L.cernels_moe_route_launches(*a) for a in ((0, 4, 8), (333, 6, 64), (6000, 4, 1024), (8192, 8, 1024))] == [1, 1, 2, 3]
+    assert L.cernels_moe_route_launches(4, 4, 1025) == -1
+
+
 def _fake(n=0x10000):
     return ctypes.c_void_p(n)
 

@@ -10,7 +10,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from helpers import assert_within_tolerance, oracle_fp64, rand_case, to_device
+from helpers import assert_within_tolerance, form_of, oracle_fp64, packed_form, rand_case, to_device
 from oracle import eager as O
 
 pytestmark = pytest.mark.gpu
@@ -21,7 +21,7 @@ FEW_ROWS, MANY_ROWS = (512, 40, 192, 320), (40, 300, 1088, 576)
 
 
 def _ids(E, mean, seed):
-    """One id per token: expert e < len(EDGES) exactly EDGES[e] times, the others evenly up to the average."""
+    """Ids: expert e < len(EDGES) exactly EDGES[e] times, the others evenly up to the average."""
     rest = E * mean - sum(EDGES)
     n = E - len(EDGES)
     counts = EDGES + [rest // n + (i < rest % n) for i in range(n)]
@@ -39,13 +39,15 @@ def _packed(c, device):
     return ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], d["idx"].shape[1]).cpu()
 
 
-def _case(shape, kind, seed=3):
+def _case(shape, kind, seed=3, K=1):
     E, mean, H, Fi = shape
     layout, act, bias = kind
     ids = _ids(E, mean, seed)
-    c = rand_case(seed, len(ids), H, Fi, E, 1, layout=layout, act=act, bias=bias, std=0.05)
-    c["idx"][:, 0] = ids
-    c["w"] = torch.rand(len(ids), 1, generator=torch.Generator().manual_seed(seed)).bfloat16()
+    T = len(ids) // K
+    c = rand_case(seed, T, H, Fi, E, K, layout=layout, act=act, bias=bias, std=0.05)
+    c["idx"] = ids.reshape(T, K)  # a token may name an expert twice
+    c["w"] = torch.rand(T, K, generator=torch.Generator().manual_seed(seed)).bfloat16()
+    assert form_of(c) == "items"
     return c
 
 
@@ -56,6 +58,15 @@ def test_items_row_edges(device, shape, kind):
     c = _case(shape, kind)
     print(f"[items {shape} {kind}]", flush=True)
     assert_within_tolerance(_packed(c, device), oracle_fp64(c), f"{shape} {kind}")
+
+
+@pytest.mark.parametrize("K", [2, 5])
+@pytest.mark.parametrize("shape", [FEW_ROWS, MANY_ROWS], ids=["few", "many"])
+def test_items_several_slots(device, shape, K):
+    """Several pairs per token: a row's token is not its pair, and the combine sums the slots."""
+    c = _case(shape, ("interleaved", "gptoss", True), seed=7, K=K)
+    print(f"[items {shape} K{K}]", flush=True)
+    assert_within_tolerance(_packed(c, device), oracle_fp64(c), f"{shape} K{K}")
 
 
 @pytest.mark.parametrize("shape", [FEW_ROWS, MANY_ROWS], ids=["few", "many"])
@@ -96,6 +107,7 @@ def test_items_nongated(device, shape, act_id):
     E, mean, H, Fi = shape
     g = torch.Generator().manual_seed(act_id)
     idx = _ids(E, mean, act_id)[:, None].int()
+    assert packed_form(len(idx), H, Fi, E, 1, act_id) == "items"
     x = torch.randn(len(idx), H, generator=g).bfloat16()
     w1 = (torch.randn(E, H, Fi, generator=g) * 0.05).bfloat16()
     w2 = (torch.randn(E, Fi, H, generator=g) * 0.05).bfloat16()

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from conftest import GOLDEN_NAMES, load_golden
-from helpers import (assert_reference_verify, assert_strict_full, assert_within_tolerance, full_case, oracle_eager,
+from helpers import (assert_reference_verify, assert_strict_full, assert_within_tolerance, form_of, full_case, oracle_eager,
                      oracle_fp64, rand_case, run_gpu, to_device)
 
 pytestmark = pytest.mark.gpu
@@ -128,9 +128,11 @@ SMALL = [
     (7, 1, 128, 64, 16, 8, "concat", "silu", False, 0, 0.0),
     (8, 1200, 256, 128, 64, 6, "concat", "silu", False, 0, 1.2),
     (9, 700, 576, 320, 3, 2, "concat", "silu", False, 0, 0.0),  # 20 and 18 fragments: idle waves in the last tile
-    # routes past the one-launch route's LDS limit (the GEMMs' work counters are then zeroed by the scan launch)
+    # routes past the one-launch route's LDS limit, before items of 128 rows (no counters): two and three launches
     (10, 6000, 64, 64, 1024, 4, "concat", "silu", False, 5, 0.0),
     (11, 8192, 64, 64, 1024, 8, "concat", "silu", False, 0, 1.0),
+    # the same before the persistent GEMMs (the scan launch zeroes their work counters)
+    (12, 8192, 64, 128, 512, 8, "concat", "silu", False, 5, 1.0),
 ]
 
 
@@ -139,6 +141,11 @@ def test_packed_small(device, case):
     seed, T, H, Fi, E, K, layout, act, bias, invalid, skew = case
     c = rand_case(seed, T, H, Fi, E, K, layout=layout, act=act, bias=bias, invalid=invalid, skew=skew,
                   std=0.05 if act == "gptoss" else 0.02)
+    if seed >= 10:
+        from cernels_amd import _native
+
+        launches = _native.lib().cernels_moe_route_launches(T, K, E)
+        assert (form_of(c), launches) == {10: ("items", 2), 11: ("items", 3), 12: ("grouped", 3)}[seed]
     print(f"[packed small {case}]", flush=True)
     out = _run_packed(c, device).cpu()
     assert_within_tolerance(out, oracle_fp64(c), str(case))
@@ -153,6 +160,7 @@ def test_packed_cost_split_many_rounds(device):
     c = rand_case(31, 2048, 128, 4096, 16, 8, skew=1.5)
     runs = torch.bincount(c["idx"].flatten(), minlength=16)
     assert int((-(-runs // 256)).sum()) * 32 >= 8 * 8 * 32  # >= 8 rounds at fw = 8 on 256 CUs
+    assert form_of(c) == "grouped_split"
     print("[packed cost split] T2048 H128 F4096 E16 k8", flush=True)
     out = _run_packed(c, device).cpu()
     rows = torch.randperm(2048, generator=torch.Generator().manual_seed(5))[:160]
@@ -160,13 +168,16 @@ def test_packed_cost_split_many_rounds(device):
     assert_reference_verify(out[rows], oracle_eager(c, rows), "cost split")
 
 
-@pytest.mark.parametrize("T", [3200, 4096], ids=["count_scan_route", "two_launch_route"])
-def test_packed_cost_split_other_route_kernels(device, T):
-    """The same per-XCD split written by the route's other two kernels: E = 1024 experts with
-    T x 8 pairs is past the one-launch route's LDS (count + scan in one launch at 25 route tiles,
-    separate launches at 32), and ~4000 small items give every workgroup 8+ rounds."""
-    c = rand_case(41, T, 64, 512, 1024, 8, skew=1.0)
-    print(f"[packed cost split, route T={T}] H64 F512 E1024 k8", flush=True)
+@pytest.mark.parametrize("T,E", [(8192, 512), (12288, 1024)])
+def test_packed_cost_split_separate_scan(device, T, E):
+    """The same per-XCD split written by the scan launch of the three-launch route: 64 and 96 route tiles of T x 8 pairs are past
+    the one-launch route's LDS, and 2000 and more items give every workgroup 8+ rounds. (The route that counts and scans in
+    one launch serves at most 58 rows per expert, where no call takes the persistent GEMMs.)"""
+    from cernels_amd import _native
+
+    c = rand_case(41, T, 64, 512, E, 8, skew=1.0)
+    assert form_of(c) == "grouped_split" and _native.lib().cernels_moe_route_launches(T, 8, E) == 3
+    print(f"[packed cost split, route T={T}] H64 F512 E{E} k8", flush=True)
     out = _run_packed(c, device).cpu()
     rows = torch.randperm(T, generator=torch.Generator().manual_seed(6))[:256]
     assert_within_tolerance(out[rows], oracle_fp64(c, rows), f"cost split route T={T}")

@@ -11,7 +11,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from helpers import assert_within_tolerance, oracle_fp64, rand_case, to_device
+from helpers import assert_within_tolerance, form_of, oracle_fp64, packed_form, rand_case, to_device
 from oracle import eager as O
 
 pytestmark = pytest.mark.gpu
@@ -29,25 +29,26 @@ def _packed(c, device):
 
 SILU, GPT = ("concat", "silu", False), ("interleaved", "gptoss", True)
 CASES = [
-    # T, H, F, E, K, (layout, act, bias), ids
-    (1, 64, 64, 1, 1, SILU, "plain"),          # one stage per projection: three of the four waves have none
-    (1, 192, 320, 1024, 16, SILU, "plain"),    # 16 pairs in one token, partial last bundles
-    (16, 128, 192, 3, 1, GPT, "plain"),        # 16 pairs, the fused down's last
-    (17, 128, 192, 3, 1, GPT, "plain"),        # 17: rows and combine
-    (4, 576, 64, 9, 4, GPT, "twice"),
-    (5, 320, 128, 6, 3, SILU, "twice"),        # rows form, an expert named twice by one token
-    (7, 128, 64, 12, 2, SILU, "invalid"),
-    (3, 128, 64, 4, 2, GPT, "none"),           # no valid id at all: zeros
-    (20, 128, 64, 4, 2, SILU, "none"),
-    (32, 128, 128, 512, 16, SILU, "plain"),    # 512 pairs
-    (32, 128, 128, 512, 17, SILU, "plain"),    # 544: the route's list (tiles)
-    (32, 1088, 448, 64, 8, GPT, "same"),       # every token on the same experts
-    (33, 128, 192, 64, 4, SILU, "invalid"),    # 33 tokens: tiles
-    (64, 256, 128, 32, 4, GPT, "plain"),       # 8 rows per expert: tiles' last
-    (65, 256, 128, 32, 4, GPT, "plain"),       # above: the grouped GEMMs
-    (512, 128, 64, 64, 1, SILU, "same"),       # one expert with 512 rows: 16 tiles
-    (513, 128, 64, 65, 1, SILU, "plain"),
-    (90, 192, 64, 40, 3, SILU, "twice"),
+    # T, H, F, E, K, (layout, act, bias), ids, the form that the call takes
+    (1, 64, 64, 1, 1, SILU, "plain", "few_sum"),  # one stage per projection: three of the four waves have none
+    (1, 192, 320, 1024, 16, SILU, "plain", "few_sum"),  # 16 pairs in one token, partial last bundles
+    (16, 128, 192, 3, 1, GPT, "plain", "few_sum"),  # 16 pairs, the fused down's last
+    (17, 128, 192, 3, 1, GPT, "plain", "few_rows"),  # 17: rows and combine
+    (4, 576, 64, 9, 4, GPT, "twice", "few_sum"),
+    (5, 320, 128, 6, 3, SILU, "twice", "few_sum"),  # an expert named twice by one token
+    (11, 320, 128, 6, 3, SILU, "twice", "few_rows"),
+    (7, 128, 64, 12, 2, SILU, "invalid", "few_sum"),
+    (3, 128, 64, 4, 2, GPT, "none", "few_sum"),  # no valid id at all: zeros
+    (20, 128, 64, 4, 2, SILU, "none", "few_rows"),
+    (32, 128, 128, 512, 16, SILU, "plain", "few_rows"),  # 512 pairs
+    (32, 128, 128, 512, 17, SILU, "plain", "tiles"),  # 544: the route's list (tiles)
+    (32, 1088, 448, 64, 8, GPT, "same", "few_rows"),  # every token on the same experts
+    (33, 128, 192, 64, 4, SILU, "invalid", "tiles"),  # 33 tokens: tiles
+    (64, 256, 128, 32, 4, GPT, "plain", "tiles"),  # 8 rows per expert: tiles' last
+    (65, 256, 128, 32, 4, GPT, "plain", "grouped"),  # above: the grouped GEMMs
+    (512, 128, 64, 64, 1, SILU, "same", "tiles"),  # one expert with 512 rows: 16 tiles
+    (513, 128, 64, 65, 1, SILU, "plain", "grouped"),
+    (90, 192, 64, 40, 3, SILU, "twice", "tiles"),
 ]
 
 
@@ -66,7 +67,8 @@ def _case(T, H, Fi, E, K, kind, ids):
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"T{c[0]}H{c[1]}F{c[2]}E{c[3]}k{c[4]}{c[5][1]}-{c[6]}")
 def test_few_rows(device, case):
-    c = _case(*case)
+    c = _case(*case[:7])
+    assert form_of(c) == case[7]
     print(f"[few rows {case}]", flush=True)
     out = _packed(c, device)
     ref = oracle_fp64(c)
@@ -76,13 +78,15 @@ def test_few_rows(device, case):
 
 
 @pytest.mark.parametrize("gain", [3000.0, 1e-4, 2.0 ** -57])
-@pytest.mark.parametrize("T,E,bias", [(5, 8, True), (30, 8, True), (40, 32, False)], ids=["fused", "rows", "tiles"])
-def test_few_rows_scaled_segments(device, T, E, bias, gain):
+@pytest.mark.parametrize("T,E,bias,form", [(5, 8, True, "few_sum"), (30, 8, True, "few_rows"), (40, 32, False, "tiles")],
+                         ids=["fused", "rows", "tiles"])
+def test_few_rows_scaled_segments(device, T, E, bias, form, gain):
     """Rows whose glu leaves fp16's range (or falls to its subnormals) are stored scaled; each row group meets the bar on its
     own scale, with columns 0-15 of two experts at zero so that scaled rows hold all-zero segments too. At 2^-57 glu lies near
     2^-115: the product of the row's, the fragment's and the routing weight's powers is subnormal, the results are not."""
     K = 3
     c = rand_case(T, T, 256, 192, E, K, std=0.05, bias=bias and gain > 1)
+    assert form_of(c) == form
     for e in (0, 3):
         c["W1"][e, :16] = 0
     odd = torch.arange(1, T, 4)
@@ -99,10 +103,11 @@ def test_few_rows_scaled_segments(device, T, E, bias, gain):
     assert_within_tolerance(out[rest], ref[rest], "other rows")
 
 
-@pytest.mark.parametrize("T", [4, 24, 60], ids=["fused", "rows", "tiles"])
-def test_few_rows_nan_token(device, T):
+@pytest.mark.parametrize("T,form", [(4, "few_sum"), (24, "few_rows"), (60, "tiles")], ids=["fused", "rows", "tiles"])
+def test_few_rows_nan_token(device, T, form):
     """A token with a nan gives an all-nan row; the others, which share its experts' workgroups, stay within the bar."""
     c = rand_case(T + 1, T, 128, 192, 32, 4)
+    assert form_of(c) == form
     bad = T // 2
     c["x"][bad, 3] = float("nan")
     print(f"[few rows nan T{T}]", flush=True)
@@ -112,12 +117,13 @@ def test_few_rows_nan_token(device, T):
     assert_within_tolerance(out[keep], oracle_fp64(c, keep), "nan token")
 
 
-@pytest.mark.parametrize("T,E,act_id", [(1, 8, 0), (30, 8, 1), (40, 16, 2), (40, 16, 0)])
-def test_few_rows_nongated(device, T, E, act_id):
+@pytest.mark.parametrize("T,E,act_id,form", [(1, 8, 0, "few_sum"), (30, 8, 1, "few_rows"), (40, 16, 2, "tiles"), (40, 16, 0, "tiles")])
+def test_few_rows_nongated(device, T, E, act_id, form):
     from cernels_amd import ops
 
     g = torch.Generator().manual_seed(T + act_id)
     H, Fi, K = 192, 320, 2
+    assert packed_form(T, H, Fi, E, K, act_id) == form
     x = torch.randn(T, H, generator=g).bfloat16()
     x[T // 2] *= 1000.0  # its segments are stored scaled
     w1 = (torch.randn(E, H, Fi, generator=g) * 0.05).bfloat16()
@@ -134,13 +140,14 @@ def test_few_rows_nongated(device, T, E, act_id):
         assert_within_tolerance(out[~big], ref[~big], "other rows")
 
 
-@pytest.mark.parametrize("T", [3, 24, 60], ids=["fused", "rows", "tiles"])
-def test_few_rows_graph_replays(device, T):
+@pytest.mark.parametrize("T,form", [(3, "few_sum"), (24, "few_rows"), (60, "tiles")], ids=["fused", "rows", "tiles"])
+def test_few_rows_graph_replays(device, T, form):
     """Captured and replayed with new inputs in the same buffers, each replay equals the eager call bit for bit (nothing is
     kept between calls)."""
     from cernels_amd import ops
 
     c = rand_case(T + 2, T, 256, 192, 32, 4)
+    assert form_of(c) == form
     d = to_device(c, device)
     pk = ops.pack_experts(d["W1"], d["W2"])
     out = torch.empty_like(d["x"])
@@ -160,14 +167,16 @@ def test_few_rows_graph_replays(device, T):
         assert torch.equal(out, ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4))
 
 
-@pytest.mark.parametrize("T,K,part", [(4, 4, 1), (5, 3, 1), (24, 4, 6), (64, 4, 40)], ids=["fused", "fused-k3", "rows", "tiles"])
-def test_few_rows_do_not_depend_on_the_other_tokens(device, T, K, part):
+@pytest.mark.parametrize("T,K,part,form", [(4, 4, 1, "few_sum"), (5, 3, 1, "few_sum"), (24, 4, 6, "few_rows"), (64, 4, 40, "tiles")],
+                         ids=["fused", "fused-k3", "rows", "tiles"])
+def test_few_rows_do_not_depend_on_the_other_tokens(device, T, K, part, form):
     """A token's row is the same bit for bit whether the call holds the other tokens or not (both calls of one form), some of
     which are stored scaled, and however the experts are numbered: its slots are summed in their own order, each from a
     reduction that is cut at places that only the layer's sizes fix. F gives 13 stages, which no number of waves divides."""
     from cernels_amd import ops
 
     c = rand_case(T + K, T, 192, 832, 32, K, layout="interleaved", act="gptoss", bias=True, std=0.05)
+    assert form_of(c) == packed_form(part, 192, 832, 32, K, "gptoss") == form
     # two slots cancel exactly (equal experts, weights 1 and -1) beside small ones: what is left of a sum that was cut or ordered
     # otherwise shows in bf16
     for name in ("W1", "W2", "b1", "b2"):
