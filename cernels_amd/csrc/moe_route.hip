@@ -218,16 +218,17 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_scatter_kernel(const int
 // Count and scan fused in one workgroup: per-tile expert histograms are built in LDS with LDS
 // atomics (thread t takes pairs t, t+1024, ... so iteration i is tile i), then scanned per expert
 // over tiles and over experts exactly as in moe_route_scan_kernel. Used while the histograms fit in
-// LDS (ntiles * E <= kRtFusedCells), which saves a launch and a pass over global memory.
+// LDS (ntiles * E <= kRtFusedCells), which saves a launch and a pass over global memory. It writes no XCD split: past the
+// one-launch route ((ntiles + 16) * E > 39 Ki cells) these sizes have more than 704 experts with at most 58 rows each, where
+// the packed path takes no persistent GEMMs; a call that asks for a split takes the separate launches.
 constexpr int kRtFusedCells = 28 * 1024;
 
 __global__ __launch_bounds__(kRouteThreads) void moe_route_count_scan_kernel(
     const int32_t* __restrict__ idx, int T, int K, int E, int BM, int ntiles, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ tile_offsets, int32_t* __restrict__ tile_expert,
-    int32_t* __restrict__ meta, int32_t* __restrict__ sched, XcdSplit split) {
+    int32_t* __restrict__ meta, int32_t* __restrict__ sched) {
     __shared__ int32_t h[kRtFusedCells];  // [ntiles][E]
     __shared__ int wave_tot[kRouteWaves];
-    __shared__ int s_split[18];
     const int tid = threadIdx.x, P = T * K;  // P <= kRtFusedCells * kRtTile here, far below 2^31
     for (int i = tid; i < ntiles * E; i += kRouteThreads) h[i] = 0;
     __syncthreads();
@@ -277,7 +278,6 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_count_scan_kernel(
     const int off = block_exclusive_scan(run, wave_tot, &valid_total);
     const int nt = ceil_div(run, BM);
     const int toff = block_exclusive_scan(nt, wave_tot, &tiles_total);
-    if (split.bounds) write_xcd_split(split, BM, run, nt, off, toff, valid_total, tiles_total, s_split);
     if (e < E) {
         offsets[e] = off;
         tile_offsets[e] = toff;
@@ -479,9 +479,9 @@ hipError_t launch_route(const int32_t* idx, int T, int K, int E, int BM, int32_t
                            T * K, idx32, w32);
         idx = idx32;
     }
-    if (route_fits_count_scan(nt, E)) {
+    if (!split && route_fits_count_scan(nt, E)) {
         hipLaunchKernelGGL(moe_route_count_scan_kernel, dim3(1), dim3(kRouteThreads), 0, stream, idx, T, K, E, BM, nt,
-                           counts, offsets, tile_offsets, tile_expert, meta, sched, sp);
+                           counts, offsets, tile_offsets, tile_expert, meta, sched);
     } else {
         hipLaunchKernelGGL(moe_route_count_kernel, dim3(nt), dim3(kRtThreads), E * sizeof(int32_t), stream, idx, T, K,
                            E, counts);

@@ -89,6 +89,16 @@ def test_packed_forms_on_their_lines(L):
     assert L.cernels_moe_route_launches(4, 4, 1025) == -1
 
 
+def test_no_split_where_one_launch_counts_and_scans(L):
+    """The count + scan launch writes no per-XCD item ranges: no call whose route takes it runs GEMMs that want them."""
+    for E in (705, 768, 900, 1024):
+        for P in range(1024 * (39 * 1024 // E - 17), 28 * 1024 * 1024 // E + 2049, 512):
+            for K in (1, 8):
+                for H, F in ((64, 64), (64, 512), (512, 64), (2048, 2816)):
+                    if P % K == 0 and L.cernels_moe_route_launches(P // K, K, E) == 2:
+                        assert _native.PACKED_FORMS[L.cernels_moe_experts_packed_form(P // K, H, F, E, K, 0)] in ("items", "tiles")
+
+
 def _fake(n=0x10000):
     return ctypes.c_void_p(n)
 
