@@ -224,8 +224,9 @@ using IC = std::integral_constant<int, N>;
 // MODE/ACT/HAS_BIAS select the projection; XPF: the reduction has at least two stages, and the
 // next item's first two stages are copied and loaded during the current item's last two steps
 // (cross-item prefetch); R3: the number of stages mod 3, which sets the k-loop's empty positions;
-// PEEL (R3 == 2, at least 5 stages): the loop's last round of three steps runs after it.
-template <int MODE, int ACT, bool HAS_BIAS, bool XPF, int R3, bool PEEL>
+// PEEL (R3 == 2, at least 5 stages): the loop's last round of three steps runs after it. YLDS (GEMM2): Y rows leave through
+// LDS (y_through_lds).
+template <int MODE, int ACT, bool HAS_BIAS, bool XPF, int R3, bool PEEL, bool YLDS>
 __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams prm) {
     static_assert(XPF || R3 == 1, "without prefetch the reduction is one stage");
     static_assert(!PEEL || R3 == 2, "peeled only where no ordinary step follows the loop");
@@ -249,12 +250,9 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
     // GEMM2: power of two of each wave's weight fragment (entry t holds fragment t % 8: every table
     // thread stores one, which keeps the table store free of a branch of its own)
     __shared__ int s_wx[2][kPkBM];
-    // GEMM2: epilogue staging, per wave: one 32-row block of its fragment's Y, 96 bytes a row, from which consecutive lanes
-    // store consecutive bytes. Straight from the accumulator's lanes a store touches 64 lines of 16 bytes each, which kept an
-    // item's epilogue busy for 7 us (128 rows x 8 fragments, all CUs at once); through LDS 11 or 12 runs of up to 96 bytes, 4 us.
-    // The first projections' rows (32 and 64 bytes a fragment) stay as they are.
+    // YLDS: epilogue staging, per wave: one 32-row block of its fragment's Y, 96 bytes a row
     constexpr int kYRow = 96;
-    __shared__ __attribute__((aligned(16))) unsigned char s_out[MODE == kModePkDown ? kPkWaves : 1][32 * kYRow];
+    __shared__ __attribute__((aligned(16))) unsigned char s_out[YLDS ? kPkWaves : 1][YLDS ? 32 * kYRow : 16];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
 
@@ -807,8 +805,9 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                 // the K rows of a token from nearly exact values, at 3/4 of fp32's bytes. A lane packs its four
                 // groups of four columns (8i + c4 + jj) into 12 bytes each; exchanging groups 0, 1 of lane
                 // l + 32 for groups 2, 3 of lane l (three dwords each) leaves lane l columns 0-15 of the row
-                // and lane l + 32 columns 16-31, 48 contiguous bytes each: three 16-byte stores (aligned: H is
-                // a multiple of 64) instead of four 12-byte ones.
+                // and lane l + 32 columns 16-31, 48 contiguous bytes each: three 16-byte pieces (aligned: H is
+                // a multiple of 64). They are stored as they are, or (YLDS) put into LDS, from which consecutive
+                // lanes store consecutive bytes.
                 unsigned char* Yb = reinterpret_cast<unsigned char*>(prm.out);
                 const float wsc = __builtin_amdgcn_ldexpf(1.0f, s_wx[tb][wave]);  // the fragment's fp16 scale
 #pragma unroll
@@ -827,17 +826,21 @@ __global__ __launch_bounds__(kPkThreads, 1) void moe_gemm_packed_kernel(PkParams
                             swap_halves(q[0].d[d], q[2].d[d]);
                             swap_halves(q[1].d[d], q[3].d[d]);
                         }
-                        u32x4* o = reinterpret_cast<u32x4*>(s_out[wave] + lrow * kYRow + 48 * half);
+                        u32x4* o;
+                        if constexpr (YLDS) o = reinterpret_cast<u32x4*>(s_out[wave] + lrow * kYRow + 48 * half);
+                        else o = reinterpret_cast<u32x4*>(Yb + ((long long)s_pair[tb][row] * prm.H + 32 * fc + 16 * half) * 3);
                         o[0] = u32x4{q[0].d[0], q[0].d[1], q[0].d[2], q[2].d[0]};
                         o[1] = u32x4{q[2].d[1], q[2].d[2], q[1].d[0], q[1].d[1]};
                         o[2] = u32x4{q[1].d[2], q[3].d[0], q[3].d[1], q[3].d[2]};
                     }
+                    if constexpr (YLDS) {
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        const int c = 64 * i + lid, rr = mb * 32 + c / 6;
-                        const u32x4 v = *reinterpret_cast<const u32x4*>(s_out[wave] + 16 * c);
-                        if (rr < rows)
-                            *reinterpret_cast<u32x4*>(Yb + ((long long)s_pair[tb][rr] * prm.H + 32 * fc) * 3 + 16 * (c % 6)) = v;
+                        for (int i = 0; i < 3; ++i) {
+                            const int c = 64 * i + lid, rr = mb * 32 + c / 6;
+                            const u32x4 v = *reinterpret_cast<const u32x4*>(s_out[wave] + 16 * c);
+                            if (rr < rows)
+                                *reinterpret_cast<u32x4*>(Yb + ((long long)s_pair[tb][rr] * prm.H + 32 * fc) * 3 + 16 * (c % 6)) = v;
+                        }
                     }
                 }
             }
@@ -884,20 +887,20 @@ static int pk_grid(int max_tiles, int n_tiles) {
     return ceil_div(max(grid, 1), 8) * 8;
 }
 
-template <int MODE, int ACT, bool HAS_BIAS>
+template <int MODE, int ACT, bool HAS_BIAS, bool YLDS = false>
 static hipError_t launch_pk_t(const PkParams& prm, int max_tiles, hipStream_t s) {
     const int grid = pk_grid(max_tiles, prm.n_tiles);
     const int nst = prm.Kd / kBK;
     if (nst < 2)
-        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, false, 1, false>), dim3(grid), dim3(kPkThreads), 0, s, prm);
+        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, false, 1, false, YLDS>), dim3(grid), dim3(kPkThreads), 0, s, prm);
     else if (nst % 3 == 0)
-        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 0, false>), dim3(grid), dim3(kPkThreads), 0, s, prm);
+        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 0, false, YLDS>), dim3(grid), dim3(kPkThreads), 0, s, prm);
     else if (nst % 3 == 1)
-        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 1, false>), dim3(grid), dim3(kPkThreads), 0, s, prm);
+        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 1, false, YLDS>), dim3(grid), dim3(kPkThreads), 0, s, prm);
     else if (nst >= 5)
-        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 2, true>), dim3(grid), dim3(kPkThreads), 0, s, prm);
+        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 2, true, YLDS>), dim3(grid), dim3(kPkThreads), 0, s, prm);
     else
-        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 2, false>), dim3(grid), dim3(kPkThreads), 0, s, prm);
+        hipLaunchKernelGGL((moe_gemm_packed_kernel<MODE, ACT, HAS_BIAS, true, 2, false, YLDS>), dim3(grid), dim3(kPkThreads), 0, s, prm);
     return hipGetLastError();
 }
 
@@ -1053,6 +1056,14 @@ static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, in
     const double w1 = (double)nf1 * H, w2 = (double)nf2 * F;
     return w1 * estimate(nf1, fw1) + w2 * estimate(nf2, fw2) > 1.08 * (w1 + w2);
 }
+
+// Whether the down GEMM's Y rows leave through LDS. Straight from the accumulators a store is 64 pieces of 16 bytes, through LDS
+// 11 or 12 runs of up to 96, which the L2 takes faster where the whole chip stores at once; with few rows per item or in all
+// the LDS round trip and the longer code cost more than they save. Down GEMM, direct -> through LDS (us): 128 experts of H 2048
+// F 768, 157 rows 136.5 -> 129.7; 31 of H 2816 F 1408, 573 rows 174.0 -> 168.7; 32 of H = F = 2880, 512 rows 307.7 -> 302.0, but 84
+// rows with Zipf 1.2 skew 149.3 -> 155.3; 64 of H 1280 F 896, 79 rows with skew 57.5 -> 61.6. Over 176 shapes of 30 and more rows
+// the line at 100 rows and 20 MB of Y is 0.2% off the better of both on average, direct alone 0.8%, LDS alone 1.7%.
+static bool y_through_lds(long long P, int E, int H) { return P >= 100LL * E && 3 * P * H >= 20'000'000; }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,
                             const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
@@ -1248,7 +1259,8 @@ hipError_t launch_prefill_packed(const void* x, const void* w1p, const float* b1
     g2.bounds = cost_split ? meta + 41 : nullptr;
     g2.bias = nullptr;  // the down bias is added by the combine
     g2.tail = 0;
-    st = launch_pk_t<kModePkDown, kActSilu, false>(g2, max_tiles, s);
+    st = y_through_lds((long long)T * K, E, H) ? launch_pk_t<kModePkDown, kActSilu, false, true>(g2, max_tiles, s)
+                                               : launch_pk_t<kModePkDown, kActSilu, false>(g2, max_tiles, s);
     if (st != hipSuccess) return st;
     mark(3);
     st = launch_combine_h(reinterpret_cast<const unsigned char*>(Y), idx, static_cast<uint16_t*>(out), T, K, E, H,

@@ -184,6 +184,31 @@ def test_packed_cost_split_separate_scan(device, T, E):
     assert_reference_verify(out[rows], oracle_eager(c, rows), f"cost split route T={T}")
 
 
+@pytest.mark.parametrize("H,F", [(2112, 64), (2112, 128), (2176, 192), (2112, 256), (2112, 320)])
+def test_packed_rows_through_lds(device, H, F):
+    """From 100 rows per expert and 20 MB of down rows on, these leave the persistent down GEMM through LDS: runs of each length
+    around a 32-row block and a whole tile, one reduction length per k-loop form, invalid ids, rows stored scaled, a nan."""
+    runs = [0, 1, 31, 32, 33, 255, 256, 257, 287, 512, 513, 1100]
+    T, E, K = sum(runs) // 2, len(runs), 2
+    c = rand_case(F, T, H, F, E, K, std=0.05)
+    assert form_of(c).startswith("grouped") and T * K >= 100 * E and 3 * T * K * H >= 20_000_000
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(runs))[: T * K]
+    c["idx"] = ids[torch.randperm(T * K, generator=torch.Generator().manual_seed(F))].reshape(T, K)
+    none, big, bad = torch.arange(3, T, 97), torch.arange(5, T, 50), 8
+    c["idx"][none] = E + 1
+    c["x"][big] = (c["x"][big].float() * 3000.0).bfloat16()
+    c["x"][bad, 3] = float("nan")
+    print(f"[packed through LDS H{H} F{F}]", flush=True)
+    out = _run_packed(c, device).cpu()
+    rest = torch.ones(T, dtype=torch.bool)
+    rest[torch.cat([none, big, torch.tensor([bad])])] = False
+    big = torch.tensor([t for t in big.tolist() if t not in none.tolist()])
+    ref = oracle_fp64(c)
+    assert not out[none].float().any() and torch.isnan(out[bad].float()).all()
+    assert_within_tolerance(out[big], ref[big], "scaled rows")
+    assert_within_tolerance(out[rest], ref[rest], "other rows")
+
+
 @pytest.mark.parametrize("name", GOLDEN_NAMES)
 def test_packed_golden(device, name):
     t, meta = load_golden(name)
