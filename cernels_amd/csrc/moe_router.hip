@@ -14,7 +14,7 @@
 // The logits GEMM ([T,H] x [E,H]ᵀ) runs on MFMA (bf16, fp32 accumulation).
 //   E <= 64  (gpt-oss): one kernel. A workgroup owns 16 tokens and all experts; its waves split the
 //            reduction, their partial sums meet in LDS (fixed order), and the same workgroup selects
-//            for its 16 tokens.
+//            for its 16 tokens. Many tokens with wide rows: 32 tokens on four waves and an LDS stage ring.
 //   E > 64   (qwen3-next): up to 256 tokens the same split over workgroups of 16 tokens x 16 experts,
 //            above that a 128-token x 64-expert tiled GEMM from LDS (stages of 64 k-columns copied
 //            HBM -> LDS directly into a ring, one wait and one barrier per stage), writes the bf16
@@ -319,6 +319,71 @@ __global__ __launch_bounds__(NE <= 2 ? 1024 : 512) void moe_router_fused_kernel(
     }
 }
 
+// ---- E <= 64, many tokens: the same on 32 tokens per workgroup, four waves and an LDS stage ring (each stage's four k-steps one
+// per wave), which reads W half as often and holds two workgroups per CU (one above 32 rows of W); grid = ceil(T / 32).
+// A 16-token workgroup of 16 waves has a CU to itself, so the split kernel goes up in steps of 4096 tokens. us per launch, split
+// -> ring: H = 2880 E = 32 T = 4096 13.5 -> 17.7, 5120 22.7 -> 17.7, 16384 43.0 -> 26.4; H = 4096 E = 64 T = 5120 43.6 -> 29.5; H =
+// 2048 E = 64 T = 8192 24.5 -> 20.0, 10240 34.0 -> 37.3, 16384 45.0 -> 38.7; H = 1024 E = 32 T = 8192 9.1 -> 11.7, 16384 17.4 -> 14.7; E =
+// 64 24.7 -> 27.9; H = 2880 E = 16 T = 8208 23.1 -> 18.0; H = 4096 E = 8 T = 32768 69.3 -> 73.1.
+static bool ring_pays(int T, int H, int ER) {
+    if (T <= 4096 || ER <= 8) return false;
+    if (T <= 8192) return ER > 16 && H >= 2048;
+    return H >= (ER > 32 ? 1536 : ER > 16 ? 1024 : 2048);
+}
+
+constexpr int kRtrRingStages = 8;
+template <int MODE, int NT>  // NT = expert blocks of 32 (1 or 2)
+__global__ __launch_bounds__(kRtrThreads) void moe_router_ring_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int T, int H,
+    int E, int K, int renorm, int S, int32_t* __restrict__ idx_out, float* __restrict__ w_out,
+    uint16_t* __restrict__ logits_out) {
+    constexpr int TM = 32, EN = 32 * NT, ROWS = TM + EN;
+    const int ER = E + (S > 0);  // rows of W and of a logits row: the experts, then the shared-expert gate
+    constexpr int kRing = kRtrRingStages * ROWS * kBK * 2;
+    static_assert(4 * TM * EN * 4 <= kRing, "partial sums reuse the stage ring");
+    __shared__ __align__(1024) char ring[kRing];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int t0 = blockIdx.x * TM;
+
+    f32x16 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+    // wave q takes k-step q of every stage; a k-step at or beyond H is skipped
+    stage_pipeline<kRtrRingStages, ROWS, TM, 4>(ring, x, w, t0, 0, T, ER, H, wave, lane, [&](const char* sb, int st) {
+        if (st * kBK + 16 * wave < H) {
+            const bf16x8 a = lds_frag(sb, 0, wave, lane);
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, lds_frag(sb, TM + 32 * n, wave, lane), acc[n], 0, 0, 0);
+        }
+    });
+    // partial sums of the four waves: element r is token 8(r/4) + 4(lane/32) + r%4, expert 32 n + lane % 32
+    float(*part)[TM][EN] = reinterpret_cast<float(*)[TM][EN]>(ring);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[wave][8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)][32 * n + (lane & 31)] = acc[n][r];
+    __syncthreads();
+    // logit = bf16(((p0 + p1) + p2) + p3 + b); kept in slice 0 and written to logits_out
+    for (int c = tid; c < TM * EN; c += kRtrThreads) {
+        const int tl = c / EN, e = c % EN;
+        if (e >= ER) continue;
+        const float b = bias != nullptr ? bf16_bits_to_f32(bias[e]) : 0.f;
+        const float v = round_bf16(((part[0][tl][e] + part[1][tl][e]) + part[2][tl][e]) + part[3][tl][e] + b);
+        part[0][tl][e] = v;
+        if (t0 + tl < T) logits_out[(long long)(t0 + tl) * ER + e] = f32_to_bf16_bits(v);
+    }
+    __syncthreads();
+    for (int tl = wave; tl < TM; tl += 4) {
+        if (t0 + tl >= T) break;  // uniform
+        float v[1] = {lane < E ? part[0][tl][min(lane, EN - 1)] : -INFINITY};
+        select_token<MODE, 1>(v, lane, t0 + tl, E, K, renorm, S, S > 0 ? part[0][tl][E] : 0.f, idx_out, w_out);
+    }
+}
+
 // ---- E > 64, few tokens: logits of 16 tokens x 16 experts per workgroup, the shared-expert gate's row among them;
 // grid = (ceil(ER / 16), ceil(T / 16)). Up to kRtrSplitMaxT tokens: H=2048 E=512 T=1 4.6 us against 19.3 of the tiled
 // kernel (whose few workgroups walk 32 stages one after the other), T=256 12.7 / 15.6, T=512 20.2 / 15.6.
@@ -433,6 +498,14 @@ template <int MODE>
 static hipError_t launch_router_m(const uint16_t* x, const uint16_t* w, const uint16_t* bias, int T, int H, int E,
                                   int K, int renorm, int S, int32_t* idx, float* wt, uint16_t* logits, hipStream_t s) {
     const int ER = E + (S > 0);
+    if (ER <= kRtrFusedMaxE && ring_pays(T, H, ER)) {
+        const dim3 grid(ceil_div(T, 32)), block(kRtrThreads);
+        if (ER <= 32)
+            hipLaunchKernelGGL((moe_router_ring_kernel<MODE, 1>), grid, block, 0, s, x, w, bias, T, H, E, K, renorm, S, idx, wt, logits);
+        else
+            hipLaunchKernelGGL((moe_router_ring_kernel<MODE, 2>), grid, block, 0, s, x, w, bias, T, H, E, K, renorm, S, idx, wt, logits);
+        return hipGetLastError();
+    }
     if (ER <= kRtrFusedMaxE) {
         const dim3 grid(ceil_div(T, 16));
 #define CMOE_RTF(NE) \

@@ -1,4 +1,4 @@
-"""Router sizes at the edges of its kernels' tiles (16 tokens x 16 experts split over waves, 128 x 64 tiled), with and
+"""Router sizes at the edges of its kernels' tiles (16 tokens x 16 experts split over waves, 32 tokens on a stage ring, 128 x 64 tiled), with and
 without the shared-expert gate's row: the bounds of test_gpu_router.py against the CPU oracle."""
 
 from __future__ import annotations
@@ -20,6 +20,12 @@ CASES = [
     (33, 528, 32, 5, O.ROUTER_SOFTMAX_TOPK, 2, True),    # 33 rows
     (40, 320, 63, 6, O.ROUTER_SOFTMAX_TOPK, 1, False),   # 64 rows: the largest fused
     (31, 176, 64, 6, O.ROUTER_SOFTMAX_TOPK, 1, False),   # 65 rows: logits, then selection
+    (4096, 2064, 17, 3, O.ROUTER_TOPK_SOFTMAX, 0, True),  # 16 tokens per workgroup: the last of this width
+    (4097, 2064, 17, 3, O.ROUTER_TOPK_SOFTMAX, 0, True),  # the stage ring: one token in the last workgroup, a quarter stage
+    (4130, 2048, 32, 4, O.ROUTER_SOFTMAX_TOPK, 1, True),  # 33 rows with the gate
+    (8193, 1040, 31, 4, O.ROUTER_SOFTMAX_TOPK, 1, False),  # 32 rows with the gate
+    (8223, 2080, 9, 2, O.ROUTER_TOPK_SOFTMAX, 0, False),
+    (8200, 1552, 64, 6, O.ROUTER_SOFTMAX_TOPK, 0, True),
     (256, 2048, 127, 8, O.ROUTER_SOFTMAX_TOPK, 1, True),  # the split kernel's last
     (257, 2048, 127, 8, O.ROUTER_SOFTMAX_TOPK, 1, True),  # the tiled kernel's first
     (1000, 592, 513, 10, O.ROUTER_TOPK_SOFTMAX, 0, True),
