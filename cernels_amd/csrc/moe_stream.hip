@@ -8,8 +8,8 @@
 // straight to registers, and no wave waits for another until the four partial sums meet in LDS at the end. Four such
 // workgroups per CU keep 128 KB of weights in flight (a plain read of 126 MB reaches 5.9 TB/s with 64 KB in flight on
 // 176 and more CUs, 4.2 TB/s on 88). What bounds it: HBM, 5.2-5.8 TB/s of weights in a launch of 130 MB and more.
-// Two, eight or five workgroups' worth of waves (64, 512 threads; 102 registers, which spill) measured 0-5%, 2-25% and
-// 35% slower.
+// Tried and slower: workgroups of one wave 0-5%, of eight waves 2-25%, five of four waves per CU (at most 102 registers,
+// which spill) 35%.
 //
 // Two forms share the first projection:
 //   few    (T <= 32 tokens, at most 512 pairs): no route. Each workgroup finds its expert and that expert's tokens from
@@ -46,6 +46,8 @@ constexpr int kFdMaxPairs = 16;    // above: rows per pair and the combine. gpt-
                                    // pairs 50.6 / 46.6 + 5.2; 33 pairs of 30B-A3B-like experts 23.1 / 15.6 + 4.0: H / 16
                                    // workgroups stream less than the whole chip, which the launch saved pays for up to here
 constexpr int kFewMaxTopk = 64;    // few_select's division by K
+// few_select: p / K as a product holds while the error p / 65536 stays below 1 / K; bit 14 of few_row lies above every pair
+static_assert(kFewMaxPairs * kFewMaxTopk <= 65536 && kFewMaxPairs <= 0x4000 && kFewMaxTokens <= kWave);
 constexpr int kTilesMaxTokens = 512;  // bounds the M-tiles of one popular expert, each of which streams its weights
 constexpr int kTilesMaxRows = 8;      // rows per expert on average
 
@@ -228,10 +230,8 @@ __device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int t
             ev[c] = (unsigned)v < (unsigned)E ? v : -1;
         }
     }
-    if (lane < kFewMaxExperts / 32) {
-        bits[lane] = 0u;
-        tokp[lane] = INT_MAX;
-    }
+    if (lane < kFewMaxExperts / 32) bits[lane] = 0u;
+    if (lane < kFewMaxTokens) tokp[lane] = INT_MAX;
 #pragma unroll
     for (int c = 0; c < kFewMaxPairs / kWave; ++c)
         if (ev[c] >= 0) atomicOr(&bits[ev[c] >> 5], 1u << (ev[c] & 31));
@@ -250,7 +250,7 @@ __device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int t
     const uint64_t hb = __ballot(holder);
     if (hb == 0ull) return -1;
     const int e = __builtin_amdgcn_readlane(eh, __ffsll((unsigned long long)hb) - 1);
-    const int magic = 65536 / K + 1;  // p / K for p < 512, K <= 64: p * magic >> 16 (error p / 65536 < 1 / K)
+    const int magic = 65536 / K + 1;  // p / K = p * magic >> 16
 #pragma unroll
     for (int c = 0; c < kFewMaxPairs / kWave; ++c)
         if (ev[c] == e) {
@@ -865,10 +865,11 @@ bool tiles_supported(int T, int K, int E) {
     return T <= kTilesMaxTokens && (long long)T * K <= (long long)kTilesMaxRows * E;
 }
 
-// Whether a call takes the few form: one 32-row block of tokens, and lists that fit the down kernel's LDS.
-bool few_supported(int T, int K, int E) {
+// Whether a call takes the few form: one 32-row block of tokens, experts that fit few_select's bitmap, lists that fit the down
+// kernel's LDS, and glu (all of it one buffer there; one expert's rows elsewhere) within 32-bit offsets.
+bool few_supported(int T, int K, int E, int F) {
     const long long P = (long long)T * K;
-    return T <= kFewMaxTokens && K <= kFewMaxTopk && P <= kFewMaxPairs;
+    return T <= kFewMaxTokens && K <= kFewMaxTopk && E <= kFewMaxExperts && P <= kFewMaxPairs && P * F * 2 < (1LL << 31);
 }
 
 // Whether the few form's down kernel sums over the slots itself (kFdMaxPairs).

@@ -79,6 +79,8 @@ def test_packed_forms_on_their_lines(L):
         ((32, 64, 64, 512, 17), "tiles"), ((33, 64, 64, 512, 16), "tiles"), ((8, 64, 64, 8, 64), "few_rows"),
         ((1, 64, 64, 1024, 64), "few_rows"), ((1, 64, 64, 1024, 65), "tiles"), ((512, 64, 64, 64, 1), "tiles"),
         ((513, 64, 64, 65, 1), "grouped"), ((64, 64, 64, 32, 4), "tiles"), ((65, 64, 64, 32, 4), "grouped"),
+        # all of glu is one buffer in the few-token kernels: 32-bit offsets
+        ((32, 64, 2**21 - 64, 8, 16), "few_rows"), ((32, 64, 2**21, 8, 16), "grouped_split"),
         ((1440, 2048, 768, 128, 8), "items"), ((1441, 2048, 768, 128, 8), "grouped"), ((4096, 2880, 2880, 32, 4), "grouped_split"),
     ]
     for sizes, form in lines:
