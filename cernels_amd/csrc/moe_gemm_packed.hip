@@ -1069,7 +1069,7 @@ hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t
                             const int32_t* sync, const int8_t* psig, const float* b2, const void* route_w,
                             hipStream_t s, int types = 0);
 
-bool few_supported(int T, int K, int E, int F);
+bool few_supported(int T, int K, int E, int nf1);
 bool few_sums(int T, int K);
 bool tiles_supported(int T, int K, int E);
 hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
@@ -1116,7 +1116,7 @@ static PackedPlan packed_plan(int T, int H, int F, int E, int K, int act, int ma
     PackedPlan pl{};
     pl.nf1 = act_is_gated(act) ? F / 16 : F / 32;
     pl.nf2 = H / 32;
-    if (few_supported(T, K, E, F)) {
+    if (few_supported(T, K, E, pl.nf1)) {
         pl.form = few_sums(T, K) ? kFormFewSum : kFormFewRows;
         return pl;
     }

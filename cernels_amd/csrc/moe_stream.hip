@@ -12,7 +12,7 @@
 // which spill) 35%.
 //
 // Two forms share the first projection:
-//   few    (T <= 32 tokens, at most 512 pairs): no route. Each workgroup finds its expert and that expert's tokens from
+//   few    (T <= 32 tokens, at most 512 pairs, see few_supported): no route. Each workgroup finds its expert and that expert's tokens from
 //          the indices by itself (rows are tokens). Up to 16 pairs the down kernel sums every expert's contribution to
 //          its 16 output columns in registers (two launches), above that it writes a row per pair and the combine sums
 //          them (three; the general path takes five).
@@ -20,8 +20,8 @@
 //          glu fixup and the combine as on the general path.
 // Measured, whole op in us, general path -> here (seeded routing, weights of three layers in turn): gpt-oss shapes (H = F =
 // 2880, E = 32, k = 4) T=1 85 -> 43, T=8 234 -> 195, T=32 299 -> 273, T=48 311 -> 297 (tiles); H=2048 F=512 E=513 k=11
-// T=3 90 -> 58, T=28 291 -> 257, T=128 580 -> 521, T=400 635 -> 599 (tiles); H=2048 F=768 E=128 k=8 T=1 82 -> 34,
-// T=32 221 -> 189, T=65 239 -> 221, T=128 245 -> 237 (tiles). Above 8 rows per expert the tiles form loses (12.5 rows:
+// T=3 90 -> 58, T=28 293 -> 256 (tiles), T=128 580 -> 521, T=400 635 -> 599 (tiles); H=2048 F=768 E=128 k=8 T=1 82 -> 34,
+// T=32 207 -> 183 (tiles), T=65 239 -> 221, T=128 245 -> 237 (tiles). Above 8 rows per expert the tiles form loses (12.5 rows:
 // 245 -> 252): each wave fetches every row's 128-byte lines itself, where the general path shares them through LDS.
 // Precision is the general path's: fp32 accumulation, glu in fp16 segments scaled where needed (moe_packed.h), fp16
 // weights scaled per fragment, the routing weight and the sum over slots in fp32, one rounding to bf16.
@@ -866,10 +866,18 @@ bool tiles_supported(int T, int K, int E) {
 }
 
 // Whether a call takes the few form: one 32-row block of tokens, experts that fit few_select's bitmap, lists that fit the down
-// kernel's LDS, and glu (all of it one buffer there; one expert's rows elsewhere) within 32-bit offsets.
-bool few_supported(int T, int K, int E, int F) {
+// kernel's LDS. Above kFdMaxPairs pairs also a bound on the ids that the first projection reads: each of its workgroups (nf1
+// fragments of each chosen expert) goes through all of them, where the other forms sort them once. Against the tiles form,
+// which takes most of these calls instead, the line is at 2^20 ids, against the grouped GEMMs at 600000. Whole op, few ->
+// tiles (us): 22 tokens of 428 experts of H 192 F 1664, top-21 (20 M ids) 216 -> 147; 28 of 76 of H 576 F 3968, top-14 (7.4 M)
+// 257 -> 190; 32 of 128 of H 2048 F 768, top-8 (1.6 M) 177 -> 183; 32 of 32 of H = F = 2880, top-4 (0.74 M) 276 -> 282; few -> grouped:
+// 30 tokens of 25 experts of H 1088 F 2112, top-16 (1.6 M) 109 -> 89; 32 of 14 of H 2816 F 1792, top-12 (0.60 M) 119 -> 101; 20 of 12
+// of H 3648 F 3776, top-9 (0.51 M) 199 -> 200. Over 1150 shapes of up to 32 tokens the two lines are 0.4% off the better form on
+// average, no line 2.5%. (So all of glu, one buffer in the down kernels, has at most 2^25 bytes.)
+bool few_supported(int T, int K, int E, int nf1) {
     const long long P = (long long)T * K;
-    return T <= kFewMaxTokens && K <= kFewMaxTopk && E <= kFewMaxExperts && P <= kFewMaxPairs && P * F * 2 < (1LL << 31);
+    if (T > kFewMaxTokens || K > kFewMaxTopk || E > kFewMaxExperts || P > kFewMaxPairs) return false;
+    return P <= kFdMaxPairs || nf1 * std::min<long long>(P, E) * P <= (tiles_supported(T, K, E) ? 1 << 20 : 600000);
 }
 
 // Whether the few form's down kernel sums over the slots itself (kFdMaxPairs).

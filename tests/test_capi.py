@@ -79,8 +79,8 @@ def test_packed_forms_on_their_lines(L):
         ((32, 64, 64, 512, 17), "tiles"), ((33, 64, 64, 512, 16), "tiles"), ((8, 64, 64, 8, 64), "few_rows"),
         ((1, 64, 64, 1024, 64), "few_rows"), ((1, 64, 64, 1024, 65), "tiles"), ((512, 64, 64, 64, 1), "tiles"),
         ((513, 64, 64, 65, 1), "grouped"), ((64, 64, 64, 32, 4), "tiles"), ((65, 64, 64, 32, 4), "grouped"),
-        # all of glu is one buffer in the few-token kernels: 32-bit offsets
-        ((32, 64, 2**21 - 64, 8, 16), "few_rows"), ((32, 64, 2**21, 8, 16), "grouped_split"),
+        ((32, 64, 128, 512, 16), "tiles"), ((32, 64, 576, 32, 16), "few_rows"), ((32, 64, 640, 32, 16), "grouped"),
+        ((32, 2880, 2880, 32, 4), "few_rows"), ((28, 576, 3968, 76, 14), "tiles"), ((1, 64, 2**20, 16, 16), "few_sum"),
         ((1440, 2048, 768, 128, 8), "items"), ((1441, 2048, 768, 128, 8), "grouped"), ((4096, 2880, 2880, 32, 4), "grouped_split"),
     ]
     for sizes, form in lines:

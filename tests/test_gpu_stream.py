@@ -1,7 +1,7 @@
 """Few rows per expert on packed weights: the streaming forms of moe_experts_packed, against the fp64 oracle.
 
 Up to 32 tokens and 512 pairs the kernels route by themselves (up to 16 pairs with the sum over slots in the down kernel,
-above that with a row per pair); up to 512 tokens with at most 8 rows per expert on average they walk the route's list in
+above that with a row per pair) where the ids that their workgroups read stay few; up to 512 tokens with at most 8 rows per expert on average they walk the route's list in
 M-tiles of 32 rows. Cases sit on both sides of each line, at the smallest and largest sizes, with ids that are out of range
 or name an expert twice, one expert taking every token, and glu segments stored scaled.
 """
@@ -40,7 +40,10 @@ CASES = [
     (7, 128, 64, 12, 2, SILU, "invalid", "few_sum"),
     (3, 128, 64, 4, 2, GPT, "none", "few_sum"),  # no valid id at all: zeros
     (20, 128, 64, 4, 2, SILU, "none", "few_rows"),
-    (32, 128, 128, 512, 16, SILU, "plain", "few_rows"),  # 512 pairs
+    (32, 128, 64, 512, 16, SILU, "plain", "few_rows"),  # 512 pairs, 2^20 ids read by the first projection's workgroups
+    (32, 128, 128, 512, 16, SILU, "plain", "tiles"),  # more ids: tiles, with few tokens
+    (32, 128, 576, 32, 16, GPT, "twice", "few_rows"),  # more than 8 rows per expert: 600000 ids
+    (32, 128, 640, 32, 16, GPT, "twice", "grouped"),  # above
     (32, 128, 128, 512, 17, SILU, "plain", "tiles"),  # 544: the route's list (tiles)
     (32, 1088, 448, 64, 8, GPT, "same", "few_rows"),  # every token on the same experts
     (33, 128, 192, 64, 4, SILU, "invalid", "tiles"),  # 33 tokens: tiles
