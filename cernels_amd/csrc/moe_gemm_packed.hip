@@ -1070,7 +1070,7 @@ hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t
                             hipStream_t s, int types = 0);
 
 bool few_supported(int T, int K, int E, int nf1);
-bool few_sums(int T, int K);
+bool few_sums(int T, int K, int E, int H, int F);
 bool tiles_supported(int T, int K, int E);
 hipError_t launch_few(const void* x, const void* w1p, const float* b1, const void* w2p, const float* b2, const int32_t* idx,
                       const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
@@ -1117,7 +1117,7 @@ static PackedPlan packed_plan(int T, int H, int F, int E, int K, int act, int ma
     pl.nf1 = act_is_gated(act) ? F / 16 : F / 32;
     pl.nf2 = H / 32;
     if (few_supported(T, K, E, pl.nf1)) {
-        pl.form = few_sums(T, K) ? kFormFewSum : kFormFewRows;
+        pl.form = few_sums(T, K, E, H, F) ? kFormFewSum : kFormFewRows;
         return pl;
     }
     if (tiles_supported(T, K, E)) {

@@ -13,8 +13,8 @@
 //
 // Two forms share the first projection:
 //   few    (T <= 32 tokens, at most 512 pairs, see few_supported): no route. Each workgroup finds its expert and that expert's tokens from
-//          the indices by itself (rows are tokens). Up to 16 pairs the down kernel sums every expert's contribution to
-//          its 16 output columns in registers (two launches), above that it writes a row per pair and the combine sums
+//          the indices by itself (rows are tokens). Up to 16 pairs the down kernel may sum every expert's contribution to
+//          its 16 output columns (two launches, few_sums), else it writes a row per pair and the combine sums
 //          them (three; the general path takes five).
 //   tiles  (up to 512 tokens, at most 8 rows per expert on average): the route's list with M-tiles of 32 rows, then the
 //          glu fixup and the combine as on the general path.
@@ -42,9 +42,7 @@ constexpr int kFewMaxPairs = 512;
 constexpr int kFewMaxExperts = 1024;  // bitmap of 32 words
 constexpr int kFdWaves = 8, kFdThreads = kFdWaves * kWave;  // few: down workgroup with the sum over slots
 constexpr int kFdStages = 4;
-constexpr int kFdMaxPairs = 16;    // above: rows per pair and the combine. gpt-oss 4 pairs 16.7 us against 15.4 + 4.6, 16
-                                   // pairs 50.6 / 46.6 + 5.2; 33 pairs of 30B-A3B-like experts 23.1 / 15.6 + 4.0: H / 16
-                                   // workgroups stream less than the whole chip, which the launch saved pays for up to here
+constexpr int kFdMaxPairs = 16;    // above: rows per pair and the combine (few_sums)
 constexpr int kFewMaxTopk = 64;    // few_select's division by K
 // few_select: p / K as a product holds while the error p / 65536 stays below 1 / K; bit 14 of few_row lies above every pair
 static_assert(kFewMaxPairs * kFewMaxTopk <= 65536 && kFewMaxPairs <= 0x4000 && kFewMaxTokens <= kWave);
@@ -880,8 +878,16 @@ bool few_supported(int T, int K, int E, int nf1) {
     return P <= kFdMaxPairs || nf1 * std::min<long long>(P, E) * P <= (tiles_supported(T, K, E) ? 1 << 20 : 600000);
 }
 
-// Whether the few form's down kernel sums over the slots itself (kFdMaxPairs).
-bool few_sums(int T, int K) { return (long long)T * K <= kFdMaxPairs; }
+// Whether the few form's down kernel sums over the slots itself, which saves the combine's launch. Its H / 16 workgroups walk all
+// chosen experts one after the other, so with short rows of the result they stream less than the whole chip, for a time that
+// goes with experts x F. Down kernel with the sum against rows and combine (us): H = F = 2880, 4 pairs 16.7 / 15.4 + 4.6, 16 pairs 50.6 /
+// 46.6 + 5.2; 33 pairs of H 2048 F 768 23.1 / 15.6 + 4.0. Whole op, sum / rows: 12 experts of H 3072 F 2304 118 / 120; 4 of H 1088 F 7488
+// 46 / 34; 15 of H 192 F 128 15.4 / 13.1; 3 of H 512 F 1280 13.4 / 17.0; one of H 128 F 8960 14.1 / 19.9. Over 400 shapes of up to
+// 16 pairs this line is 1.3% off the better of both, the sum alone 20%, rows alone 2.6%.
+bool few_sums(int T, int K, int E, int H, int F) {
+    const long long P = (long long)T * K, um = std::min<long long>(P, E);
+    return P <= kFdMaxPairs && (H >= 2048 || um <= 2 || um * F <= 2000);
+}
 
 // Parts of the lists that the few form passes from its first to its second launch, at `lists`: um experts, um x T glu rows,
 // um x nf1 flags, each to a multiple of 16 bytes.
@@ -945,7 +951,7 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
     q.NF = H / 32;
     q.KS = F / 16;
     q.out = static_cast<uint16_t*>(out);
-    if (!few_sums(T, K)) {
+    if (!few_sums(T, K, E, H, F)) {
         q.Y = Y;
         hipLaunchKernelGGL(moe_few_down_rows_kernel, dim3(q.NF, um), dim3(kStThreads), 0, s, q);
         st = hipGetLastError();

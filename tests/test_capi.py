@@ -80,7 +80,8 @@ def test_packed_forms_on_their_lines(L):
         ((1, 64, 64, 1024, 64), "few_rows"), ((1, 64, 64, 1024, 65), "tiles"), ((512, 64, 64, 64, 1), "tiles"),
         ((513, 64, 64, 65, 1), "grouped"), ((64, 64, 64, 32, 4), "tiles"), ((65, 64, 64, 32, 4), "grouped"),
         ((32, 64, 128, 512, 16), "tiles"), ((32, 64, 576, 32, 16), "few_rows"), ((32, 64, 640, 32, 16), "grouped"),
-        ((32, 2880, 2880, 32, 4), "few_rows"), ((28, 576, 3968, 76, 14), "tiles"), ((1, 64, 2**20, 16, 16), "few_sum"),
+        ((32, 2880, 2880, 32, 4), "few_rows"), ((28, 576, 3968, 76, 14), "tiles"), ((1, 2048, 2**16, 16, 16), "few_sum"),
+        ((1, 1984, 128, 15, 16), "few_sum"), ((1, 1984, 128, 16, 16), "few_rows"), ((4, 64, 8960, 2, 4), "few_sum"),
         ((1440, 2048, 768, 128, 8), "items"), ((1441, 2048, 768, 128, 8), "grouped"), ((4096, 2880, 2880, 32, 4), "grouped_split"),
     ]
     for sizes, form in lines:
