@@ -999,6 +999,7 @@ __global__ __launch_bounds__(256) void moe_glu_fixup_kernel(uint16_t* __restrict
 }
 
 int packed_tile_m() { return kPkBM; }
+int mid_tile_m();
 
 // Fragments per item. Items of one projection all have the same cost, so a launch takes
 // ceil(items / CUs) rounds; narrower items (fewer active waves) cut the last, partly empty round at
@@ -1026,11 +1027,11 @@ static int pick_fw(long long P, int E, int NF, int Kd, int cus) {
     return best_w;
 }
 
-// M-tiles of kPkBM rows that an expert of r rows on average has on average: rows per expert spread as sqrt(r) under
-// routing without skew, so next to a multiple of kPkBM part of the experts need one tile more.
-static double expected_tiles(double r) {
+// M-tiles of bm rows that an expert of r rows on average has on average: rows per expert spread as sqrt(r) under
+// routing without skew, so next to a multiple of bm part of the experts need one tile more.
+static double expected_tiles(double r, int bm) {
     double t = 1;
-    for (int j = 1; j * kPkBM < r + 4 * std::sqrt(r); ++j) t += 0.5 * std::erfc((j * kPkBM + 0.5 - r) / std::sqrt(2 * r));
+    for (int j = 1; j * bm < r + 4 * std::sqrt(r); ++j) t += 0.5 * std::erfc((j * bm + 0.5 - r) / std::sqrt(2 * r));
     return t;
 }
 
@@ -1040,21 +1041,31 @@ static double expected_tiles(double r) {
 //   persistent -> items (us): 128 experts of H 2048 F 768, 12.5 / 31 / 87 rows 225 -> 212, 239 -> 230, 271 -> 262; 513 experts
 //   of F 512, 43 rows 663 -> 662, 88 rows 763 -> 723 and with Zipf 1.2 skew 540 -> 473. At 112 rows (289 -> 308) and with
 //   fewer items (8 experts of F 5632, 25 rows: 95 -> 107) they lose.
-// - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM's
-//   estimate is 1.2 for items of up to 4 fragments (half of a workgroup's waves idle), else 0.95 ceil(R) / R for R rounds, and
-//   1 for at most one round (nothing to split); the mean, weighted by work, has to pass 1.08. Over 150 shapes of 8 to 513
-//   experts the mid items measured 1.00 to 1.30 times as fast wherever it does (8 experts of F 5632, 1024 rows, non-gated: 533
-//   -> 421; 64 of H 1280 F 896, 384 rows: 259 -> 230; 21 of H 1920 F 1024, 325 rows: 145 -> 108), and 0.78 to 1.12 times
-//   where it does not (32 of H = F = 2880, 188 rows: 397 -> 435, 1024 rows: 1502 -> 1605).
+//   Over 858 shapes of 8 to 90 rows, 278 of which take it, the items are 1.07 times as fast on average and up to 4% slower in 5.
+// - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM on R
+//   rounds of persistent items is estimated at 0.95 ceil(R) / R, of up to 4 fragments (half of a workgroup's waves idle) at up to
+//   1.3, and at 1 for about one round (nothing to split); on Q rounds of two items per CU at 1, and a tenth of what the last
+//   round leaves idle. The ratio of the means, weighted by work, has to pass 1.06, and no GEMM may leave most CUs without an item
+//   that narrower persistent items fill. Measured over 992 shapes of 4 to 1024 experts, with and without skew: the 422 that take it are
+//   1.13 times as fast on average (8 experts of F 5632, 1024 rows, non-gated: 533 -> 421 us; 64 of H 1280 F 896, 384 rows: 259 -> 230)
+//   and 8 of them more than 1.5% slower (10 of H = F = 2688, 322 rows: 189 -> 209; 26 of H = F = 1856, 120 rows, non-gated: 148 -> 160; the
+//   others up to 5%); where it does not take them items are 0.75 to 1.73 times as fast (32 of H = F = 2880, 188 rows: 397 -> 435).
 static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, int fw1, int fw2, int cus) {
     const double r = (double)P / E;
     if (r <= 90) return (long long)E * ceil_div(std::min(nf1, nf2), kPkWaves) >= 2LL * cus;
-    auto estimate = [&](int nf, int fw) {
-        const double R = E * expected_tiles(r) * ceil_div(nf, fw) / cus;
-        return R <= 1 ? 1.0 : fw <= 4 ? 1.2 : 0.95 * std::ceil(R - 0.02) / R;
+    const double tiles = E * expected_tiles(r, kPkBM) / cus, items = E * expected_tiles(r, mid_tile_m()) / (2.0 * cus);
+    double persistent = 0, mid = 0;
+    bool fills = true;
+    auto add = [&](int nf, int fw, double work) {
+        const double R = tiles * ceil_div(nf, fw), Q = items * ceil_div(nf, kPkWaves);
+        const double rounds = std::ceil(R - 0.02) / R;
+        persistent += work * (R <= 1.05 ? 1.0 : fw <= 4 ? std::min(1.3, 1.15 * rounds) : 0.95 * rounds);
+        mid += work * (Q > 1 ? 1 + 0.1 * std::max(0.0, std::ceil(Q - 0.02) - Q) / Q : 1.0);
+        fills = fills && 2 * Q >= 0.6 * std::min(R, 1.0);
     };
-    const double w1 = (double)nf1 * H, w2 = (double)nf2 * F;
-    return w1 * estimate(nf1, fw1) + w2 * estimate(nf2, fw2) > 1.08 * (w1 + w2);
+    add(nf1, fw1, (double)nf1 * H);
+    add(nf2, fw2, (double)nf2 * F);
+    return fills && persistent > 1.06 * mid;
 }
 
 // Whether the down GEMM's Y rows leave through LDS. Straight from the accumulators a store is 64 pieces of 16 bytes, through LDS
@@ -1076,7 +1087,6 @@ hipError_t launch_few(const void* x, const void* w1p, const float* b1, const voi
                       const void* route_w, int types, int T, int H, int F, int E, int K, int bias_interleaved, int act, void* out,
                       uint16_t* glu, int8_t* gexp, unsigned char* Y, unsigned char* lists, hipStream_t s, hipEvent_t* ev);
 int stream_tile_m();
-int mid_tile_m();
 hipError_t launch_stream_gemm1(const void* x, const void* w1p, const float* b1, int T, int H, int F, int E, int K,
                                int bias_interleaved, int act, const int32_t* offsets, const int32_t* tile_offsets,
                                const int32_t* meta, const int32_t* sorted_pairs, const int32_t* tile_expert, int max_tiles,
