@@ -72,7 +72,8 @@ def _usable(t, dtype, device_index: int, shape) -> bool:
 
 def _dims(x, gate_up_proj, down_proj, indices, weights, topk, layout, gate_up_bias, down_bias):
     """(T, H, F, E) of inputs that hold to the contract, else None: the caller then runs _check_inputs, which says what is
-    wrong. indices and weights may have any type that the native entries read."""
+    wrong. indices and weights may have any type that the native entries read. One expression without messages, since it is on
+    every short call's path; a condition added to _check_inputs belongs here too."""
     try:
         T, H = x.shape
         E, n1, n2 = gate_up_proj.shape
@@ -285,7 +286,8 @@ def pack_experts(gate_up_proj, down_proj, *, layout=LAYOUT_CONCAT, act=ACT_SILU,
 
 
 def _packed_ok(x, packed, dev: int) -> bool:
-    """Whether ``packed`` holds the buffers of its own sizes on x's device: the kernels read packed_weight_bytes of each."""
+    """Whether ``packed`` holds the buffers of its own sizes on x's device: the kernels read packed_weight_bytes of each. What it
+    refuses goes to moe_experts_packed, which says what is wrong; a condition added there belongs here too."""
     try:
         H, F, E = packed.H, packed.F, packed.E
         gu_which = _native.GATE_UP if packed.act in (ACT_SILU, ACT_GPTOSS) else _native.UP
@@ -617,6 +619,7 @@ def megablocks_moe(x, w1, w2, indices, weights, topk, act_id):
 
 __all__ = [
     "moe_experts", "route", "decode_supported", "PackedExperts", "pack_weights", "pack_experts", "moe_experts_packed",
+    "experts_packed", "experts_decode", "moe_block", "routing",
     "cohere2_moe_experts", "cohere2_moe_experts_decode",
     "deepseek_ocr2_moe_experts", "deepseek_ocr2_moe_experts_decode",
     "qwen3_next_moe_experts", "gpt_oss_moe_experts", "megablocks_moe", "pack_experts_nongated", "moe_router",
