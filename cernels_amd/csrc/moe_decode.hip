@@ -259,12 +259,14 @@ __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
 // its run QB pairs at a time (all their down rows and glu rows in flight together) and loads an expert's rows
 // only where the expert changes: consecutive pairs of one expert reuse the rows already in registers. Each lane
 // accumulates the sums of the token it holds; the eight waves' partial sums are added in wave order at the end,
-// so the result does not depend on timing. Run entries are wave-uniform (scalar loads).
-template <bool HAS_BIAS, int MAXC, int QB, int HB>
+// so the result does not depend on timing. Run entries are wave-uniform (scalar loads). BY_ORDER: route_w holds the pairs' weights
+// in the order of `order`; a choice at run time cost calls with fp32 weights up to 5% of this launch (19 tokens, H 1904 F 232,
+// top-11: 28.2 -> 29.6 us).
+template <bool HAS_BIAS, int MAXC, int QB, int HB, bool BY_ORDER>
 __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
     const uint16_t* __restrict__ glu, const uint16_t* __restrict__ w2, const float* __restrict__ b2,
-    const int32_t* __restrict__ order, const float* __restrict__ route_w, int by_order, uint16_t* __restrict__ out, int T,
-    int H, int F, int K) {
+    const int32_t* __restrict__ order, const float* __restrict__ route_w, uint16_t* __restrict__ out, int T, int H,
+    int F, int K) {
     static_assert(QB == 1 || QB == 2, "pairs per batch");
     __shared__ float part[kDnWaves][HB][kDecMaxTokens];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -329,7 +331,7 @@ __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
         for (int q = 0; q < QB; ++q) {
             if (q == 1 && !two) break;  // wave-uniform
             const int pp = q == 0 ? p0 : p1, ee = q == 0 ? e0 : e1;
-            const float wp = route_w[by_order ? i + q : pp];
+            const float wp = route_w[BY_ORDER ? i + q : pp];
             const int t = pp / K;
 #pragma unroll
             for (int j = 0; j < HB; ++j) {
@@ -396,13 +398,18 @@ static void launch_gateup_t(const uint16_t* x, const uint16_t* w1, const float* 
 // three workgroups per CU resident, so T=8's 640 workgroups (H=1280) run in one wave of residency.
 template <bool HAS_BIAS, int MAXC, int QB, int HB>
 static void launch_down_k(const uint16_t* glu, const uint16_t* w2, const float* b2, const int32_t* order,
-                          const float* route_w, int by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
-    hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB>), dim3(ceil_div(H, HB)), dim3(kDnThreads), 0, s,
-                       glu, w2, b2, order, route_w, by_order, out, T, H, F, K);
+                          const float* route_w, bool by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
+    const dim3 grid(ceil_div(H, HB)), block(kDnThreads);
+    if (by_order)
+        hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB, true>), grid, block, 0, s, glu, w2, b2, order, route_w, out,
+                           T, H, F, K);
+    else
+        hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB, false>), grid, block, 0, s, glu, w2, b2, order, route_w,
+                           out, T, H, F, K);
 }
 template <bool HAS_BIAS, int MAXC>
 static void launch_down_t(const uint16_t* glu, const uint16_t* w2, const float* b2, const int32_t* order,
-                          const float* route_w, int by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
+                          const float* route_w, bool by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
     const bool one = T * K <= kDnWaves;  // at most one pair per wave
     if constexpr (MAXC <= 2) {
         if (H / 4 >= 2 * dec_cu_count()) {
@@ -446,7 +453,7 @@ hipError_t launch_decode(const uint16_t* x, const uint16_t* w1, const float* b1,
     // ev (optional): 3 events recorded before gate_up, after gate_up, after down. order_w (required for bf16 weights): the
     // down GEMV then reads the weights from there, fp32 in the pair order that gate_up writes.
     const float* route_w = order_w ? order_w : static_cast<const float*>(w);
-    const int by_order = order_w != nullptr;
+    const bool by_order = order_w != nullptr;
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     if (E > kDecMaxExperts) return hipErrorInvalidValue;
     const int cg = pick_maxc(H), cd = pick_maxc(F);
