@@ -1042,14 +1042,15 @@ static double expected_tiles(double r, int bm) {
 //   of F 512, 43 rows 663 -> 662, 88 rows 763 -> 723 and with Zipf 1.2 skew 540 -> 473. At 112 rows (289 -> 308) and with
 //   fewer items (8 experts of F 5632, 25 rows: 95 -> 107) they lose.
 //   Over 858 shapes of 8 to 90 rows, 278 of which take it, the items are 1.07 times as fast on average and up to 4% slower in 5.
-// - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM on R
-//   rounds of persistent items is estimated at 0.95 ceil(R) / R, of up to 4 fragments (half of a workgroup's waves idle) at up to
-//   1.3, and at 1 for about one round (nothing to split); on Q rounds of two items per CU at 1, and a tenth of what the last
-//   round leaves idle. The ratio of the means, weighted by work, has to pass 1.06, and no GEMM may leave most CUs without an item
-//   that narrower persistent items fill. Measured over 992 shapes of 4 to 1024 experts, with and without skew: the 422 that take it are
-//   1.13 times as fast on average (8 experts of F 5632, 1024 rows, non-gated: 533 -> 421 us; 64 of H 1280 F 896, 384 rows: 259 -> 230)
-//   and 8 of them more than 1.5% slower (10 of H = F = 2688, 322 rows: 189 -> 209; 26 of H = F = 1856, 120 rows, non-gated: 148 -> 160; the
-//   others up to 5%); where it does not take them items are 0.75 to 1.73 times as fast (32 of H = F = 2880, 188 rows: 397 -> 435).
+// - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM on
+//   R rounds of persistent items is estimated at 0.95 ceil(R) / R, of up to 4 fragments (half of a workgroup's waves idle) at
+//   up to 1.3, and at 1 for about one round (nothing to split); on Q rounds of two items per CU at 1, and a tenth of what the
+//   last round leaves idle. The ratio of the means, weighted by work, has to pass 1.06, and no GEMM may leave most CUs
+//   without an item that narrower persistent items fill. Measured over 992 shapes of 4 to 1024 experts, with and without
+//   skew: the 422 that take it are 1.13 times as fast on average (8 experts of F 5632, 1024 rows, non-gated: 533 -> 421 us;
+//   64 of H 1280 F 896, 384 rows: 259 -> 230) and 8 of them more than 1.5% slower (10 of H = F = 2688, 322 rows: 189 -> 209;
+//   26 of H = F = 1856, 120 rows, non-gated: 148 -> 160; the others up to 5%); where it does not take them items are 0.75 to
+//   1.73 times as fast (32 of H = F = 2880, 188 rows: 397 -> 435).
 static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, int fw1, int fw2, int cus) {
     const double r = (double)P / E;
     if (r <= 90) return (long long)E * ceil_div(std::min(nf1, nf2), kPkWaves) >= 2LL * cus;
@@ -1068,12 +1069,13 @@ static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, in
     return fills && persistent > 1.06 * mid;
 }
 
-// Whether the down GEMM's Y rows leave through LDS. Straight from the accumulators a store is 64 pieces of 16 bytes, through LDS
-// 11 or 12 runs of up to 96, which the L2 takes faster where the whole chip stores at once; with few rows per item or in all
-// the LDS round trip and the longer code cost more than they save. Down GEMM, direct -> through LDS (us): 128 experts of H 2048
-// F 768, 157 rows 136.5 -> 129.7; 31 of H 2816 F 1408, 573 rows 174.0 -> 168.7; 32 of H = F = 2880, 512 rows 307.7 -> 302.0, but 84
-// rows with Zipf 1.2 skew 149.3 -> 155.3; 64 of H 1280 F 896, 79 rows with skew 57.5 -> 61.6. Over 176 shapes of 30 and more rows
-// the line at 100 rows and 20 MB of Y is 0.2% off the better of both on average, direct alone 0.8%, LDS alone 1.7%.
+// Whether the down GEMM's Y rows leave through LDS. Straight from the accumulators a store is 64 pieces of 16 bytes, through
+// LDS 11 or 12 runs of up to 96, which the L2 takes faster where the whole chip stores at once; with few rows per item or in
+// all the LDS round trip and the longer code cost more than they save. Down GEMM, direct -> through LDS (us): 128 experts of
+// H 2048 F 768, 157 rows 136.5 -> 129.7; 31 of H 2816 F 1408, 573 rows 174.0 -> 168.7; 32 of H = F = 2880, 512 rows 307.7 ->
+// 302.0, but 84 rows with Zipf 1.2 skew 149.3 -> 155.3; 64 of H 1280 F 896, 79 rows with skew 57.5 -> 61.6. Over 176 shapes
+// of 30 and more rows the line at 100 rows and 20 MB of Y is 0.2% off the better of both on average, direct alone 0.8%, LDS
+// alone 1.7%.
 static bool y_through_lds(long long P, int E, int H) { return P >= 100LL * E && 3 * P * H >= 20'000'000; }
 
 hipError_t launch_combine_h(const unsigned char* Y, const int32_t* idx, uint16_t* out, int T, int K, int E, int H,

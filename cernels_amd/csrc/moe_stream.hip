@@ -12,10 +12,10 @@
 // which spill) 35%.
 //
 // Two forms share the first projection:
-//   few    (T <= 32 tokens, at most 512 pairs, see few_supported): no route. Each workgroup finds its expert and that expert's tokens from
-//          the indices by itself (rows are tokens). Up to 16 pairs the down kernel may sum every expert's contribution to
-//          its 16 output columns (two launches, few_sums), else it writes a row per pair and the combine sums
-//          them (three; the general path takes five).
+//   few    (T <= 32 tokens, at most 512 pairs, see few_supported): no route. Each workgroup finds its expert and that
+//          expert's tokens from the indices by itself (rows are tokens). Up to 16 pairs the down kernel may sum every
+//          expert's contribution to its 16 output columns (two launches, few_sums), else it writes a row per pair and the
+//          combine sums them (three; the general path takes five).
 //   tiles  (up to 512 tokens, at most 8 rows per expert on average): the route's list with M-tiles of 32 rows, then the
 //          glu fixup and the combine as on the general path.
 // Measured, whole op in us, general path -> here (seeded routing, weights of three layers in turn): gpt-oss shapes (H = F =
@@ -213,9 +213,9 @@ __device__ __forceinline__ void store_y(unsigned char* Y, long long p, int H, in
     pack_y(v, ws, reinterpret_cast<u32x4*>(Y + (p * H + 32 * fc + 16 * half) * 3));
 }
 
-// few: the u-th smallest distinct expert of the indices (-1: fewer than u + 1), and in tokp[t] the first pair of token t
-// that names it, with bit 16 set if further pairs of t do (INT_MAX: none). One wave by itself: its own LDS words (a wave's LDS operations run in order), no
-// workgroup barrier.
+// few: the u-th smallest distinct expert of the indices (-1: fewer than u + 1), and in tokp[t] the first pair of token t that
+// names it, with bit 16 set if further pairs of t do (INT_MAX: none). One wave by itself: its own LDS words (a wave's LDS
+// operations run in order), no workgroup barrier.
 __device__ __forceinline__ int few_select(const int32_t* __restrict__ idx, int types, int P, int E, int K, int u, int lane,
                                           uint32_t* bits, int* tokp) {
     int ev[kFewMaxPairs / kWave];
@@ -651,10 +651,10 @@ constexpr int kYRow = 96;  // bytes of a fragment's 32 columns of a Y row
 constexpr int kMidGroups = 2;  // 64-column groups of an activation stage (32 KB)
 
 // The k-loop of one wave: one weight fragment (rw) times NMB row blocks. Group g (64 columns) of the reduction sits in
-// subtile g % kMidGroups of LDS buffer (g / kMidGroups) & 1; a stage is kMidGroups groups. Weight groups are loaded two groups ahead into slot
-// g & 1, and a stage's activations while the stage before it is multiplied; past the end both load the last group again.
-// buf(i): LDS buffer i, as an array of its own (a wait that the compiler adds before a read then covers the copies into that
-// array only).
+// subtile g % kMidGroups of LDS buffer (g / kMidGroups) & 1; a stage is kMidGroups groups. Weight groups are loaded two
+// groups ahead into slot g & 1, and a stage's activations while the stage before it is multiplied; past the end both load the
+// last group again. buf(i): LDS buffer i, as an array of its own (a wait that the compiler adds before a read then covers the
+// copies into that array only).
 template <typename OpT, int NMB, typename Buf, typename CopyA>
 __device__ __forceinline__ void mid_loop(__amdgpu_buffer_rsrc_t rw, uint32_t wo, int bs, __amdgpu_buffer_rsrc_t ra, int nG,
                                          int lane, Buf&& buf, CopyA&& copy_a, f32x16 (&acc)[kMidMB]) {
@@ -863,27 +863,29 @@ bool tiles_supported(int T, int K, int E) {
     return T <= kTilesMaxTokens && (long long)T * K <= (long long)kTilesMaxRows * E;
 }
 
-// Whether a call takes the few form: one 32-row block of tokens, experts that fit few_select's bitmap, lists that fit the down
-// kernel's LDS. Above kFdMaxPairs pairs also a bound on the ids that the first projection reads: each of its workgroups (nf1
-// fragments of each chosen expert) goes through all of them, where the other forms sort them once. Against the tiles form,
-// which takes most of these calls instead, the line is at 2^20 ids, against the grouped GEMMs at 600000. Whole op, few ->
-// tiles (us): 22 tokens of 428 experts of H 192 F 1664, top-21 (20 M ids) 216 -> 147; 28 of 76 of H 576 F 3968, top-14 (7.4 M)
-// 257 -> 190; 32 of 128 of H 2048 F 768, top-8 (1.6 M) 177 -> 183; 32 of 32 of H = F = 2880, top-4 (0.74 M) 276 -> 282; few -> grouped:
-// 30 tokens of 25 experts of H 1088 F 2112, top-16 (1.6 M) 109 -> 89; 32 of 14 of H 2816 F 1792, top-12 (0.60 M) 119 -> 101; 20 of 12
-// of H 3648 F 3776, top-9 (0.51 M) 199 -> 200. Over 1150 shapes of up to 32 tokens the two lines are 0.4% off the better form on
-// average, no line 2.5%. (So all of glu, one buffer in the down kernels, has at most 2^25 bytes.)
+// Whether a call takes the few form: one 32-row block of tokens, experts that fit few_select's bitmap, lists that fit the
+// down kernel's LDS. Above kFdMaxPairs pairs also a bound on the ids that the first projection reads: each of its workgroups
+// (nf1 fragments of each chosen expert) goes through all of them, where the other forms sort them once. Against the tiles
+// form, which takes most of these calls instead, the line is at 2^20 ids, against the grouped GEMMs at 600000. Whole op, few
+// -> tiles (us): 22 tokens of 428 experts of H 192 F 1664, top-21 (20 M ids) 216 -> 147; 28 of 76 of H 576 F 3968, top-14
+// (7.4 M) 257 -> 190; 32 of 128 of H 2048 F 768, top-8 (1.6 M) 177 -> 183; 32 of 32 of H = F = 2880, top-4 (0.74 M) 276 ->
+// 282; few -> grouped: 30 tokens of 25 experts of H 1088 F 2112, top-16 (1.6 M) 109 -> 89; 32 of 14 of H 2816 F 1792, top-12
+// (0.60 M) 119 -> 101; 20 of 12 of H 3648 F 3776, top-9 (0.51 M) 199 -> 200. Over 1150 shapes of up to 32 tokens the two
+// lines are 0.4% off the better form on average, no line 2.5%. (So glu, one buffer in the down kernels, stays far below 2^31
+// bytes there.)
 bool few_supported(int T, int K, int E, int nf1) {
     const long long P = (long long)T * K;
     if (T > kFewMaxTokens || K > kFewMaxTopk || E > kFewMaxExperts || P > kFewMaxPairs) return false;
     return P <= kFdMaxPairs || nf1 * std::min<long long>(P, E) * P <= (tiles_supported(T, K, E) ? 1 << 20 : 600000);
 }
 
-// Whether the few form's down kernel sums over the slots itself, which saves the combine's launch. Its H / 16 workgroups walk all
-// chosen experts one after the other, so with short rows of the result they stream less than the whole chip, for a time that
-// goes with experts x F. Down kernel with the sum against rows and combine (us): H = F = 2880, 4 pairs 16.7 / 15.4 + 4.6, 16 pairs 50.6 /
-// 46.6 + 5.2; 33 pairs of H 2048 F 768 23.1 / 15.6 + 4.0. Whole op, sum / rows: 12 experts of H 3072 F 2304 118 / 120; 4 of H 1088 F 7488
-// 46 / 34; 15 of H 192 F 128 15.4 / 13.1; 3 of H 512 F 1280 13.4 / 17.0; one of H 128 F 8960 14.1 / 19.9. Over 400 shapes of up to
-// 16 pairs this line is 1.3% off the better of both, the sum alone 20%, rows alone 2.6%.
+// Whether the few form's down kernel sums over the slots itself, which saves the combine's launch. Its H / 16 workgroups walk
+// all chosen experts one after the other, so with short rows of the result they stream less than the whole chip, for a time
+// that goes with experts x F. Down kernel with the sum against rows and combine (us): H = F = 2880, 4 pairs 16.7 / 15.4 +
+// 4.6, 16 pairs 50.6 / 46.6 + 5.2; 33 pairs of H 2048 F 768 23.1 / 15.6 + 4.0. Whole op, sum / rows: 15 experts of H 3072 F
+// 2304 118 / 120; 4 of H 1088 F 7488 46 / 34; 15 of H 192 F 128 15.4 / 13.1; 3 of H 512 F 1280 13.4 / 17.0; one of H 128 F
+// 8960 14.1 / 19.9. Over 400 shapes of up to 16 pairs this line is 1.3% off the better of both, the sum alone 20%, rows alone
+// 2.6%.
 bool few_sums(int T, int K, int E, int H, int F) {
     const long long P = (long long)T * K, um = std::min<long long>(P, E);
     return P <= kFdMaxPairs && (H >= 2048 || um <= 2 || um * F <= 2000);

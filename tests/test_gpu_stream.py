@@ -1,8 +1,8 @@
 """Few rows per expert on packed weights: the streaming forms of moe_experts_packed, against the fp64 oracle.
 
-Up to 32 tokens and 512 pairs the kernels route by themselves (up to 16 pairs with the sum over slots in the down kernel
-where its workgroups suffice, else with a row per pair) where the ids that their workgroups read stay few; up to 512 tokens with at most 8 rows per expert on average they walk the route's list in
-M-tiles of 32 rows. Cases sit on both sides of each line, at the smallest and largest sizes, with ids that are out of range
+Up to 32 tokens and 512 pairs the kernels route by themselves while the ids that their workgroups read stay few (up to 16
+pairs with the sum over slots in the down kernel where its workgroups suffice, else with a row per pair); up to 512 tokens
+with at most 8 rows per expert on average they walk the route's list in M-tiles of 32 rows. Cases sit on both sides of each line, at the smallest and largest sizes, with ids that are out of range
 or name an expert twice, one expert taking every token, and glu segments stored scaled.
 """
 
