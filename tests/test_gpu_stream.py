@@ -33,6 +33,8 @@ CASES = [
     (1, 64, 64, 1, 1, SILU, "plain", "few_sum"),  # one stage per projection: three of the four waves have none
     (1, 192, 320, 1024, 16, SILU, "plain", "few_rows"),  # 16 pairs in one token, partial last bundles
     (1, 2048, 192, 20, 16, SILU, "plain", "few_sum"),  # long rows of the result: the sum is in the down kernel
+    (2, 2048, 2112, 3, 3, GPT, "twice", "few_sum"),  # 33 stages: eight shares of an expert, 5 + 7 x 4
+    (3, 2048, 1088, 4, 3, SILU, "plain", "few_sum"),  # 17 stages: four shares
     (1, 1984, 128, 20, 16, SILU, "plain", "few_rows"),  # shorter ones with more than 2000 columns of glu over all experts
     (1, 192, 64, 40, 16, GPT, "plain", "few_sum"),  # fewer
     (8, 64, 1088, 2, 2, GPT, "plain", "few_sum"),  # or two experts
@@ -174,17 +176,17 @@ def test_few_rows_graph_replays(device, T, form):
         assert torch.equal(out, ops.moe_experts_packed(d["x"], pk, d["idx"], d["w"], 4))
 
 
-@pytest.mark.parametrize("T,K,part,H,E,form", [(4, 4, 1, 2048, 10, "few_sum"), (5, 3, 1, 2048, 10, "few_sum"),
-                                               (24, 4, 6, 192, 32, "few_rows"), (64, 4, 40, 192, 32, "tiles")],
+@pytest.mark.parametrize("T,K,part,H,Fi,E,form", [(4, 4, 1, 2048, 832, 10, "few_sum"), (5, 3, 1, 2048, 2112, 6, "few_sum"),
+                                                  (24, 4, 6, 192, 832, 32, "few_rows"), (64, 4, 40, 192, 832, 32, "tiles")],
                          ids=["fused", "fused-k3", "rows", "tiles"])
-def test_few_rows_do_not_depend_on_the_other_tokens(device, T, K, part, H, E, form):
+def test_few_rows_do_not_depend_on_the_other_tokens(device, T, K, part, H, Fi, E, form):
     """A token's row is the same bit for bit whether the call holds the other tokens or not (both calls of one form), some of
     which are stored scaled, and however the experts are numbered: its slots are summed in their own order, each from a
-    reduction that is cut at places that only the layer's sizes fix. F gives 13 stages, which no number of waves divides."""
+    reduction that is cut at places that only the layer's sizes fix. F gives 13 or 33 stages, which no number of shares divides."""
     from cernels_amd import ops
 
-    c = rand_case(T + K, T, H, 832, E, K, layout="interleaved", act="gptoss", bias=True, std=0.05)
-    assert form_of(c) == packed_form(part, H, 832, E, K, "gptoss") == form
+    c = rand_case(T + K, T, H, Fi, E, K, layout="interleaved", act="gptoss", bias=True, std=0.05)
+    assert form_of(c) == packed_form(part, H, Fi, E, K, "gptoss") == form
     # two slots cancel exactly (equal experts, weights 1 and -1) beside small ones: what is left of a sum that was cut or ordered
     # otherwise shows in bf16
     for name in ("W1", "W2", "b1", "b2"):
