@@ -883,14 +883,14 @@ bool few_supported(int T, int K, int E, int nf1) {
 
 // Whether the few form's down kernel sums over the slots itself, which saves the combine's launch. Its H / 16 workgroups walk
 // all chosen experts one after the other, so with short rows of the result they stream less than the whole chip, for a time
-// that goes with experts x F. Down kernel with the sum against rows and combine (us): H = F = 2880, 4 pairs 16.7 / 15.4 +
-// 4.6, 16 pairs 50.6 / 46.6 + 5.2; 33 pairs of H 2048 F 768 23.1 / 15.6 + 4.0. Whole op, sum / rows: 15 experts of H 3072 F
-// 2304 118 / 120; 4 of H 1088 F 7488 46 / 34; 15 of H 192 F 128 15.4 / 13.1; 3 of H 512 F 1280 13.4 / 17.0; one of H 128 F
-// 8960 14.1 / 19.9. Over 400 shapes of up to 16 pairs this line is 1.3% off the better of both, the sum alone 20%, rows alone
-// 2.6%.
+// that goes with experts x F. Whole op, sum / rows and combine (us): 4 experts of H = F = 2880 35.8 / 37.3; 11 of H 2048 F
+// 512 18.9 / 21.1; 6 of H 1280 F 896 15.7 / 17.0, 12 23.8 / 22.4; 14 of H 1280 F 640 20.8 / 23.0; 8 of H 896 F 1024 14.0 /
+// 12.5; 8 of H 1472 F 2560 36.6 / 33.0; 2 of H 1664 F 3968 14.3 / 17.6. Over 500 shapes of up to 16 pairs this line is 0.2%
+// off the better of both, the sum alone 3%, rows alone 10%. Above 16 pairs rows: 33 pairs of H 2048 F 768, the down kernel
+// alone, 23.1 / 15.6 + 4.0.
 bool few_sums(int T, int K, int E, int H, int F) {
     const long long P = (long long)T * K, um = std::min<long long>(P, E);
-    return P <= kFdMaxPairs && (H >= 2048 || um <= 2 || um * F <= 2000);
+    return P <= kFdMaxPairs && (H >= 2048 || um <= 2 || um * F <= std::max(5000, 8 * H));
 }
 
 // Parts of the lists that the few form passes from its first to its second launch, at `lists`: um experts, um x T glu rows,

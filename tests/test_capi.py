@@ -81,7 +81,8 @@ def test_packed_forms_on_their_lines(L):
         ((513, 64, 64, 65, 1), "grouped"), ((64, 64, 64, 32, 4), "tiles"), ((65, 64, 64, 32, 4), "grouped"),
         ((32, 64, 128, 512, 16), "tiles"), ((32, 64, 576, 32, 16), "few_rows"), ((32, 64, 640, 32, 16), "grouped"),
         ((32, 2880, 2880, 32, 4), "few_rows"), ((28, 576, 3968, 76, 14), "tiles"), ((1, 2048, 2**16, 16, 16), "few_sum"),
-        ((1, 1984, 128, 15, 16), "few_sum"), ((1, 1984, 128, 16, 16), "few_rows"), ((4, 64, 8960, 2, 4), "few_sum"),
+        ((1, 1984, 960, 16, 16), "few_sum"), ((1, 1984, 1024, 16, 16), "few_rows"),
+        ((1, 64, 320, 15, 16), "few_sum"), ((1, 64, 320, 16, 16), "few_rows"), ((4, 64, 8960, 2, 4), "few_sum"),
         # few wide items that would leave most CUs idle where narrow ones fill them; near-full rounds of narrow items; about one round
         ((289, 960, 2176, 16, 6), "grouped"), ((681, 4096, 2944, 17, 5), "grouped"), ((1235, 2688, 1088, 5, 3), "grouped"),
         ((4096, 1280, 896, 64, 6), "items"), ((3245, 1472, 1536, 28, 9), "items"),

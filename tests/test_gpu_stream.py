@@ -35,8 +35,9 @@ CASES = [
     (1, 2048, 192, 20, 16, SILU, "plain", "few_sum"),  # long rows of the result: the sum is in the down kernel
     (2, 2048, 2112, 3, 3, GPT, "twice", "few_sum"),  # 33 stages: eight shares of an expert, 5 + 7 x 4
     (3, 2048, 1088, 4, 3, SILU, "plain", "few_sum"),  # 17 stages: four shares
-    (1, 1984, 128, 20, 16, SILU, "plain", "few_rows"),  # shorter ones with more than 2000 columns of glu over all experts
-    (1, 192, 64, 40, 16, GPT, "plain", "few_sum"),  # fewer
+    (1, 1024, 512, 20, 16, SILU, "plain", "few_sum"),  # shorter ones with up to 8 H columns of glu over all experts
+    (1, 1024, 576, 20, 16, SILU, "plain", "few_rows"),  # more
+    (1, 192, 256, 40, 16, GPT, "plain", "few_sum"),  # or up to 5000
     (8, 64, 1088, 2, 2, GPT, "plain", "few_sum"),  # or two experts
     (16, 128, 192, 3, 1, GPT, "plain", "few_sum"),  # 16 pairs, the fused down's last
     (17, 128, 192, 3, 1, GPT, "plain", "few_rows"),  # 17: rows and combine
