@@ -1045,12 +1045,13 @@ static double expected_tiles(double r, int bm) {
 // - Above, where the persistent items fall badly into rounds of one per CU. Relative to full rounds of wide items, a GEMM on
 //   R rounds of persistent items is estimated at 0.95 ceil(R) / R, of up to 4 fragments (half of a workgroup's waves idle) at
 //   up to 1.3, and at 1 for about one round (nothing to split); on Q rounds of two items per CU at 1, and a tenth of what the
-//   last round leaves idle. The ratio of the means, weighted by work, has to pass 1.06, and no GEMM may leave most CUs
-//   without an item that narrower persistent items fill. Measured over 992 shapes of 4 to 1024 experts, with and without
-//   skew: the 422 that take it are 1.13 times as fast on average (8 experts of F 5632, 1024 rows, non-gated: 533 -> 421 us;
-//   64 of H 1280 F 896, 384 rows: 259 -> 230) and 8 of them more than 1.5% slower (10 of H = F = 2688, 322 rows: 189 -> 209;
-//   26 of H = F = 1856, 120 rows, non-gated: 148 -> 160; the others up to 5%); where it does not take them items are 0.75 to
-//   1.73 times as fast (32 of H = F = 2880, 188 rows: 397 -> 435).
+//   last round leaves idle. The ratio of the means, weighted by work, has to pass 1.06, and in neither GEMM may the items
+//   occupy less than 0.55 of the CUs that narrower persistent items keep busy over their rounds (16 experts of H 960 F 2176,
+//   108 rows: 86 -> 96 us, but 8 of H 2048 F 5632, 241 rows, non-gated: 254 -> 169). Measured over 992 shapes of 4 to 1024
+//   experts, with and without skew: the 427 that take it are 1.13 times as fast on average (8 experts of F 5632, 1024 rows,
+//   non-gated: 533 -> 421 us; 64 of H 1280 F 896, 384 rows: 259 -> 230) and 8 of them more than 1.5% slower (10 of H = F =
+//   2688, 322 rows: 189 -> 209; 26 of H = F = 1856, 120 rows, non-gated: 148 -> 160; the others up to 5%); where it does not
+//   take them items are 0.75 to 1.73 times as fast (32 of H = F = 2880, 188 rows: 397 -> 435).
 static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, int fw1, int fw2, int cus) {
     const double r = (double)P / E;
     if (r <= 90) return (long long)E * ceil_div(std::min(nf1, nf2), kPkWaves) >= 2LL * cus;
@@ -1059,10 +1060,10 @@ static bool mid_supported(long long P, int E, int nf1, int nf2, int H, int F, in
     bool fills = true;
     auto add = [&](int nf, int fw, double work) {
         const double R = tiles * ceil_div(nf, fw), Q = items * ceil_div(nf, kPkWaves);
-        const double rounds = std::ceil(R - 0.02) / R;
+        const double whole = std::max(1.0, std::ceil(R - 0.02)), rounds = whole / R;
         persistent += work * (R <= 1.05 ? 1.0 : fw <= 4 ? std::min(1.3, 1.15 * rounds) : 0.95 * rounds);
         mid += work * (Q > 1 ? 1 + 0.1 * std::max(0.0, std::ceil(Q - 0.02) - Q) / Q : 1.0);
-        fills = fills && 2 * Q >= 0.6 * std::min(R, 1.0);
+        fills = fills && 2 * Q >= 0.55 * R / whole;
     };
     add(nf1, fw1, (double)nf1 * H);
     add(nf2, fw2, (double)nf2 * F);

@@ -90,6 +90,7 @@ def test_packed_forms_on_their_lines(L):
     ]
     for sizes, form in lines:
         assert _native.PACKED_FORMS[L.cernels_moe_experts_packed_form(*sizes, 0)] == form, sizes
+    assert _native.PACKED_FORMS[L.cernels_moe_experts_packed_form(964, 2048, 5632, 8, 2, 2)] == "items"  # narrow items in little more than a round
     for bad in ((0, 64, 64, 8, 2, 0), (4, 96, 64, 8, 2, 0), (4, 64, 64, 1025, 2, 0), (4, 64, 64, 8, 2, 9), (4, 64, 64, 8, 0, 0)):
         assert L.cernels_moe_experts_packed_form(*bad) == -1
     assert [L.cernels_moe_route_launches(*a) for a in ((0, 4, 8), (333, 6, 64), (6000, 4, 1024), (8192, 8, 1024))] == [1, 1, 2, 3]
