@@ -261,12 +261,14 @@ __global__ __launch_bounds__(kDecThreads) void moe_decode_gateup_kernel(
 // accumulates the sums of the token it holds; the eight waves' partial sums are added in wave order at the end,
 // so the result does not depend on timing. Run entries are wave-uniform (scalar loads). BY_ORDER: route_w holds the pairs' weights
 // in the order of `order`; a choice at run time cost calls with fp32 weights up to 5% of this launch (19 tokens, H 1904 F 232,
-// top-11: 28.2 -> 29.6 us).
+// top-11: 28.2 -> 29.6 us). With BY_ORDER by_order is 1 all the same: the choice keeps the weight's load behind the pair's. Scalar
+// loads return out of order, so issued together the wait for the pair, which the row loads need, is for both (one token of H
+// 2048 F 768: 16.3 -> 16.9 us a call).
 template <bool HAS_BIAS, int MAXC, int QB, int HB, bool BY_ORDER>
 __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
     const uint16_t* __restrict__ glu, const uint16_t* __restrict__ w2, const float* __restrict__ b2,
-    const int32_t* __restrict__ order, const float* __restrict__ route_w, uint16_t* __restrict__ out, int T, int H,
-    int F, int K) {
+    const int32_t* __restrict__ order, const float* __restrict__ route_w, int by_order, uint16_t* __restrict__ out, int T,
+    int H, int F, int K) {
     static_assert(QB == 1 || QB == 2, "pairs per batch");
     __shared__ float part[kDnWaves][HB][kDecMaxTokens];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(kDnThreads) void moe_decode_down_kernel(
         for (int q = 0; q < QB; ++q) {
             if (q == 1 && !two) break;  // wave-uniform
             const int pp = q == 0 ? p0 : p1, ee = q == 0 ? e0 : e1;
-            const float wp = route_w[BY_ORDER ? i + q : pp];
+            const float wp = route_w[BY_ORDER && by_order ? i + q : pp];
             const int t = pp / K;
 #pragma unroll
             for (int j = 0; j < HB; ++j) {
@@ -401,11 +403,11 @@ static void launch_down_k(const uint16_t* glu, const uint16_t* w2, const float* 
                           const float* route_w, bool by_order, uint16_t* out, int T, int H, int F, int K, hipStream_t s) {
     const dim3 grid(ceil_div(H, HB)), block(kDnThreads);
     if (by_order)
-        hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB, true>), grid, block, 0, s, glu, w2, b2, order, route_w, out,
+        hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB, true>), grid, block, 0, s, glu, w2, b2, order, route_w, 1, out,
                            T, H, F, K);
     else
         hipLaunchKernelGGL((moe_decode_down_kernel<HAS_BIAS, MAXC, QB, HB, false>), grid, block, 0, s, glu, w2, b2, order, route_w,
-                           out, T, H, F, K);
+                           0, out, T, H, F, K);
 }
 template <bool HAS_BIAS, int MAXC>
 static void launch_down_t(const uint16_t* glu, const uint16_t* w2, const float* b2, const int32_t* order,
